@@ -13,6 +13,7 @@
 #include "vv_device.hpp"
 #include "vv_internal.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 
@@ -702,17 +703,13 @@ hipError_t make_lic_args(const LicLaunch& L, LicArgs& a)
     a.ty = L.tile[1];
     a.tz = L.tile[2];
     if (a.tx * a.ty * a.tz != kThreads) return hipErrorInvalidValue;
-    a.sx = L.super_tile[0] > 0 ? L.super_tile[0] : 1;
-    a.sy = L.super_tile[1] > 0 ? L.super_tile[1] : 1;
-    a.sz = L.super_tile[2] > 0 ? L.super_tile[2] : 1;
-    // the grid of tiles is rounded up to whole super-tiles; tiles past the
-    // volume exit at the voxel bounds check
-    a.sgx = (L.field.n[0] + a.tx * a.sx - 1) / (a.tx * a.sx);
-    a.sgy = (L.field.n[1] + a.ty * a.sy - 1) / (a.ty * a.sy);
-    const int sgz = (L.field.n[2] + a.tz * a.sz - 1) / (a.tz * a.sz);
-    a.gx = a.sgx * a.sx;
-    a.gy = a.sgy * a.sy;
-    a.gz = sgz * a.sz;
+    a.gx = (L.field.n[0] + a.tx - 1) / a.tx;
+    a.gy = (L.field.n[1] + a.ty - 1) / a.ty;
+    a.gz = (L.field.n[2] + a.tz - 1) / a.tz;
+    // a super-tile is at most the tile grid
+    a.sx = std::min(std::max(L.super_tile[0], 1), a.gx);
+    a.sy = std::min(std::max(L.super_tile[1], 1), a.gy);
+    a.sz = std::min(std::max(L.super_tile[2], 1), a.gz);
     a.nblocks = a.gx * a.gy * a.gz;
     a.per_xcd = (a.nblocks + 7) / 8;
     return hipSuccess;
