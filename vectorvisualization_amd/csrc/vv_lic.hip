@@ -171,7 +171,9 @@ __global__ void __launch_bounds__(kThreads) k_field_decode(const T* field, int n
 
 // LIC copy of the field for equal field and noise grids: every CLAMP-padded
 // texel p keeps its rgb and carries in channel 3 the noise byte of REPEAT
-// texel (p - 1) mod n per axis, a value each texel type holds exactly
+// texel (p - 1) mod n per axis, a value each texel type holds exactly.  FP32
+// texels hold two halves there instead, the byte and the next texel's byte
+// (along x) minus it.
 template <typename T>
 __global__ void __launch_bounds__(kThreads) k_pack_lic_field(const T* field, const uint8_t* noise, int nx, int ny,
                                                              int nz, T* out)
@@ -185,7 +187,10 @@ __global__ void __launch_bounds__(kThreads) k_pack_lic_field(const T* field, con
     const uint32_t b = noise[((long long)iz * (ny + 1) + iy) * (nx + 1) + ix];
     if constexpr (std::is_same<T, float4>::value) {
         float4 v = field[q];
-        v.w = (float)b;
+        const int jx = ix + 1 == nx ? 0 : ix + 1;
+        const int d = (int)noise[((long long)iz * (ny + 1) + iy) * (nx + 1) + jx] - (int)b;
+        v.w = __uint_as_float((uint32_t)__half_as_ushort(__float2half((float)b)) |
+                              ((uint32_t)__half_as_ushort(__float2half((float)d)) << 16));
         out[q] = v;
     } else if constexpr (std::is_same<T, half4_t>::value) {
         uint2 u = reinterpret_cast<const uint2*>(field)[q];

@@ -147,10 +147,20 @@ __device__ __forceinline__ void store_repeat(T* out, int osy, int osz, int x, in
 // those of tri(), so results do not change.
 // NCH = 3: the field direction; NCH = 4: also the noise byte that the LIC
 // copy of the field carries in channel 3 (equal field and noise grids)
-// A cache is keyed by the three floors of its cell (x = u n - 0.5), so a hit
-// costs three compares and no index arithmetic; NaN keys never hit.  (Cells
+// A cache is keyed by the three floors k of its cell.  A texel coordinate t =
+// u n - 0.5 lies in the cell when every t - k is in [0, 1), and t - k is then
+// the fraction t - floor(t) itself, so a hit needs no floor: the three
+// differences are compared at once as unsigned words (the bits of a float in
+// [0, 1) lie below those of 1, a negative, larger or NaN difference above).
+// NaN keys never hit; a coordinate so little below an integer that its
+// fraction rounds to 1 is filled again, with the same texels.  (Cells
 // outside the volume with different floors but the same clamped texels are
-// reloaded, with the same values.)
+// reloaded, with the same values.)  On gfx950 floor, compare, convert, med3
+// and 24-bit multiplies issue at about 0.9 wave64 instructions per clock per
+// CU, fma, add, sub, mul and mov at 1.4-1.6 (measured), so the kernels spend
+// their compares and conversions on a miss: 256^3, L = 40, FP16 4.44 -> 4.27 ms,
+// UNORM8 4.73 -> 4.53, FP16 with noise on another grid 7.04 -> 6.31; FP32, which
+// waits for the L1, 5.60 -> 5.59.
 // v_fma_mix_f32 with one half operand, which the instruction widens exactly
 // (every half is a float), so each form is one rounding of the exact result:
 //   fma_half<HI>(a, b, w) = fmaf(a, b, (float)h), h the low (HI 0) or high
@@ -198,6 +208,49 @@ struct FieldCache {
             v0[ch][k] = t0[ch];
             dx[ch][k] = t1[ch] - t0[ch];
         }
+    }
+};
+
+// r = fmaf(f, (float)hi, (float)lo) of a word holding two halves (lo in the
+// low bits), both widened exactly
+__device__ __forceinline__ float lerp_pair(float f, unsigned w)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, %2, %2 op_sel:[0,1,0] op_sel_hi:[0,1,1]" : "=v"(r) : "v"(f), "v"(w));
+    return r;
+}
+
+// FP32 texels of the LIC copy: channel 3 holds the noise byte and the
+// difference to the next texel's as two halves (whole numbers up to 255, held
+// exactly), so a fill subtracts three channels instead of four and keeps one
+// noise word per row instead of two floats: the kernel fits its 80 registers
+// without the five spills it had (256^3, L = 40: 5.65 -> 5.59 ms).  A load of 8
+// to 16 bytes per lane occupies the L1 for 16 clocks or more whichever lanes
+// take part (measured), and the eight loads of a fill make that the bound of
+// the FP32 kernel: 1.1 fills per step, 145 of its 155 clocks per step.
+template <>
+struct FieldCache<float4, 4> {
+    float kx, ky, kz;
+    bool same;
+    float v0[3][4], dx[3][4];
+    unsigned nw[4];
+    __device__ __forceinline__ void reset() { kx = ky = kz = __builtin_nanf(""); same = false; }
+    template <int CH>
+    __device__ __forceinline__ float xlerp(int k, float fx) const
+    {
+        if constexpr (CH == 3)
+            return lerp_pair(fx, nw[k]);
+        else
+            return fmaf(fx, dx[CH][k], v0[CH][k]);
+    }
+    __device__ __forceinline__ void set_row(int k, const float* t0, const float* t1)
+    {
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) {
+            v0[ch][k] = t0[ch];
+            dx[ch][k] = t1[ch] - t0[ch];
+        }
+        nw[k] = __float_as_uint(t0[3]);
     }
 };
 
@@ -260,25 +313,36 @@ __device__ __forceinline__ float tri_cached(const float* v0, const float* dx, fl
     return lerpf(c0, c1, fz);
 }
 
-// axis coordinate: floor and fraction of x = u*n - 0.5 (shared by the
-// CLAMP field cell and, on the same grid, the REPEAT noise cell)
-struct Ax {
-    float fl, f;
+// texel coordinate of u on an axis of n texels
+__device__ __forceinline__ float texel(float u, int n) { return fmaf(u, (float)n, -0.5f); }
+
+// a position in texel units, or its fractions in a cell
+struct P3 {
+    float x, y, z;
 };
 
-__device__ __forceinline__ Ax axis(float u, int n)
+__device__ __forceinline__ bool in_cell(const P3& f)
 {
-    Ax r;
-    const float x = fmaf(u, (float)n, -0.5f);
-    r.fl = floorf(x);
-    r.f = x - r.fl;
-    return r;
+    return max(max(__float_as_uint(f.x), __float_as_uint(f.y)), __float_as_uint(f.z)) < 0x3f800000u;
 }
 
-// corner index of a CLAMP-padded axis: clamp(floor, -1, n-1) + 1
-__device__ __forceinline__ unsigned clamp_idx(float fl, float nm1)
+// fractions of t in the cell keyed by a cache's floors; false when t lies in
+// another cell
+template <typename CACHE>
+__device__ __forceinline__ bool cell_hit(const CACHE& c, const P3& t, P3& f)
 {
-    return (unsigned)((int)__builtin_amdgcn_fmed3f(fl, -1.0f, nm1) + 1);
+    f = P3{t.x - c.kx, t.y - c.ky, t.z - c.kz};
+    return in_cell(f);
+}
+
+// makes t's cell the cached one (its texels follow)
+template <typename CACHE>
+__device__ __forceinline__ void cell_rekey(CACHE& c, const P3& t, P3& f)
+{
+    c.kx = floorf(t.x);
+    c.ky = floorf(t.y);
+    c.kz = floorf(t.z);
+    f = P3{t.x - c.kx, t.y - c.ky, t.z - c.kz};
 }
 
 // corner index of a REPEAT-padded axis: floor mod n
@@ -308,7 +372,8 @@ struct FieldLoad;
 
 // The loaders fill NCH channels (3: rgb, 4: rgb + channel 3) of the texels
 // x0 and x1 of a cell row.
-// float4 texels: two 12- or 16-byte loads (x0 and x1)
+// float4 texels: 12 or 16 bytes of x0 and 12 of x1 (the LIC copy's channel 3
+// of x0 covers both texels)
 template <>
 struct FieldLoad<float4> {
     static constexpr unsigned kShift = 4;
@@ -317,10 +382,9 @@ struct FieldLoad<float4> {
     {
         const gfloat* q = (const gfloat*)((gchar)base + off);
 #pragma unroll
-        for (int ch = 0; ch < NCH; ++ch) {
-            t0[ch] = q[ch];
-            t1[ch] = q[4 + ch];
-        }
+        for (int ch = 0; ch < NCH; ++ch) t0[ch] = q[ch];
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) t1[ch] = q[4 + ch];
     }
 };
 
@@ -395,13 +459,33 @@ struct CachedArgs {
     unsigned bsy, bsz;        // BRICK: brick-row and brick-plane strides (elements)
     const unsigned char* nr;  // noise bytes
     float fnm1[3];      // field n-1 per axis
+    float fpx;          // padded field row, n+2
     unsigned fsy, fsz;  // field element strides
     unsigned nsy, nsz;  // noise element strides
 };
 
-__device__ __forceinline__ bool key_hit(float kx, float ky, float kz, const Ax& ax, const Ax& ay, const Ax& az)
+// element of the corner (x0, y0, z0) of a CLAMP-padded cell from its clamped
+// floors m (clamp(floor, -1, n-1) + 1 per axis).  The offset in the plane is
+// an integer below 2^24 (the launch rule of the cached kernels), so float
+// arithmetic is exact and costs one conversion instead of two and a 24-bit
+// product.
+__device__ __forceinline__ unsigned clamp_corner(const CachedArgs& c, const P3& m)
 {
-    return ax.fl == kx && ay.fl == ky && az.fl == kz;
+    const float xy = fmaf(m.y, c.fpx, m.x + (c.fpx + 1.0f));
+    return __umul24((unsigned)(int)(m.z + 1.0f), c.fsz) + (unsigned)(int)xy;
+}
+
+__device__ __forceinline__ P3 clamp_floors(const CachedArgs& c, float kx, float ky, float kz)
+{
+    return P3{__builtin_amdgcn_fmed3f(kx, -1.0f, c.fnm1[0]), __builtin_amdgcn_fmed3f(ky, -1.0f, c.fnm1[1]),
+              __builtin_amdgcn_fmed3f(kz, -1.0f, c.fnm1[2])};
+}
+
+// element of the corner of a REPEAT-padded noise cell from its floors
+__device__ __forceinline__ unsigned repeat_corner(const LicArgs& a, const CachedArgs& c, const NoiseCache& nc)
+{
+    return __umul24(repeat_idx(nc.kz, a.noise.n[2]), c.nsz) + __umul24(repeat_idx(nc.ky, a.noise.n[1]), c.nsy) +
+           repeat_idx(nc.kx, a.noise.n[0]);
 }
 
 // Equal field and noise grids with freq 1 (SAME): the LIC copy of the field
@@ -411,26 +495,21 @@ __device__ __forceinline__ bool key_hit(float kx, float ky, float kz, const Ax& 
 // then hold the same noise bytes, so the field fill brings the noise cell
 // with it: no noise loads.  Outside that range (a streamline that left the
 // volume) the noise comes from the REPEAT array.  The noise value and its
-// arithmetic are those of noise_from_axes.  field_from_axes sets fc.same
-// for a cell whose three floors lie in that range.
+// arithmetic are those of noise_at_cell.  field_at sets fc.same for a cell
+// whose three floors lie in that range.
 
 template <typename FT, int NCH, bool BRICK = false>
-__device__ __forceinline__ float3 field_from_axes(const CachedArgs& c, FieldCache<FT, NCH>& fc, const Ax& ax,
-                                                  const Ax& ay, const Ax& az)
+__device__ __forceinline__ float3 field_at(const CachedArgs& c, FieldCache<FT, NCH>& fc, const P3& t, P3& f)
 {
-    if (!key_hit(fc.kx, fc.ky, fc.kz, ax, ay, az)) {
-        fc.kx = ax.fl;
-        fc.ky = ay.fl;
-        fc.kz = az.fl;
+    if (!cell_hit(fc, t, f)) {
+        cell_rekey(fc, t, f);
         // clamped floors; a floor the clamp leaves unchanged lies in [-1, n-1]
-        const float mx = __builtin_amdgcn_fmed3f(ax.fl, -1.0f, c.fnm1[0]);
-        const float my = __builtin_amdgcn_fmed3f(ay.fl, -1.0f, c.fnm1[1]);
-        const float mz = __builtin_amdgcn_fmed3f(az.fl, -1.0f, c.fnm1[2]);
-        if constexpr (NCH == 4) fc.same = mx == ax.fl && my == ay.fl && mz == az.fl;
+        const P3 m = clamp_floors(c, fc.kx, fc.ky, fc.kz);
+        if constexpr (NCH == 4) fc.same = m.x == fc.kx && m.y == fc.ky && m.z == fc.kz;
         if constexpr (BRICK) {
             // float4 texels in 8^3 bricks (c.fr): the element of padded
             // texel (x, y, z) is xb(x) + yb(y) + zb(z)
-            const unsigned x0 = (unsigned)((int)mx + 1), y0 = (unsigned)((int)my + 1), z0 = (unsigned)((int)mz + 1);
+            const unsigned x0 = (unsigned)((int)m.x + 1), y0 = (unsigned)((int)m.y + 1), z0 = (unsigned)((int)m.z + 1);
             const unsigned xb[2] = {((x0 >> 3) << 9) | (x0 & 7u), (((x0 + 1) >> 3) << 9) | ((x0 + 1) & 7u)};
             const unsigned yb[2] = {__umul24(y0 >> 3, c.bsy) + ((y0 & 7u) << 3),
                                     __umul24((y0 + 1) >> 3, c.bsy) + (((y0 + 1) & 7u) << 3)};
@@ -443,18 +522,15 @@ __device__ __forceinline__ float3 field_from_axes(const CachedArgs& c, FieldCach
                 const gfloat* q1 = (const gfloat*)((gchar)c.fr + ((row + xb[1]) << 4));
                 float t0[NCH], t1[NCH];
 #pragma unroll
-                for (int ch = 0; ch < NCH; ++ch) {
-                    t0[ch] = q0[ch];
-                    t1[ch] = q1[ch];
-                }
+                for (int ch = 0; ch < NCH; ++ch) t0[ch] = q0[ch];
+#pragma unroll
+                for (int ch = 0; ch < 3; ++ch) t1[ch] = q1[ch];
                 fc.set_row(k, t0, t1);
             }
         } else {
-            const unsigned base = __umul24((unsigned)((int)mz + 1), c.fsz) + __umul24((unsigned)((int)my + 1), c.fsy) +
-                                  (unsigned)((int)mx + 1);
             // one byte offset for the four rows; each row's start is a
             // block-uniform pointer (scalar arithmetic)
-            const unsigned boff = base << FieldLoad<FT>::kShift;
+            const unsigned boff = clamp_corner(c, m) << FieldLoad<FT>::kShift;
             const size_t off[4] = {0u, (size_t)c.fsy << FieldLoad<FT>::kShift, (size_t)c.fsz << FieldLoad<FT>::kShift,
                                    (size_t)(c.fsz + c.fsy) << FieldLoad<FT>::kShift};
 #pragma unroll
@@ -466,31 +542,30 @@ __device__ __forceinline__ float3 field_from_axes(const CachedArgs& c, FieldCach
         }
     }
     float3 r;
-    r.x = FieldScale<FT>::apply(tri_fc<0>(fc, ax.f, ay.f, az.f));
-    r.y = FieldScale<FT>::apply(tri_fc<1>(fc, ax.f, ay.f, az.f));
-    r.z = FieldScale<FT>::apply(tri_fc<2>(fc, ax.f, ay.f, az.f));
+    r.x = FieldScale<FT>::apply(tri_fc<0>(fc, f.x, f.y, f.z));
+    r.y = FieldScale<FT>::apply(tri_fc<1>(fc, f.x, f.y, f.z));
+    r.z = FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z));
     return r;
 }
 
-// corrector sample: the field cell and the noise cell of the same position.
-// Both fills are issued before either result is used, so the two gathers
-// overlap (one memory round trip instead of two); values and arithmetic
-// are those of field_from_axes and noise_from_axes.
+// corrector sample: the field cell (texel position t) and the noise cell
+// (texel position q) of the same position.  Both fills are issued before
+// either result is used, so the two gathers overlap (one memory round trip
+// instead of two); values and arithmetic are those of field_at and
+// noise_at_cell.
 template <typename FT>
 __device__ __forceinline__ float3 field_and_noise(const LicArgs& a, const CachedArgs& c, FieldCache<FT, 3>& fc,
-                                                  NoiseCache& nc, const Ax& ax, const Ax& ay,
-                                                  const Ax& az, const Ax& nx_, const Ax& ny_,
-                                                  const Ax& nz_, float& noise)
+                                                  NoiseCache& nc, const P3& t, const P3& q, float& noise)
 {
-    const bool fmiss = !key_hit(fc.kx, fc.ky, fc.kz, ax, ay, az);
-    const bool nmiss = !key_hit(nc.kx, nc.ky, nc.kz, nx_, ny_, nz_);
+    P3 f, g;
+    const bool fmiss = !cell_hit(fc, t, f);
+    const bool nmiss = !cell_hit(nc, q, g);
     unsigned short nraw[4];
     constexpr bool kHalf = std::is_same<FT, half4_t>::value;
     RowLoad<half4_t, 3> hrows[kHalf ? 4 : 1];  // FP16: the raw rows until both fills are in flight
     if (fmiss) {
-        const unsigned fb = __umul24(clamp_idx(az.fl, c.fnm1[2]), c.fsz) +
-                            __umul24(clamp_idx(ay.fl, c.fnm1[1]), c.fsy) + clamp_idx(ax.fl, c.fnm1[0]);
-        const unsigned boff = fb << FieldLoad<FT>::kShift;
+        cell_rekey(fc, t, f);
+        const unsigned boff = clamp_corner(c, clamp_floors(c, fc.kx, fc.ky, fc.kz)) << FieldLoad<FT>::kShift;
         const size_t off[4] = {0u, (size_t)c.fsy << FieldLoad<FT>::kShift, (size_t)c.fsz << FieldLoad<FT>::kShift,
                                (size_t)(c.fsz + c.fsy) << FieldLoad<FT>::kShift};
 #pragma unroll
@@ -510,16 +585,13 @@ __device__ __forceinline__ float3 field_and_noise(const LicArgs& a, const Cached
         }
     }
     if (nmiss) {
-        const unsigned nb = __umul24(repeat_idx(nz_.fl, a.noise.n[2]), c.nsz) +
-                            __umul24(repeat_idx(ny_.fl, a.noise.n[1]), c.nsy) + repeat_idx(nx_.fl, a.noise.n[0]);
+        cell_rekey(nc, q, g);
+        const unsigned nb = repeat_corner(a, c, nc);
         const unsigned off[4] = {0u, c.nsy, c.nsz, c.nsz + c.nsy};
 #pragma unroll
         for (int k = 0; k < 4; ++k) nraw[k] = (unsigned short)noise_pair(c.nr, nb + off[k]);
     }
     if (fmiss) {
-        fc.kx = ax.fl;
-        fc.ky = ay.fl;
-        fc.kz = az.fl;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             if constexpr (kHalf) {
@@ -531,9 +603,6 @@ __device__ __forceinline__ float3 field_and_noise(const LicArgs& a, const Cached
         }
     }
     if (nmiss) {
-        nc.kx = nx_.fl;
-        nc.ky = ny_.fl;
-        nc.kz = nz_.fl;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const float t0 = (float)(nraw[k] & 0xffu), t1 = (float)(nraw[k] >> 8);
@@ -541,23 +610,20 @@ __device__ __forceinline__ float3 field_and_noise(const LicArgs& a, const Cached
             nc.dx[k] = t1 - t0;
         }
     }
-    noise = tri_cached(nc.v0, nc.dx, nx_.f, ny_.f, nz_.f);
+    noise = tri_cached(nc.v0, nc.dx, g.x, g.y, g.z);
     float3 r;
-    r.x = FieldScale<FT>::apply(tri_fc<0>(fc, ax.f, ay.f, az.f));
-    r.y = FieldScale<FT>::apply(tri_fc<1>(fc, ax.f, ay.f, az.f));
-    r.z = FieldScale<FT>::apply(tri_fc<2>(fc, ax.f, ay.f, az.f));
+    r.x = FieldScale<FT>::apply(tri_fc<0>(fc, f.x, f.y, f.z));
+    r.y = FieldScale<FT>::apply(tri_fc<1>(fc, f.x, f.y, f.z));
+    r.z = FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z));
     return r;
 }
 
-__device__ __forceinline__ float noise_from_axes(const LicArgs& a, const CachedArgs& c, NoiseCache& nc,
-                                                 const Ax& ax, const Ax& ay, const Ax& az)
+__device__ __forceinline__ float noise_at_cell(const LicArgs& a, const CachedArgs& c, NoiseCache& nc, const P3& t)
 {
-    if (!key_hit(nc.kx, nc.ky, nc.kz, ax, ay, az)) {
-        nc.kx = ax.fl;
-        nc.ky = ay.fl;
-        nc.kz = az.fl;
-        const unsigned base = __umul24(repeat_idx(az.fl, a.noise.n[2]), c.nsz) +
-                              __umul24(repeat_idx(ay.fl, a.noise.n[1]), c.nsy) + repeat_idx(ax.fl, a.noise.n[0]);
+    P3 f;
+    if (!cell_hit(nc, t, f)) {
+        cell_rekey(nc, t, f);
+        const unsigned base = repeat_corner(a, c, nc);
         const unsigned off[4] = {0u, c.nsy, c.nsz, c.nsz + c.nsy};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -568,7 +634,7 @@ __device__ __forceinline__ float noise_from_axes(const LicArgs& a, const CachedA
             nc.dx[k] = t1 - t0;
         }
     }
-    return tri_cached(nc.v0, nc.dx, ax.f, ay.f, az.f);
+    return tri_cached(nc.v0, nc.dx, f.x, f.y, f.z);
 }
 
 // REPEAT corner index (floor mod n) with float arithmetic instead of an
@@ -586,13 +652,12 @@ __device__ __forceinline__ unsigned repeat_idx_f(float fl, float nm1)
     return (unsigned)(int)__builtin_amdgcn_fmed3f(w, 0.0f, nm1);
 }
 
-// noise sample of a REPEAT cell on the field's grid, without the cache (a
-// lane whose streamline left the volume)
-__device__ __forceinline__ float noise_direct(const LicArgs& a, const CachedArgs& c, const Ax& ax, const Ax& ay,
-                                              const Ax& az)
+// noise sample of the REPEAT cell with floors (kx, ky, kz) on the field's
+// grid, without the cache (a lane whose streamline left the volume)
+__device__ __forceinline__ float noise_direct(const CachedArgs& c, float kx, float ky, float kz, const P3& f)
 {
-    const unsigned base = __umul24(repeat_idx_f(az.fl, c.fnm1[2]), c.nsz) +
-                          __umul24(repeat_idx_f(ay.fl, c.fnm1[1]), c.nsy) + repeat_idx_f(ax.fl, c.fnm1[0]);
+    const unsigned base = __umul24(repeat_idx_f(kz, c.fnm1[2]), c.nsz) +
+                          __umul24(repeat_idx_f(ky, c.fnm1[1]), c.nsy) + repeat_idx_f(kx, c.fnm1[0]);
     const unsigned off[4] = {0u, c.nsy, c.nsz, c.nsz + c.nsy};
     float v0[4], dx[4];
 #pragma unroll
@@ -601,22 +666,21 @@ __device__ __forceinline__ float noise_direct(const LicArgs& a, const CachedArgs
         v0[k] = (float)(u & 0xffu);
         dx[k] = (float)(u >> 8) - v0[k];
     }
-    return tri_cached(v0, dx, ax.f, ay.f, az.f);
+    return tri_cached(v0, dx, f.x, f.y, f.z);
 }
 
 // noise of the cell just fetched into fc (SAME): channel 3 of the cache, or
 // the REPEAT array for a cell outside the volume
 template <typename FT>
-__device__ __forceinline__ float noise_same(const LicArgs& a, const CachedArgs& c, const FieldCache<FT, 4>& fc,
-                                            const Ax& ax, const Ax& ay, const Ax& az)
+__device__ __forceinline__ float noise_same(const CachedArgs& c, const FieldCache<FT, 4>& fc, const P3& f)
 {
-    if (fc.same) return tri_fc<3>(fc, ax.f, ay.f, az.f);
-    return noise_direct(a, c, ax, ay, az);
+    if (fc.same) return tri_fc<3>(fc, f.x, f.y, f.z);
+    return noise_direct(c, fc.kx, fc.ky, fc.kz, f);
 }
 
 // LIC of one seed with the per-lane cell caches (scalar noise without gate):
 // the shader's sum of (noise / 255) * weight, before the final scaling by
-// scl.  The noise helpers of the cached path (noise_same, noise_from_axes,
+// scl.  The noise helpers of the cached path (noise_same, noise_at_cell,
 // noise_direct, field_and_noise) return byte units (0..255).  SAME: the noise grid
 // equals the field grid and freq == 1, so the noise cell of the corrector
 // position reuses the corrector's floors and fractions.  The caches may hold
@@ -641,21 +705,21 @@ __device__ __forceinline__ float lic_point_cached(const LicArgs& a, const Cached
                                                   NoiseCache& ncache, float sx, float sy, float sz)
 {
     const int nx = a.field.n[0], ny = a.field.n[1], nz = a.field.n[2];
-    auto noise = [&](float px, float py, float pz, const Ax& ax, const Ax& ay, const Ax& az) -> float {
-        if constexpr (SAME) {
-            return noise_same<FT>(a, c, fc, ax, ay, az);
-        } else {
-            const float q0 = px * a.freq, q1 = py * a.freq, q2 = pz * a.freq;
-            return noise_from_axes(a, c, ncache, axis(q0, a.noise.n[0]), axis(q1, a.noise.n[1]),
-                                   axis(q2, a.noise.n[2]));
-        }
+    auto noise_texel = [&](float px, float py, float pz) {
+        return P3{texel(px * a.freq, a.noise.n[0]), texel(py * a.freq, a.noise.n[1]), texel(pz * a.freq, a.noise.n[2])};
     };
-    Ax ax = axis(sx, nx), ay = axis(sy, ny), az = axis(sz, nz);
-    const float3 s0 = field_from_axes<FT, SAME ? 4 : 3, BRICK>(c, fc, ax, ay, az);
+    P3 f;
+    const float3 s0 =
+        field_at<FT, SAME ? 4 : 3, BRICK>(c, fc, P3{texel(sx, nx), texel(sy, ny), texel(sz, nz)}, f);
+    float n0;
+    if constexpr (SAME)
+        n0 = noise_same<FT>(c, fc, f);
+    else
+        n0 = noise_at_cell(a, c, ncache, noise_texel(sx, sy, sz));
     // the weights are global memory; the cast keeps the batch kernel, which
     // reads this pointer from a descriptor, on scalar loads
     const gfloat* w = (const gfloat*)a.w;
-    float acc = (noise(sx, sy, sz, ax, ay, az) * kInv255) * w[0];
+    float acc = (n0 * kInv255) * w[0];
 
 #pragma unroll 1
     for (int dirn = 0; dirn < 2; ++dirn) {
@@ -674,24 +738,20 @@ __device__ __forceinline__ float lic_point_cached(const LicArgs& a, const Cached
             const float d1z = decode_step(s.z, h);
             const float qx = px + d1x, qy = py + d1y, qz = pz + d1z;
             const float3 s2 =
-                field_from_axes<FT, SAME ? 4 : 3, BRICK>(c, fc, axis(qx, nx), axis(qy, ny), axis(qz, nz));
+                field_at<FT, SAME ? 4 : 3, BRICK>(c, fc, P3{texel(qx, nx), texel(qy, ny), texel(qz, nz)}, f);
             const float d2x = decode_step(s2.x, h);
             const float d2y = decode_step(s2.y, h);
             const float d2z = decode_step(s2.z, h);
             px = fmaf(0.5f, d1x + d2x, px);
             py = fmaf(0.5f, d1y + d2y, py);
             pz = fmaf(0.5f, d1z + d2z, pz);
-            ax = axis(px, nx);
-            ay = axis(py, ny);
-            az = axis(pz, nz);
+            const P3 t{texel(px, nx), texel(py, ny), texel(pz, nz)};
             float nval;
             if constexpr (SAME) {
-                s = field_from_axes<FT, 4, BRICK>(c, fc, ax, ay, az);
-                nval = noise_same<FT>(a, c, fc, ax, ay, az);
+                s = field_at<FT, 4, BRICK>(c, fc, t, f);
+                nval = noise_same<FT>(c, fc, f);
             } else {
-                s = field_and_noise<FT>(a, c, fc, ncache, ax, ay, az, axis(px * a.freq, a.noise.n[0]),
-                                        axis(py * a.freq, a.noise.n[1]), axis(pz * a.freq, a.noise.n[2]),
-                                        nval);
+                s = field_and_noise<FT>(a, c, fc, ncache, t, noise_texel(px, py, pz), nval);
             }
             acc = acc + (nval * kInv255) * wk[i];
         }
@@ -709,6 +769,7 @@ __device__ __forceinline__ CachedArgs cached_args(const LicArgs& a)
     c.fnm1[0] = (float)(a.field.n[0] - 1);
     c.fnm1[1] = (float)(a.field.n[1] - 1);
     c.fnm1[2] = (float)(a.field.n[2] - 1);
+    c.fpx = (float)a.field.sy;
     c.fsy = (unsigned)a.field.sy;
     c.fsz = (unsigned)a.field.sz;
     c.nsy = (unsigned)a.noise.sy;

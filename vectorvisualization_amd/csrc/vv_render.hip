@@ -1677,7 +1677,7 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
     const Vol<FT> fv{(const FT*)a.field.p, {a.field.n[0], a.field.n[1], a.field.n[2]}, a.field.sy, a.field.sz};
     const CachedArgs c = cached_args(L);
     float dest[4] = {0.f, 0.f, 0.f, 0.f};
-    unsigned long long ns = 0;
+    unsigned ns = 0;
     Ray r;
     bool alive;
     // ray policy state
@@ -1704,8 +1704,6 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
         const long long k = bk + sub;
         bool ok;
         float src[4] = {0.f, 0.f, 0.f, 0.f};
-        float nxt[3] = {0.f, 0.f, 0.f};
-        bool nxt_out = true;
         float pos[3];
         Ray rs;
         if constexpr (SLICES) {
@@ -1739,11 +1737,9 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
                 if (outside(pos, vb)) ok = false;
             }
             for (int q = 0; q < 3; ++q) {
-                nxt[q] = fmaf(r.dir[q], a.step, pos[q]);
                 rs.dir[q] = r.dir[q];
                 rs.V[q] = r.V[q];
             }
-            nxt_out = !ok || outside(nxt, vb);
         }
         if (ok) {
             const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
@@ -1812,7 +1808,11 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
         }
         if constexpr (!SLICES) {
             if (alive) {
+                // the next round's first position, from the last lane's sample
                 const int last = gl0 + G - 1;
+                float nxt[3];
+                for (int q = 0; q < 3; ++q) nxt[q] = fmaf(r.dir[q], a.step, pos[q]);
+                const bool nxt_out = !ok || outside(nxt, vb);
                 for (int q = 0; q < 3; ++q) base[q] = __shfl(nxt[q], last);
                 if (__shfl((int)nxt_out, last)) alive = false;
             }
@@ -1826,7 +1826,7 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
         else
             reinterpret_cast<float4*>(a.image)[pix] = make_float4(dest[0], dest[1], dest[2], dest[3]);
     }
-    if (a.counter) add_samples(a.counter, sub == 0 ? ns : 0ull, red);
+    if (a.counter) add_samples(a.counter, sub == 0 ? (unsigned long long)ns : 0ull, red);
 }
 
 }  // namespace
