@@ -1,0 +1,86 @@
+"""Frames through the sample volume (LIC value and field channel in one array)
+equal frames from the two volumes bit for bit.  A context makes it once the
+frames since the last change of either are worth the pass, so a tiny frame
+before a large one reads the volumes and the same frame after it the sample
+volume."""
+import numpy as np
+import pytest
+
+import vectorvisualization_amd as vv
+from vectorvisualization_amd import fields
+
+pytestmark = pytest.mark.gpu
+
+
+def _field(dims, seed):
+    rng = np.random.default_rng(seed)
+    return rng.normal(size=(dims[2], dims[1], dims[0], 3)).astype(np.float32)
+
+
+def _cams(ctx):
+    ext, _, cen = ctx.field_geometry()
+    return (fields.orbit_camera(9, 7, cen, 0.7, 0.4), fields.orbit_camera(300, 260, cen, -0.5, 0.3))
+
+
+def _same(ctx, adjoint=False):
+    """The small frame (and its adjoint) before and after the large one."""
+    small, large = _cams(ctx)
+    out = []
+    for _ in range(2):
+        got = [ctx.render(small)]
+        if adjoint:
+            got.append(ctx.render_record(small))
+            d = np.random.default_rng(2).normal(size=small.width * small.height * 4).astype(np.float32)
+            got += list(ctx.render_adjoint(small, d))
+        out.append(got)
+        ctx.render(large)
+    assert np.max(out[0][0]) > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", [vv.STORE_FP32, vv.STORE_FP16, vv.STORE_UNORM8])
+@pytest.mark.parametrize("dims,spacing", [((40, 33, 37), (1.0, 1.0, 1.0)), ((41, 24, 40), (1.0, 1.5, 2.0)),
+                                          ((36, 40, 44), (0.5, 1.0, 0.7))])
+def test_frames_equal(ctx, storage, dims, spacing):
+    ctx.upload_field(_field(dims, 1), dims, spacing=spacing, storage=storage)
+    ctx.generate_noise(3, vv.NOISE_UNIFORM, 0.0, dims)
+    p = vv.default_lic_params()
+    p.steps_forward = p.steps_backward = 4
+    p.gradient_scale = 4.0
+    ctx.set_lic_params(p)
+    ctx.set_tf(*fields.tf_magnitude(0.05, 0.2))
+    ctx.compute_lic()
+    _same(ctx, adjoint=True)
+    # another TF channel, an opacity scale, another field and another LIC
+    # volume: each drops the sample volume
+    p.tf_index = vv.TF_INDEX_MAG
+    ctx.set_lic_params(p)
+    _same(ctx)
+    ctx.set_opacity_scale(np.random.default_rng(5).uniform(0.5, 1.5, dims[0] * dims[1] * dims[2]).astype(np.float32))
+    _same(ctx, adjoint=True)
+    ctx.upload_field(_field(dims, 9), dims, spacing=spacing, storage=storage)
+    _same(ctx)
+    ctx.upload_lic(np.random.default_rng(6).uniform(0.0, 2.0, dims[0] * dims[1] * dims[2]).astype(np.float32), 1, dims)
+    _same(ctx)
+
+
+def test_stale_sample_volume_is_not_read(ctx):
+    """A frame after each change equals the frame of a fresh context."""
+    dims = (32, 32, 32)
+
+    def load(c, seed, index):
+        c.upload_field(_field(dims, seed), dims)
+        c.generate_noise(seed, vv.NOISE_UNIFORM, 0.0, dims)
+        p = vv.default_lic_params()
+        p.steps_forward = p.steps_backward = 3
+        p.tf_index = index
+        c.set_lic_params(p)
+        c.compute_lic()
+
+    for seed, index in ((1, vv.TF_INDEX_B), (2, vv.TF_INDEX_B), (2, vv.TF_INDEX_MAG), (3, vv.TF_INDEX_B)):
+        load(ctx, seed, index)
+        with vv.Context(0) as fresh:
+            load(fresh, seed, index)
+            for cam in _cams(ctx)[::-1]:
+                assert np.array_equal(ctx.render(cam), fresh.render(cam))

@@ -168,6 +168,7 @@ vv_status vv_upload_field_ex(vv_ctx* c, const float* v0, const float* v1, float 
                 d1 = (const float*)c->stage2.p;
             }
         }
+        drop_pair(c);
         HIPCHK(c, c->field.ensure((size_t)field_texel_bytes(storage) * (size_t)clamp_elems(dims)));
         HIPCHK(c, c->counter.ensure(64));
         uint32_t* maxbits = (uint32_t*)c->counter.p;
@@ -592,8 +593,9 @@ vv_status vv_compute_lic(vv_ctx* c)
         vv_status st = fill_lic_launch(c, L, nullptr);
         if (st) return st;
         const int nc = c->nch;
-        HIPCHK(c, c->lic.ensure(sizeof(float) * nc * (size_t)repeat_elems(c->fdims)));
+        HIPCHK(c, lic_buffer(c, nc, c->fdims));
         L.out = make_repeat_desc(c->lic.p, c->fdims);
+        (void)pair_allowed(c);  // notes a capture
         HIPCHK(c, launch_lic(L, c->stream));  // also writes the REPEAT halo planes
         // the opacity scale lives on the LIC grid: drop it when that grid changes
         if (c->ldims[0] != c->fdims[0] || c->ldims[1] != c->fdims[1] || c->ldims[2] != c->fdims[2])
@@ -647,7 +649,7 @@ vv_status vv_upload_lic(vv_ctx* c, const float* lic, int channels, const int dim
         const size_t bytes = sizeof(float) * channels * (size_t)nvox(dims);
         vv_status st = upload(c, c->stage, lic, bytes, on_device);
         if (st) return st;
-        HIPCHK(c, c->lic.ensure(sizeof(float) * channels * (size_t)repeat_elems(dims)));
+        HIPCHK(c, lic_buffer(c, channels, dims));
         HIPCHK(c, launch_pad_repeat_f32((const float*)c->stage.p, channels, dims, (float*)c->lic.p, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         for (int a = 0; a < 3; ++a) c->ldims[a] = dims[a];
@@ -953,10 +955,10 @@ vv_status vv_set_opacity_scale(vv_ctx* c, const float* sigma, int on_device)
 // Launch descriptor and checkpoint count of an adjoint call.  Samples per ray
 // are bounded by the box diagonal in texture space over the shortest
 // per-step displacement (|dir| >= min scale).
-static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A)
+static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A, bool allow_pair = true)
 {
     std::memset(&A, 0, sizeof(A));
-    vv_status st = fill_render_launch(c, cam, A.r);
+    vv_status st = fill_render_launch(c, cam, A.r, true, allow_pair);
     if (st) return st;
     double diag = 0.0, smin = 1e30;
     for (int a = 0; a < 3; ++a) {
@@ -1163,7 +1165,8 @@ vv_status vv_render_adjoint_noalloc(vv_ctx* c, const vv_camera* cam, const float
                         "line-illumination tables are not on the device: render once with this material first");
         HIPCHK(c, hipSetDevice(c->device));
         AdjointLaunch A;
-        vv_status st = adjoint_setup(c, cam, A);
+        // no sample volume: it may need an allocation, and a captured call would read a stale one
+        vv_status st = adjoint_setup(c, cam, A, false);
         if (st) return st;
         const long long nrays = (long long)cam->width * cam->height;
         const long long nv = nvox(c->ldims);

@@ -38,6 +38,7 @@ struct BatchStep {
     int storage;
     DevBuf field, noise, lic;
     DevBuf lic_field;  // field copy with the noise byte in channel 3 (launch_pack_lic_field)
+    DevBuf pair;       // sample volume of the ray caster (RenderLaunch::pair), made in each run
     int tile[3] = {16, 4, 4};
     int super[3] = {2, 8, 8};
 };
@@ -162,6 +163,7 @@ vv_status build_view_launch(vv_batch* b, const BatchView& v, RenderLaunch& R)
         if (st) return st;
         illum_lut_ptrs(c, R);
     }
+    R.pair_scale = pair_scale(st->storage);
     R.illum_scale = p.illum_scale;
     const float l0 = v.cam.light_pos[0], l1 = v.cam.light_pos[1], l2 = v.cam.light_pos[2];
     const float ld = std::sqrt(l0 * l0 + l1 * l1 + l2 * l2);
@@ -234,6 +236,7 @@ vv_status vv_batch_destroy(vv_batch* b)
             st->noise.release();
             st->lic.release();
             st->lic_field.release();
+            st->pair.release();
             delete st;
         }
         DevBuf* bufs[] = {&b->jobs, &b->first, &b->rviews, &b->vfirst, &b->ctr};
@@ -287,6 +290,7 @@ vv_status vv_batch_add_timestep(vv_batch* b, const float* v0, const int dims[3],
             st->noise.release();
             st->lic.release();
             st->lic_field.release();
+            st->pair.release();
             delete st;
             return s;
         };
@@ -300,6 +304,14 @@ vv_status vv_batch_add_timestep(vv_batch* b, const float* v0, const int dims[3],
         if (!e) e = st->noise.ensure((size_t)repeat_elems(dims));
         if (!e) e = st->lic.ensure(sizeof(float) * (size_t)repeat_elems(dims));
         if (!e) e = st->lic_field.ensure((size_t)field_texel_bytes(storage) * (size_t)clamp_elems(dims));
+        if (!e) {
+            // without memory for it the ray caster samples field and LIC volume
+            const hipError_t ep = st->pair.ensure(sizeof(float) * 2 * (size_t)clamp_elems(dims));
+            if (ep == hipErrorOutOfMemory)
+                (void)hipGetLastError();
+            else
+                e = ep;
+        }
         if (!e) e = c->counter.ensure(64);
         if (!e) e = launch_fill_u32((uint32_t*)c->counter.p, 0u, 1, c->stream);
         if (!e) e = launch_field_maxlen(d0, d0, 0.0f, n, (uint32_t*)c->counter.p, c->stream);
@@ -476,12 +488,26 @@ vv_status vv_batch_run(vv_batch* b)
                 ++k;
             }
             gtiles[g] = b->host_vfirst.back();
+            // the step's sample volume, when its views are worth the pass
+            BatchStep* st = b->steps[t];
+            double samples = 0.0;
+            bool usable = st->pair.p && c->params.illum_mode < VV_ILLUM_MALLO && k > (size_t)b->gview[g];
+            for (size_t v = b->gview[g]; v < k; ++v) {
+                const ViewBlock& vb = b->host_views[v].view;
+                samples += pair_samples(vb.width, vb.height, c->params.step_size_vol);
+                usable = usable && sample_pair_ok(vb.tex_max, st->dims);
+            }
+            if (usable && samples >= kPairSamplesPerVoxel * (double)nvox(st->dims))
+                for (size_t v = b->gview[g]; v < k; ++v) b->host_views[v].pair = (const float*)st->pair.p;
         }
         b->gview[nsteps] = (int)k;
         b->ngroups = (int)nsteps;
         int cus = 0;
         HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-        const int render_grid = cus * render_batch_blocks_per_cu(ftype, 1, bx * by, b->render_group);
+        // persistent blocks of a time step's render launch: all its views have
+        // the step's sample volume or none
+        const int render_grid[2] = {cus * render_batch_blocks_per_cu(ftype, 1, bx * by, b->render_group, 0),
+                                    cus * render_batch_blocks_per_cu(ftype, 1, bx * by, b->render_group, 1)};
         // Descriptors of this run (the graph's kernels read them from device
         // memory).  They are uploaded only when they differ from the last
         // upload, after the previous run has finished reading them; the
@@ -512,7 +538,7 @@ vv_status vv_batch_run(vv_batch* b)
             b->up_vfirst = b->host_vfirst;
             b->up_views.assign(views_bytes, views_bytes + views_size);
         }
-        std::vector<long long> key = {(long long)nsteps, (long long)nv, render_grid, bx, by, b->render_group, ftype, same,
+        std::vector<long long> key = {(long long)nsteps, (long long)nv, render_grid[0], render_grid[1], bx, by, b->render_group, ftype, same,
                                       (long long)(intptr_t)b->jobs.p, (long long)(intptr_t)b->first.p,
                                       (long long)(intptr_t)b->rviews.p, (long long)(intptr_t)b->vfirst.p,
                                       (long long)(intptr_t)b->ctr.p};
@@ -521,6 +547,9 @@ vv_status vv_batch_run(vv_batch* b)
             key.push_back(b->gview[g + 1] - b->gview[g]);
             key.push_back(gtiles[g]);
             key.push_back(b->host_first[2 * b->order[g] + 1]);
+            // the sample volume's pass takes its arguments by value
+            const RenderLaunch* R0 = b->gview[g + 1] > b->gview[g] ? &b->host_views[b->gview[g]] : nullptr;
+            key.push_back(R0 && R0->pair ? R0->tf_ch : -1);
         }
         const bool speed = c->params.speed_of_flow != 0;
         key.push_back(speed);
@@ -562,7 +591,13 @@ vv_status vv_batch_run(vv_batch* b)
                 RB.block[0] = bx;
                 RB.block[1] = by;
                 RB.group = b->render_group;
-                RB.grid = render_grid;
+                const RenderLaunch& R0 = b->host_views[b->gview[g]];
+                RB.pair = R0.pair != nullptr;
+                if (RB.pair)
+                    e = launch_sample_pair(R0.field.p, ftype, R0.tf_ch, (const float*)R0.lic.p, R0.field.n, (float*)R0.pair,
+                                           c->stream);
+                if (e) break;
+                RB.grid = render_grid[RB.pair];
                 RB.field_type = ftype;
                 RB.lc = 1;
                 // the views of this step, after its LIC volume
@@ -727,12 +762,24 @@ vv_status vv_batch_autotune(vv_batch* b)
             static const int blocks[][2] = {{16, 16}, {32, 8}, {64, 4}, {16, 4}, {32, 4}};
             float best = 1e30f;
             int pick[3] = {16, 16, 4};
+            // as the batch renders: through the step's sample volume where it can
+            BatchStep* st0 = b->steps[b->views[0].step];
+            RenderLaunch V;
+            s = build_view_launch(b, b->views[0], V);
+            if (s) return s;
+            float* pair = nullptr;
+            if (st0->pair.p && V.illum < VV_ILLUM_MALLO && sample_pair_ok(V.view.tex_max, st0->dims)) {
+                pair = (float*)st0->pair.p;
+                HIPCHK(c, launch_sample_pair(V.field.p, st0->storage, V.tf_ch, (const float*)V.lic.p, st0->dims, pair,
+                                             c->stream));
+            }
             for (const auto& bl : blocks) {
                 b->render_block[0] = bl[0];
                 b->render_block[1] = bl[1];
                 RenderLaunch R;
                 s = build_view_launch(b, b->views[0], R);
                 if (s) return s;
+                R.pair = pair;
                 hipError_t e = hipSuccess;
                 const float ms = time_ms(c->stream, [&] { return launch_render(R, c->stream); }, 3, &e);
                 if (e) return fail(c, VV_EDEVICE, "autotune render: %s", hipGetErrorString(e));
@@ -747,6 +794,7 @@ vv_status vv_batch_autotune(vv_batch* b)
                 RenderLaunch R;
                 s = build_view_launch(b, b->views[0], R);
                 if (s) return s;
+                R.pair = pair;
                 hipError_t e = hipSuccess;
                 const float ms = time_ms(c->stream, [&] { return launch_render_rg(R, G, c->stream); }, 3, &e);
                 if (e) return fail(c, VV_EDEVICE, "autotune render: %s", hipGetErrorString(e));

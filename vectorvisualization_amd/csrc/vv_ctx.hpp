@@ -100,6 +100,18 @@ struct vv_ctx {
     DevBuf weights;
     std::vector<float> weights_host;  // what `weights` holds
 
+    // the ray casters' sample volume of lic and the field's channel pair_ch
+    // (RenderLaunch::pair), made once the frames since either changed are
+    // worth it; pair_used counts their samples.  It lies behind the LIC volume
+    // in `lic` (lic_buffer), so no frame allocates.
+    void* pair = nullptr;
+    bool pair_ok = false;
+    int pair_ch = 0;
+    double pair_used = 0.0;
+    // a graph that captured the context's LIC or frames replays without its
+    // flags: no sample volume from then on
+    bool pair_off = false;
+
     // launch tuning (vv_set_tuning)
     int lic_tile[3] = {16, 4, 4};
     int lic_super[3] = {2, 16, 16};
@@ -421,9 +433,67 @@ inline void illum_lut_ptrs(vv_ctx* c, RenderLaunch& R)
     R.lut_mallo_spec = base + 256 * 256 * 5;
 }
 
+// whether a sample volume may be used and kept: not while the context's
+// stream is being captured, nor after (vv_ctx::pair_off)
+inline bool pair_allowed(vv_ctx* c)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) c->pair_off = true;
+    return !c->pair_off;
+}
+
+// drops the sample volume of a LIC volume or field about to change
+inline void drop_pair(vv_ctx* c)
+{
+    c->pair_ok = false;
+    c->pair_used = 0.0;
+}
+
+// room for a LIC volume of d voxels and, behind a scalar one, for its sample
+// volume (pair stays null where memory does not suffice)
+inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
+{
+    const size_t lic = (sizeof(float) * channels * (size_t)repeat_elems(d) + 255) / 256 * 256;
+    const size_t pair = channels == 1 ? sizeof(float) * 2 * (size_t)clamp_elems(d) : 0;
+    drop_pair(c);
+    c->pair = nullptr;
+    const hipError_t e = c->lic.ensure(lic + pair);
+    if (e == hipErrorOutOfMemory && pair) {
+        (void)hipGetLastError();
+        return c->lic.ensure(lic);
+    }
+    if (e == hipSuccess && pair) c->pair = (char*)c->lic.p + lic;
+    return e;
+}
+
+// R.pair: the sample volume of the context's scalar LIC volume and field, made
+// here once the frames drawn since they changed are worth the pass
+// (kPairSamplesPerVoxel).  Without it the ray caster samples both volumes.
+inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
+{
+    if (!c->pair || R.illum >= VV_ILLUM_MALLO || !sample_pair_ok(R.view.tex_max, c->fdims)) return VV_OK;
+    for (int a = 0; a < 3; ++a)
+        if (c->ldims[a] != c->fdims[a]) return VV_OK;
+    if (!pair_allowed(c)) return VV_OK;
+    if (!c->pair_ok || c->pair_ch != R.tf_ch) {
+        if (c->pair_ch != R.tf_ch) drop_pair(c);
+        c->pair_ch = R.tf_ch;
+        c->pair_used += pair_samples(R.view.width, R.view.height, R.step);
+        if (c->pair_used < kPairSamplesPerVoxel * (double)nvox(c->fdims)) return VV_OK;
+        HIPCHK(c, launch_sample_pair(c->field.p, c->storage, R.tf_ch, (const float*)c->lic.p, c->fdims, (float*)c->pair,
+                                     c->stream));
+        c->pair_ok = true;
+    }
+    R.pair = (const float*)c->pair;
+    R.pair_scale = pair_scale(c->storage);
+    return VV_OK;
+}
+
 // need_lic: the LIC-volume ray caster; without it (the fused caster) the
 // shading channels are those of the noise
-inline vv_status fill_render_launch(vv_ctx* c, const vv_camera* cam, RenderLaunch& R, bool need_lic = true)
+// (allow_pair: it may sample through ensure_pair's volume)
+inline vv_status fill_render_launch(vv_ctx* c, const vv_camera* cam, RenderLaunch& R, bool need_lic = true,
+                                    bool allow_pair = true)
 {
     if (!c->has_field) return fail(c, VV_ESTATE, "no vector field uploaded");
     if (need_lic && !c->has_lic) return fail(c, VV_ESTATE, "no LIC volume (call vv_compute_lic or vv_upload_lic)");
@@ -475,7 +545,7 @@ inline vv_status fill_render_launch(vv_ctx* c, const vv_camera* cam, RenderLaunc
     if (nt > 256 || nt % 64)
         return fail(c, VV_EINVAL, "render block %dx%d must hold 64, 128, 192 or 256 threads", R.block[0],
                     R.block[1]);
-    return VV_OK;
+    return need_lic && allow_pair ? ensure_pair(c, R) : VV_OK;
 }
 
 }  // namespace vv_host

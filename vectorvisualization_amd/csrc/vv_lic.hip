@@ -430,6 +430,22 @@ __global__ void __launch_bounds__(kThreads) k_repeat_halo_f32(float* vol, int nc
     for (int c = 0; c < nc; ++c) vol[q * nc + c] = vol[s * nc + c];
 }
 
+// The ray casters' sample volume (RenderLaunch::pair).  A pass of its own over
+// 28 bytes per voxel (FP32 field): written at the end of the LIC kernels
+// instead it cost them as much (256^3: 5.59 -> 5.69-5.75 ms), also for a
+// program that draws no frame.  256^3 FP32: 91 us, 5.3 TB/s.
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_sample_pair(const T* field, int ch, const float* lic, int nx, int ny, int nz,
+                                                          float2* pair)
+{
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y, z = blockIdx.z;
+    if (x >= nx + 2 || y >= ny + 2) return;
+    const int ix = x == 0 ? nx - 1 : x - 1, iy = y == 0 ? ny - 1 : y - 1, iz = z == 0 ? nz - 1 : z - 1;
+    const long long q = ((long long)z * (ny + 2) + y) * (nx + 2) + x;
+    // the REPEAT layout holds texel n as a copy of texel 0
+    pair[q] = make_float2(lic[((long long)iz * (ny + 1) + iy) * (nx + 1) + ix], ld1(field + q, 0, ch));
+}
+
 // ---- LIC ---------------------------------------------------------------------
 #include "vv_lic_dev.hpp"
 
@@ -667,6 +683,17 @@ hipError_t launch_unpad_repeat_f32(const float* src, int nc, const int d[3], flo
     hipLaunchKernelGGL(k_unpad_repeat_f32, dim3(blocks_for(n)), dim3(kThreads), 0, s, src, nc, d[0], d[1],
                        d[2], dst);
     return hipGetLastError();
+}
+
+hipError_t launch_sample_pair(const void* field, int field_type, int tf_ch, const float* lic, const int d[3], float* pair,
+                              hipStream_t s)
+{
+    const dim3 block(64, 4), grid((d[0] + 2 + 63) / 64, (d[1] + 2 + 3) / 4, d[2] + 2);
+    return with_field_type(field_type, [&](auto tag) {
+        using FT = typename decltype(tag)::type;
+        hipLaunchKernelGGL(k_sample_pair<FT>, grid, block, 0, s, (const FT*)field, tf_ch, lic, d[0], d[1], d[2],
+                           (float2*)pair);
+    });
 }
 
 hipError_t launch_repeat_halo_f32(float* vol, int nc, const int d[3], hipStream_t s)

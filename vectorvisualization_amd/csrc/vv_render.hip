@@ -11,6 +11,7 @@
 // opacity table live in LDS.  The build is -ffp-contract=off; fmaf marks
 // every fused operation of the shared formulation.
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "vv_device.hpp"
@@ -41,6 +42,16 @@ struct Sample {
 struct Ray {
     float pos[3], dir[3], V[3];
 };
+
+// Source of a ray sample: a field texel type (the LIC value and the TF
+// coordinate from two volumes), or pair_t (both from RenderLaunch::pair: one
+// cell, four 16-byte loads).  Of the eight field-channel loads that pair_t
+// does without, each took 4 bytes of every 16: a strided 4-byte load keeps
+// the L1 busy for 33 to 64 clocks per wave, a 16-byte one for 16 or more
+// (measured).  The line modes of illum >= 2 read the field's direction and
+// take the field types.  1024^2 oblique frame of 256^3, step 1/256: FP32 392 ->
+// 211 us, FP16 468 -> 217, UNORM8 555 -> 220.
+struct pair_t {};
 
 __device__ __forceinline__ void normalize3(const float v[3], float o[3])
 {
@@ -124,76 +135,106 @@ __device__ __forceinline__ bool outside(const float p[3], const ViewBlock& v)
            p[2] < 0.0f || p[2] > v.tex_max[2];
 }
 
+// the four channels of the transfer function at v: lut1d of each, the two
+// table entries read as 16 bytes
+__device__ __forceinline__ void lut_tf(const float* tf, float v, float t4[4])
+{
+    const float x = fmaf(v, 256.0f, -0.5f);
+    float fl = floorf(x);
+    const float f = x - fl;
+    fl = fminf(fmaxf(fl, -1.0f), 255.0f);
+    const int i = (int)fl;
+    const float4 a = reinterpret_cast<const float4*>(tf)[i < 0 ? 0 : i];
+    const float4 b = reinterpret_cast<const float4*>(tf)[i + 1 > 255 ? 255 : i + 1];
+    t4[0] = lerpf(a.x, b.x, f);
+    t4[1] = lerpf(a.y, b.y, f);
+    t4[2] = lerpf(a.z, b.z, f);
+    t4[3] = lerpf(a.w, b.w, f);
+}
+
+// Line illumination (illum 2 and 3) of one sample with the field direction as
+// tangent (vectorData.xyz; tangent = normalize(2 t - 1)); false in the other
+// modes.
+template <typename FT>
+__device__ __forceinline__ bool shade_line(const RenderLaunch& a, const Ray& r, const Vol<FT>& fv, const Cell& cf,
+                                           const float t4[4], float l, Sample& s)
+{
+    if (a.illum < 2) return false;
+    const float g = a.illum_scale;
+    const float3 fr = tri_rgb(fv, cf);
+    const float tg[3] = {fmaf(2.0f, fr.x, -1.0f), fmaf(2.0f, fr.y, -1.0f), fmaf(2.0f, fr.z, -1.0f)};
+    float T[3];
+    normalize3(tg, T);
+    const float* L = a.light;
+    if (a.illum == 3) {
+        // illumZoeckler (inc_illum.glsl:117-154); the table is LUMINANCE_ALPHA,
+        // so .rg reads (L, L): both shading terms are the luminance channel
+        float V[3];
+        normalize3(r.dir, V);
+        const float u = fmaf(0.5f, L[0] * T[0] + L[1] * T[1] + L[2] * T[2], 0.5f);
+        const float w = fmaf(0.5f, V[0] * T[0] + V[1] * T[1] + V[2] * T[2], 0.5f);
+        const float lum = lut2d(a.lut_zoeckler, 2, 0, u, w);
+        const float shr = lum * g;
+        const float sp = 0.9f * lum;
+        for (int c = 0; c < 3; ++c) {
+            s.rgb[c] = (t4[c] * l) * shr + sp;
+            s.m[c] = l * shr;
+        }
+    } else {
+        // illumMallo (inc_illum.glsl:46-113)
+        const float vd[3] = {-r.dir[0], -r.dir[1], -r.dir[2]};
+        float V[3], bn[3], Bv[3], N[3], hv[3], H[3];
+        normalize3(vd, V);
+        bn[0] = T[1] * V[2] - T[2] * V[1];
+        bn[1] = T[2] * V[0] - T[0] * V[2];
+        bn[2] = T[0] * V[1] - T[1] * V[0];
+        normalize3(bn, Bv);
+        N[0] = Bv[1] * T[2] - Bv[2] * T[1];
+        N[1] = Bv[2] * T[0] - Bv[0] * T[2];
+        N[2] = Bv[0] * T[1] - Bv[1] * T[0];
+        for (int c = 0; c < 3; ++c) hv[c] = V[c] + L[c];
+        normalize3(hv, H);
+        const float lx = L[0] * N[0] + L[1] * N[1] + L[2] * N[2];
+        const float ly = L[0] * T[0] + L[1] * T[1] + L[2] * T[2];
+        const float lz = H[0] * N[0] + H[1] * N[1] + H[2] * N[2];
+        const float lw = H[0] * T[0] + H[1] * T[1] + H[2] * T[2];
+        const float ql = sqrtf(fmaxf(1.0f - ly * ly, 0.0f)), qh = sqrtf(fmaxf(1.0f - lw * lw, 0.0f));
+        const float tx = 1.0f / ql, ty = 1.0f / qh;
+        const float ud = fmaf(0.5f, lx * tx, 0.5f);
+        const float vdc = fmaf(0.5f, ly, 0.5f);
+        const float vs = fmaf(0.5f, lz * ty, 0.5f);
+        // pow(tmp.y, -spotExponent) = (1 - (H.T)^2)^(n/2)
+        const float att = ipow(qh, a.spec_exp);
+        for (int c = 0; c < 3; ++c) {
+            const float dif = lut2d(a.lut_mallo_diff, 3, c, ud, vdc) * g;
+            const float spc = clamp01(lut2d(a.lut_mallo_spec, 3, c, ud, vs) * att);
+            s.rgb[c] = (t4[c] * l) * dif + spc;
+            s.m[c] = l * dif;
+        }
+    }
+    return true;
+}
+
 // Shading and opacity of one sample from its LIC value(s) l4 (LC channels):
 // TF lookup, illumination mode, opacity table, opacity scale and the alpha
-// correction.  fv/cf: the field and its cell at pos.
+// correction.  v: the TF coordinate; fv/cf: the field and its cell at pos
+// (pair_t: the cell alone).
 template <typename FT, int LC>
 __device__ __forceinline__ void shade_sample(const RenderLaunch& a, const float* tf, const float* op,
                                              const Ray& r, const float pos[3], const Vol<FT>& fv, const Cell& cf,
-                                             const float l4[4], Sample& s)
+                                             float v, const float l4[4], Sample& s)
 {
-    const float v = tri_ch(fv, cf, a.tf_ch);
     s.tfu = v;
     float t4[4];
-    for (int ch = 0; ch < 4; ++ch) t4[ch] = lut1d(tf, 256, 4, ch, v);
+    lut_tf(tf, v, t4);
     s.tfa = t4[3];
     const float g = a.illum_scale;
     const float l = LC == 1 ? l4[0] : l4[3];
     s.l = l;
-    if (a.illum >= 2) {
-        // line illumination with the field direction as tangent
-        // (vectorData.xyz; tangent = normalize(2 t - 1))
-        const float3 fr = tri_rgb(fv, cf);
-        const float tg[3] = {fmaf(2.0f, fr.x, -1.0f), fmaf(2.0f, fr.y, -1.0f), fmaf(2.0f, fr.z, -1.0f)};
-        float T[3];
-        normalize3(tg, T);
-        const float* L = a.light;
-        if (a.illum == 3) {
-            // illumZoeckler (inc_illum.glsl:117-154); the table is LUMINANCE_ALPHA,
-            // so .rg reads (L, L): both shading terms are the luminance channel
-            float V[3];
-            normalize3(r.dir, V);
-            const float u = fmaf(0.5f, L[0] * T[0] + L[1] * T[1] + L[2] * T[2], 0.5f);
-            const float w = fmaf(0.5f, V[0] * T[0] + V[1] * T[1] + V[2] * T[2], 0.5f);
-            const float lum = lut2d(a.lut_zoeckler, 2, 0, u, w);
-            const float shr = lum * g;
-            const float sp = 0.9f * lum;
-            for (int c = 0; c < 3; ++c) {
-                s.rgb[c] = (t4[c] * l) * shr + sp;
-                s.m[c] = l * shr;
-            }
-        } else {
-            // illumMallo (inc_illum.glsl:46-113)
-            const float vd[3] = {-r.dir[0], -r.dir[1], -r.dir[2]};
-            float V[3], bn[3], Bv[3], N[3], hv[3], H[3];
-            normalize3(vd, V);
-            bn[0] = T[1] * V[2] - T[2] * V[1];
-            bn[1] = T[2] * V[0] - T[0] * V[2];
-            bn[2] = T[0] * V[1] - T[1] * V[0];
-            normalize3(bn, Bv);
-            N[0] = Bv[1] * T[2] - Bv[2] * T[1];
-            N[1] = Bv[2] * T[0] - Bv[0] * T[2];
-            N[2] = Bv[0] * T[1] - Bv[1] * T[0];
-            for (int c = 0; c < 3; ++c) hv[c] = V[c] + L[c];
-            normalize3(hv, H);
-            const float lx = L[0] * N[0] + L[1] * N[1] + L[2] * N[2];
-            const float ly = L[0] * T[0] + L[1] * T[1] + L[2] * T[2];
-            const float lz = H[0] * N[0] + H[1] * N[1] + H[2] * N[2];
-            const float lw = H[0] * T[0] + H[1] * T[1] + H[2] * T[2];
-            const float ql = sqrtf(fmaxf(1.0f - ly * ly, 0.0f)), qh = sqrtf(fmaxf(1.0f - lw * lw, 0.0f));
-            const float tx = 1.0f / ql, ty = 1.0f / qh;
-            const float ud = fmaf(0.5f, lx * tx, 0.5f);
-            const float vdc = fmaf(0.5f, ly, 0.5f);
-            const float vs = fmaf(0.5f, lz * ty, 0.5f);
-            // pow(tmp.y, -spotExponent) = (1 - (H.T)^2)^(n/2)
-            const float att = ipow(qh, a.spec_exp);
-            for (int c = 0; c < 3; ++c) {
-                const float dif = lut2d(a.lut_mallo_diff, 3, c, ud, vdc) * g;
-                const float spc = clamp01(lut2d(a.lut_mallo_spec, 3, c, ud, vs) * att);
-                s.rgb[c] = (t4[c] * l) * dif + spc;
-                s.m[c] = l * dif;
-            }
-        }
+    constexpr bool kPair = std::is_same<FT, pair_t>::value;
+    bool shaded = false;
+    if constexpr (!kPair) shaded = shade_line<FT>(a, r, fv, cf, t4, l, s);
+    if (shaded) {
     } else if (LC == 1 || a.illum == 0) {
         // illumLIC: rgb = illum * tf.rgb * gradient.g
         for (int c = 0; c < 3; ++c) s.rgb[c] = l * t4[c] * g;
@@ -225,7 +266,11 @@ __device__ __forceinline__ void shade_sample(const RenderLaunch& a, const float*
         // per-voxel opacity scale: alpha * sigma, clamped to [0,1]
         const Vol<float> sv{(const float*)a.sigma.p, {a.sigma.n[0], a.sigma.n[1], a.sigma.n[2]},
                             a.sigma.sy, a.sigma.sz};
-        const Cell cs = cell_clamp(sv, pos[0], pos[1], pos[2]);
+        Cell cs;
+        if constexpr (kPair)
+            cs = cf;  // the sample volume's layout is the opacity scale's
+        else
+            cs = cell_clamp(sv, pos[0], pos[1], pos[2]);
         s.sg = tri_f(sv, cs);
         al = al * s.sg;
         if (al > 1.0f) {
@@ -241,32 +286,43 @@ __device__ __forceinline__ void shade_sample(const RenderLaunch& a, const float*
     s.a = 1.0f - pow_corr(1.0f - al, a.alpha_corr, a.corr_mode);
 }
 
-// One sample of the LIC-volume ray caster: LIC value(s) trilinear from the
-// volume, then shade_sample.
+// One sample of the LIC-volume ray caster: LIC value(s) and TF coordinate
+// trilinear from their volumes, then shade_sample.
 template <typename FT, int LC>
 __device__ __forceinline__ void eval_sample(const RenderLaunch& a, const float* tf, const float* op,
                                             const Ray& r, const float pos[3], Sample& s)
 {
-    const Vol<FT> fv{(const FT*)a.field.p, {a.field.n[0], a.field.n[1], a.field.n[2]}, a.field.sy,
-                     a.field.sz};
-    const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
     float l4[4];
-    if constexpr (LC == 1) {
-        const Vol<float> lv{(const float*)a.lic.p, {a.lic.n[0], a.lic.n[1], a.lic.n[2]}, a.lic.sy,
-                            a.lic.sz};
-        const Cell cl = cell_repeat(lv, pos[0], pos[1], pos[2]);
-        l4[0] = tri_f(lv, cl);
+    if constexpr (std::is_same<FT, pair_t>::value) {
+        static_assert(LC == 1, "a scalar LIC volume");
+        typedef float f4 __attribute__((ext_vector_type(4), aligned(8)));
+        const Vol<pair_t> pv{nullptr, {a.field.n[0], a.field.n[1], a.field.n[2]}, a.field.sy, a.field.sz};
+        const Cell c = cell_clamp(pv, pos[0], pos[1], pos[2]);
+        const float2* p = reinterpret_cast<const float2*>(a.pair);
+        const f4 r00 = *reinterpret_cast<const f4*>(p + c.base), r10 = *reinterpret_cast<const f4*>(p + (c.base + pv.sy));
+        const f4 r01 = *reinterpret_cast<const f4*>(p + (c.base + pv.sz));
+        const f4 r11 = *reinterpret_cast<const f4*>(p + (c.base + pv.sz + pv.sy));
+        l4[0] = tri(r00.x, r00.z, r10.x, r10.z, r01.x, r01.z, r11.x, r11.z, c);
+        const float v = tri(r00.y, r00.w, r10.y, r10.w, r01.y, r01.w, r11.y, r11.w, c) * a.pair_scale;
+        shade_sample<FT, LC>(a, tf, op, r, pos, pv, c, v, l4, s);
     } else {
-        const Vol<float4> lv{(const float4*)a.lic.p, {a.lic.n[0], a.lic.n[1], a.lic.n[2]}, a.lic.sy,
-                             a.lic.sz};
-        const Cell cl = cell_repeat(lv, pos[0], pos[1], pos[2]);
-        const float4 q = tri_f4(lv, cl);
-        l4[0] = q.x;
-        l4[1] = q.y;
-        l4[2] = q.z;
-        l4[3] = q.w;
+        const Vol<FT> fv{(const FT*)a.field.p, {a.field.n[0], a.field.n[1], a.field.n[2]}, a.field.sy, a.field.sz};
+        const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
+        if constexpr (LC == 1) {
+            const Vol<float> lv{(const float*)a.lic.p, {a.lic.n[0], a.lic.n[1], a.lic.n[2]}, a.lic.sy, a.lic.sz};
+            const Cell cl = cell_repeat(lv, pos[0], pos[1], pos[2]);
+            l4[0] = tri_f(lv, cl);
+        } else {
+            const Vol<float4> lv{(const float4*)a.lic.p, {a.lic.n[0], a.lic.n[1], a.lic.n[2]}, a.lic.sy, a.lic.sz};
+            const Cell cl = cell_repeat(lv, pos[0], pos[1], pos[2]);
+            const float4 q = tri_f4(lv, cl);
+            l4[0] = q.x;
+            l4[1] = q.y;
+            l4[2] = q.z;
+            l4[3] = q.w;
+        }
+        shade_sample<FT, LC>(a, tf, op, r, pos, fv, cf, tri_ch(fv, cf, a.tf_ch), l4, s);
     }
-    shade_sample<FT, LC>(a, tf, op, r, pos, fv, cf, l4, s);
 }
 
 __device__ __forceinline__ void load_tables(const float* g, float* tf, float* op)
@@ -340,7 +396,7 @@ __device__ __forceinline__ void add_samples(unsigned long long* counter, unsigne
 template <typename FT, int LC>
 __global__ void __launch_bounds__(kRThreads) k_render(RenderLaunch a)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     load_tables(a.tf, tf, op);
@@ -519,7 +575,7 @@ template <typename FT, int LC, int GT>
 __global__ void __launch_bounds__(kRThreads) k_render_rg(RenderLaunch a, int G_rt)
 {
     const int G = GT > 0 ? GT : G_rt;
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     load_tables(a.tf, tf, op);
@@ -545,7 +601,7 @@ k_render_batch(const RenderLaunch* views, const int* first,
                                                            int nviews, int total, unsigned* counter,
                                                            unsigned long long* done, unsigned long long* begun)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     __shared__ int item_s;
@@ -703,7 +759,7 @@ __device__ __forceinline__ AdjColumn adj_column(const AdjointLaunch& A, long lon
 template <typename FT, int LC>
 __global__ void __launch_bounds__(kRThreads) k_adjoint_forward(AdjointLaunch A)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     const RenderLaunch& a = A.r;
@@ -796,7 +852,7 @@ __global__ void __launch_bounds__(kRThreads) k_adjoint_forward_rg(AdjointLaunch 
 {
     static_assert(GT == 2 || GT == 4, "quad groups only");
     static_assert(kSub % GT == 0, "a round lies in one part");
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     const RenderLaunch& a = A.r;
@@ -984,7 +1040,7 @@ __global__ void __launch_bounds__(256) k_adjoint_bound(AdjointLaunch A)
 template <typename FT, int LC>
 __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(4))) k_render_adjoint(AdjointLaunch A)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ long long dtf[1024];
     __shared__ long long win[kWin];
@@ -1182,7 +1238,7 @@ __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(
 k_render_adjoint_rg(AdjointLaunch A)
 {
     static_assert(GT == 2 || GT == 4, "quad groups only");
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ long long dtf[1024];
     __shared__ long long win[kWin];
@@ -1458,7 +1514,7 @@ template <typename FT, int NC, bool GATE, int MODE>
 __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(3)))
 k_render_fused(RenderLaunch a, LicArgs L)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     load_tables(a.tf, tf, op);
@@ -1492,7 +1548,7 @@ k_render_fused(RenderLaunch a, LicArgs L)
                 }
                 const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
                 Sample s;
-                shade_sample<FT, NC>(a, tf, op, r, pos, fv, cf, l4, s);
+                shade_sample<FT, NC>(a, tf, op, r, pos, fv, cf, tri_ch(fv, cf, a.tf_ch), l4, s);
                 composite(dest, s);
                 ++ns;
                 for (int q = 0; q < 3; ++q) pos[q] = fmaf(r.dir[q], a.step, pos[q]);
@@ -1548,7 +1604,7 @@ template <typename FT, int NC, bool GATE, int MODE>
 __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(3)))
 k_render_slices(RenderLaunch a, LicArgs L, SliceSetup S)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     load_tables(a.tf, tf, op);
@@ -1614,7 +1670,7 @@ k_render_slices(RenderLaunch a, LicArgs L, SliceSetup S)
                 l4[3] = acc.w * L.scl;
             }
             Sample s;
-            shade_sample<FT, NC>(a, tf, op, r, pos, fv, cf, l4, s);
+            shade_sample<FT, NC>(a, tf, op, r, pos, fv, cf, tfu, l4, s);
             if (S.blend) {
                 const float src[4] = {s.rgb[0] * s.a, s.rgb[1] * s.a, s.rgb[2] * s.a, s.a};
                 blend_u8(dest, src);
@@ -1655,7 +1711,7 @@ template <typename FT, int NC, bool GATE, int MODE, bool SLICES>
 __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(3)))
 k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
 {
-    __shared__ float tf[1024];
+    __shared__ __align__(16) float tf[1024];
     __shared__ float op[256];
     __shared__ unsigned long long red[kRThreads / 64];
     load_tables(a.tf, tf, op);
@@ -1744,7 +1800,11 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
         if (ok) {
             const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
             bool visible = true;
-            if constexpr (SLICES) visible = lut1d(tf, 256, 4, 3, tri_ch(fv, cf, a.tf_ch)) > 0.05f;
+            float tfu = 0.0f;
+            if constexpr (SLICES) {
+                tfu = tri_ch(fv, cf, a.tf_ch);
+                visible = lut1d(tf, 256, 4, 3, tfu) > 0.05f;
+            }
             if (visible) {
                 float l4[4];
                 if constexpr (MODE > 0) {
@@ -1765,7 +1825,8 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
                     l4[3] = acc.w * L.scl;
                 }
                 Sample sm;
-                shade_sample<FT, NC>(a, tf, op, rs, pos, fv, cf, l4, sm);
+                if constexpr (!SLICES) tfu = tri_ch(fv, cf, a.tf_ch);
+                shade_sample<FT, NC>(a, tf, op, rs, pos, fv, cf, tfu, l4, sm);
                 for (int q = 0; q < 3; ++q) src[q] = sm.rgb[q] * sm.a;
                 src[3] = sm.a;
             } else {
@@ -1829,6 +1890,24 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
     if (a.counter) add_samples(a.counter, sub == 0 ? (unsigned long long)ns : 0ull, red);
 }
 
+// Host-side dispatch of the LIC-volume ray casters: fn(TypeTag<source>{},
+// integral_constant<int, LC>{}).  A scalar LIC volume with its sample volume
+// takes pair_t unless a line mode needs the field's direction.
+template <typename Fn>
+hipError_t with_sample_type(const RenderLaunch& R, Fn&& fn)
+{
+    if (R.pair && R.lc == 1 && R.illum < 2) {
+        fn(TypeTag<pair_t>{}, std::integral_constant<int, 1>{});
+        return hipGetLastError();
+    }
+    return with_field_type(R.field_type, [&](auto tag) {
+        if (R.lc == 4)
+            fn(tag, std::integral_constant<int, 4>{});
+        else
+            fn(tag, std::integral_constant<int, 1>{});
+    });
+}
+
 }  // namespace
 
 hipError_t launch_render(const RenderLaunch& R, hipStream_t s)
@@ -1837,12 +1916,9 @@ hipError_t launch_render(const RenderLaunch& R, hipStream_t s)
     if (bx * by > kRThreads || (bx * by) % 64) return hipErrorInvalidValue;
     dim3 block(bx, by);
     dim3 grid((R.view.width + bx - 1) / bx, (R.view.height + by - 1) / by);
-    return with_field_type(R.field_type, [&](auto tag) {
+    return with_sample_type(R, [&](auto tag, auto lc) {
         using FT = typename decltype(tag)::type;
-        if (R.lc == 4)
-            hipLaunchKernelGGL((k_render<FT, 4>), grid, block, 0, s, R);
-        else
-            hipLaunchKernelGGL((k_render<FT, 1>), grid, block, 0, s, R);
+        hipLaunchKernelGGL((k_render<FT, lc.value>), grid, block, 0, s, R);
     });
 }
 
@@ -1852,25 +1928,18 @@ hipError_t launch_render_rg(const RenderLaunch& R, int G, hipStream_t s)
     const long long nblocks = rg_blocks(G, R.view.width, R.view.height);
     if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
     dim3 grid((unsigned)nblocks), block(kRThreads);
-#define VV_RG_LAUNCH(LC)                                                                    \
-    do {                                                                                    \
-        if (G == 2)                                                                         \
-            hipLaunchKernelGGL((k_render_rg<FT, LC, 2>), grid, block, 0, s, R, G);          \
-        else if (G == 4)                                                                    \
-            hipLaunchKernelGGL((k_render_rg<FT, LC, 4>), grid, block, 0, s, R, G);          \
-        else if (G == 8)                                                                    \
-            hipLaunchKernelGGL((k_render_rg<FT, LC, 8>), grid, block, 0, s, R, G);          \
-        else                                                                                \
-            hipLaunchKernelGGL((k_render_rg<FT, LC, 0>), grid, block, 0, s, R, G);          \
-    } while (0)
-    return with_field_type(R.field_type, [&](auto tag) {
+    return with_sample_type(R, [&](auto tag, auto lc) {
         using FT = typename decltype(tag)::type;
-        if (R.lc == 4)
-            VV_RG_LAUNCH(4);
+        constexpr int LC = lc.value;
+        if (G == 2)
+            hipLaunchKernelGGL((k_render_rg<FT, LC, 2>), grid, block, 0, s, R, G);
+        else if (G == 4)
+            hipLaunchKernelGGL((k_render_rg<FT, LC, 4>), grid, block, 0, s, R, G);
+        else if (G == 8)
+            hipLaunchKernelGGL((k_render_rg<FT, LC, 8>), grid, block, 0, s, R, G);
         else
-            VV_RG_LAUNCH(1);
+            hipLaunchKernelGGL((k_render_rg<FT, LC, 0>), grid, block, 0, s, R, G);
     });
-#undef VV_RG_LAUNCH
 }
 
 namespace {
@@ -2025,29 +2094,19 @@ hipError_t launch_adjoint_forward(const AdjointLaunch& A, hipStream_t s)
         const long long nblocks = rg_blocks(G, A.r.view.width, A.r.view.height);
         if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
         dim3 grid((unsigned)nblocks), block(kRThreads);
-        return with_field_type(A.r.field_type, [&](auto tag) {
+        return with_sample_type(A.r, [&](auto tag, auto lc) {
             using FT = typename decltype(tag)::type;
-            if (A.r.lc == 4) {
-                if (G == 2)
-                    hipLaunchKernelGGL((k_adjoint_forward_rg<FT, 4, 2>), grid, block, 0, s, A);
-                else
-                    hipLaunchKernelGGL((k_adjoint_forward_rg<FT, 4, 4>), grid, block, 0, s, A);
-            } else {
-                if (G == 2)
-                    hipLaunchKernelGGL((k_adjoint_forward_rg<FT, 1, 2>), grid, block, 0, s, A);
-                else
-                    hipLaunchKernelGGL((k_adjoint_forward_rg<FT, 1, 4>), grid, block, 0, s, A);
-            }
+            if (G == 2)
+                hipLaunchKernelGGL((k_adjoint_forward_rg<FT, lc.value, 2>), grid, block, 0, s, A);
+            else
+                hipLaunchKernelGGL((k_adjoint_forward_rg<FT, lc.value, 4>), grid, block, 0, s, A);
         });
     }
     dim3 block(kBX, kBY);
     dim3 grid((A.r.view.width + kBX - 1) / kBX, (A.r.view.height + kBY - 1) / kBY);
-    return with_field_type(A.r.field_type, [&](auto tag) {
+    return with_sample_type(A.r, [&](auto tag, auto lc) {
         using FT = typename decltype(tag)::type;
-        if (A.r.lc == 4)
-            hipLaunchKernelGGL((k_adjoint_forward<FT, 4>), grid, block, 0, s, A);
-        else
-            hipLaunchKernelGGL((k_adjoint_forward<FT, 1>), grid, block, 0, s, A);
+        hipLaunchKernelGGL((k_adjoint_forward<FT, lc.value>), grid, block, 0, s, A);
     });
 }
 
@@ -2060,37 +2119,24 @@ hipError_t launch_render_adjoint(const AdjointLaunch& A, hipStream_t s)
         const long long nblocks = rg_blocks(G, A.r.view.width, A.r.view.height);
         if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
         dim3 grid((unsigned)nblocks), block(kRThreads);
-#define VV_ADJ_RG(LC, GT)                                                                        \
-    do {                                                                                         \
-        if (A.full_col)                                                                          \
-            hipLaunchKernelGGL((k_render_adjoint_rg<FT, LC, GT, false>), grid, block, 0, s, A); \
-        else                                                                                     \
-            hipLaunchKernelGGL((k_render_adjoint_rg<FT, LC, GT, true>), grid, block, 0, s, A);  \
-    } while (0)
-        return with_field_type(A.r.field_type, [&](auto tag) {
+        return with_sample_type(A.r, [&](auto tag, auto lc) {
             using FT = typename decltype(tag)::type;
-            if (A.r.lc == 4) {
-                if (G == 2)
-                    VV_ADJ_RG(4, 2);
-                else
-                    VV_ADJ_RG(4, 4);
-            } else {
-                if (G == 2)
-                    VV_ADJ_RG(1, 2);
-                else
-                    VV_ADJ_RG(1, 4);
-            }
+            constexpr int LC = lc.value;
+            if (G == 2 && A.full_col)
+                hipLaunchKernelGGL((k_render_adjoint_rg<FT, LC, 2, false>), grid, block, 0, s, A);
+            else if (G == 2)
+                hipLaunchKernelGGL((k_render_adjoint_rg<FT, LC, 2, true>), grid, block, 0, s, A);
+            else if (A.full_col)
+                hipLaunchKernelGGL((k_render_adjoint_rg<FT, LC, 4, false>), grid, block, 0, s, A);
+            else
+                hipLaunchKernelGGL((k_render_adjoint_rg<FT, LC, 4, true>), grid, block, 0, s, A);
         });
-#undef VV_ADJ_RG
     }
     dim3 block(kBX, kBY);
     dim3 grid((A.r.view.width + kBX - 1) / kBX, (A.r.view.height + kBY - 1) / kBY);
-    return with_field_type(A.r.field_type, [&](auto tag) {
+    return with_sample_type(A.r, [&](auto tag, auto lc) {
         using FT = typename decltype(tag)::type;
-        if (A.r.lc == 4)
-            hipLaunchKernelGGL((k_render_adjoint<FT, 4>), grid, block, 0, s, A);
-        else
-            hipLaunchKernelGGL((k_render_adjoint<FT, 1>), grid, block, 0, s, A);
+        hipLaunchKernelGGL((k_render_adjoint<FT, lc.value>), grid, block, 0, s, A);
     });
 }
 
@@ -2101,22 +2147,20 @@ hipError_t launch_render_batch(const RenderBatchLaunch& B, hipStream_t s)
     if (B.group == 1 && (bx * by > kRThreads || (bx * by) % 64)) return hipErrorInvalidValue;
     dim3 block = B.group > 1 ? dim3(kRThreads) : dim3(bx, by);
     dim3 grid((unsigned)B.grid);
-#define VV_RB_LAUNCH(LC, GT)                                                                               \
-    hipLaunchKernelGGL((k_render_batch<FT, LC, GT>), grid, block, 0, s, B.views, B.first, B.nviews, B.total, \
-                       B.counter, B.done, B.begun)
-    return with_field_type(B.field_type, [&](auto tag) {
+    RenderLaunch kind{};  // what the views share
+    kind.pair = B.pair ? (const float*)&kind : nullptr;  // only whether it is there counts
+    kind.lc = B.lc;
+    kind.field_type = B.field_type;
+    return with_sample_type(kind, [&](auto tag, auto lc) {
         using FT = typename decltype(tag)::type;
-        if (B.lc == 4) {
-            if (B.group == 4) VV_RB_LAUNCH(4, 4);
-            else if (B.group == 2) VV_RB_LAUNCH(4, 2);
-            else VV_RB_LAUNCH(4, 0);
-        } else {
-            if (B.group == 4) VV_RB_LAUNCH(1, 4);
-            else if (B.group == 2) VV_RB_LAUNCH(1, 2);
-            else VV_RB_LAUNCH(1, 0);
-        }
+        constexpr int LC = lc.value;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, s, B.views, B.first, B.nviews, B.total, B.counter, B.done, B.begun);
+        };
+        if (B.group == 4) launch(k_render_batch<FT, LC, 4>);
+        else if (B.group == 2) launch(k_render_batch<FT, LC, 2>);
+        else launch(k_render_batch<FT, LC, 0>);
     });
-#undef VV_RB_LAUNCH
 }
 
 hipError_t launch_stamp(unsigned long long* t0, hipStream_t s)
@@ -2137,19 +2181,24 @@ hipError_t launch_fixed_to_float(const unsigned long long* hdr, const long long*
 
 namespace vv {
 
-int render_batch_blocks_per_cu(int field_type, int lc, int threads, int group)
+int render_batch_blocks_per_cu(int field_type, int lc, int threads, int group, int pair)
 {
     int n = 0;
     hipError_t e = hipSuccess;
-    const hipError_t d = with_field_type(field_type, [&](auto tag) {
+    RenderLaunch kind{};
+    kind.pair = pair ? (const float*)&kind : nullptr;  // only whether it is there counts
+    kind.lc = lc;
+    kind.field_type = field_type;
+    const hipError_t d = with_sample_type(kind, [&](auto tag, auto lcv) {
         using FT = typename decltype(tag)::type;
+        constexpr int LC = lcv.value;
         auto occ = [&](auto kernel, int nt) { e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, nt, 0); };
         if (group == 4)
-            lc == 4 ? occ(k_render_batch<FT, 4, 4>, kRThreads) : occ(k_render_batch<FT, 1, 4>, kRThreads);
+            occ(k_render_batch<FT, LC, 4>, kRThreads);
         else if (group == 2)
-            lc == 4 ? occ(k_render_batch<FT, 4, 2>, kRThreads) : occ(k_render_batch<FT, 1, 2>, kRThreads);
+            occ(k_render_batch<FT, LC, 2>, kRThreads);
         else
-            lc == 4 ? occ(k_render_batch<FT, 4, 0>, threads) : occ(k_render_batch<FT, 1, 0>, threads);
+            occ(k_render_batch<FT, LC, 0>, threads);
     });
     return (d == hipSuccess && e == hipSuccess && n > 0) ? n : 1;
 }
