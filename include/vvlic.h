@@ -501,9 +501,10 @@ vv_status vv_anim_destroy(vv_anim* a);
  * workload, off by default), "adjoint.window" (0/1: accumulate the opacity-scale gradient in
  * an LDS window per ray segment before the global integer atomics),
  * "render.volume_group" (lanes per ray of vv_render, a power of two up to
- * 64; 1 = one lane per pixel; 0 = 4 for views of 2^18 rays or more, about
- * 2^20 lanes in total below; the forward pass of vv_render_record and of the
- * adjoints and the adjoints' backward walk take the same number up to 4;
+ * 64; 1 = one lane per pixel; 0 = the power of two, at most 16, below
+ * 16 / (step_size_vol sqrt(width height)), at least 1; the forward pass of
+ * vv_render_record and of the adjoints and the adjoints' backward walk take
+ * 4, or the set value if it is smaller;
  * gradients do not depend on it), "render.block_x", "render.block_y" (pixel
  * tile of vv_render with one lane per pixel, 64 to 256 threads in
  * multiples of 64), "render.ray_group" (lanes per ray of vv_render_fused /

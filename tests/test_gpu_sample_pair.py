@@ -84,3 +84,26 @@ def test_stale_sample_volume_is_not_read(ctx):
             load(fresh, seed, index)
             for cam in _cams(ctx)[::-1]:
                 assert np.array_equal(ctx.render(cam), fresh.render(cam))
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf, 3e38])
+def test_groups_with_values_that_are_not_finite(ctx, bad):
+    """Samples that are not finite reach the image as with one lane per pixel
+    (the grouped casters clamp finite rounds with the hardware's modifier,
+    which would drop a NaN)."""
+    dims = (24, 24, 24)
+    ctx.upload_field(_field(dims, 4), dims)
+    lic = np.random.default_rng(8).uniform(0.0, 1.0, (24, 24, 24)).astype(np.float32)
+    lic[12:, 5:9, 7] = bad
+    lic[3, 4, 20:] = -bad
+    ctx.upload_lic(lic, 1, dims)
+    ctx.set_tf(*fields.tf_magnitude(0.05, 0.3))
+    cam = _cams(ctx)[1]
+    cam.width, cam.height = 61, 47
+    img = {}
+    for G in (1, 2, 4, 8, 16, 32):
+        ctx.set_tuning("render.volume_group", G)
+        img[G] = ctx.render(cam, count_samples=True)
+    for G, (im, n) in img.items():
+        np.testing.assert_array_equal(im, img[1][0], err_msg=str(G))
+        assert n == img[1][1]

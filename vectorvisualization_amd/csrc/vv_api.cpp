@@ -740,18 +740,22 @@ vv_status vv_view_block(const vv_ctx* c, const vv_camera* cam, float out24[24])
     });
 }
 
-// Lanes per ray of the LIC-volume caster: the tuning value, else 4 for views
-// of 2^18 rays or more and about 2^20 lanes in all below (at most 64 per
-// ray).  With one lane per pixel the longest rays set the frame time while
-// most waves have finished.  Measured on MI355X (256^3 LIC volume, step
-// 1/256, mean of four views): 1024^2 0.70 -> 0.44 ms (G = 4), 512^2
-// 0.50 -> 0.23 ms (4), 256^2 0.35 -> 0.14 ms (16).
+// Lanes per ray of the LIC-volume caster: the tuning value, else the power of
+// two (at most 16) below 16 L / sqrt(rays), L the steps across the volume.  A
+// ray's lanes share its rounds but every one of them composites all of its
+// samples, so more lanes pay as long as long rays set the time: more of them
+// for longer rays, fewer for views that fill the GPU by themselves.  Mean of
+// four views (us, lanes 1 / 2 / 4 / 8 / 16):
+//   256^3, step 1/256   256^2 193 115  83  68  66,   512^2 207 149 106  99 138,
+//                      1024^2 261 178 174 241 442,  1448^2 244 221 265 411 819
+//   96^3, step 1/128    256^2  71  58  47  45  48,   512^2  69  63  60  65  98,
+//                      1024^2 104  90 105 158 305,  1448^2 114 125 160 268 569
 static int volume_group_for(const vv_ctx* c, const vv_camera* cam)
 {
     if (c->volume_group > 0) return c->volume_group;
-    const long long rays = (long long)cam->width * cam->height;
-    int G = 4;
-    while (G < 64 && rays < (1ll << 18) && rays * G < (1ll << 20)) G *= 2;
+    const double g = 16.0 / ((double)c->params.step_size_vol * std::sqrt((double)cam->width * cam->height));
+    int G = 1;
+    while (G < 16 && 2.0 * G <= g) G *= 2;
     return G;
 }
 
@@ -970,9 +974,9 @@ static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A
     A.r.max_samples = A.r.max_samples < geo ? A.r.max_samples : geo;
     A.max_ckpt = (int)((A.r.max_samples + kAdjSeg - 1) / kAdjSeg);
     A.use_window = c->adj_window;
-    // the forward pass takes the frame's lanes per ray, at most 4
-    const int G = volume_group_for(c, cam);
-    A.group = G >= 4 ? 4 : G;
+    // both walks take 4 lanes per ray unless the tuning asks for fewer (with 2
+    // the voxel boxes of the opacity-scale windows overflow on oblique views)
+    A.group = c->volume_group > 0 && c->volume_group < 4 ? c->volume_group : 4;
     return VV_OK;
 }
 

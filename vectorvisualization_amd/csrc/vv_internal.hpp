@@ -84,9 +84,11 @@ struct ViewBlock {
 // cell of RenderLaunch::pair: no sample of a ray lies past tex_max, whose
 // texel coordinate must stay below n (a spacing below 1 on the longest axis
 // stretches the texture range past the volume, where the LIC volume repeats
-// and the field clamps).
+// and the field clamps).  Its texels are addressed with 32-bit byte offsets
+// and 24-bit row numbers.
 inline bool sample_pair_ok(const float tex_max[3], const int n[3])
 {
+    if (clamp_elems(n) * 8 >= (1ll << 32) || (long long)(n[1] + 2) * (n[2] + 2) >= (1ll << 24)) return false;
     for (int a = 0; a < 3; ++a)
         if (!(tex_max[a] * (float)n[a] - 0.5f < (float)n[a] - 0.25f)) return false;
     return true;
