@@ -541,17 +541,37 @@ vv_status fill_lic_launch(vv_ctx* c, LicLaunch& L, void* out)
     L.field_bytes = (unsigned long long)clamp_elems(c->fdims) * field_texel_bytes(L.field_type);
     L.noise_bytes = (unsigned long long)repeat_elems(c->ndims) * (unsigned long long)nc;
     // the cached kernels address through 32-bit byte offsets
-    // and 24-bit index multiplies (plane strides below 2^24 elements); with
-    // SPEED_OF_FLOW the LIC reads the field's magnitude channel, which the
-    // cached kernels do not keep: the one-lane-per-voxel kernels run
+    // and 24-bit index multiplies (plane strides below 2^24 elements)
     L.speed = p.speed_of_flow;
-    L.cache = c->lic_cache && !L.speed && L.field_bytes < (1ull << 32) && L.noise_bytes < (1ull << 32) &&
-              (long long)L.field.sz < (1ll << 24) && (long long)L.noise.sz < (1ll << 24);
-    // scalar noise on the field's grid at freq 1 (the cached SAME kernels):
-    // the LIC reads the field copy that carries the noise bytes, built once per
-    // field/noise pair.  Without memory for the copy it reads the noise volume.
-    if (L.cache && nc == 1 && !L.gate && L.freq == 1.0f && c->ndims[0] == c->fdims[0] &&
-        c->ndims[1] == c->fdims[1] && c->ndims[2] == c->fdims[2]) {
+    L.cache = c->lic_cache && L.field_bytes < (1ull << 32) && L.noise_bytes < (1ull << 32) &&
+              (long long)L.field.sz < (1ll << 24) && (long long)L.noise.sz < (1ll << 24) &&
+              (!L.gate || (unsigned long long)clamp_elems(c->sdims) < (1ull << 32));
+    // noise on the field's grid: the LIC reads the field copy that carries the
+    // noise bytes, built once per field/noise pair (scalar noise at freq 1 for
+    // every storage, RGBA noise, which has no frequency, for FP32: its texel has
+    // room for the four bytes, and the volume at 128^3 with 20+20 steps takes
+    // .42 ms with the copy, .48 without; in FP16 and UNORM8 the copy would be
+    // wider than the field).  Without memory for the copy it reads the noise
+    // volume.
+    const bool grid = c->ndims[0] == c->fdims[0] && c->ndims[1] == c->fdims[1] && c->ndims[2] == c->fdims[2];
+    if (L.cache && !L.speed && nc == 4 && c->storage == VV_STORE_FP32 && grid) {
+        if (!c->lic_field_ok) {
+            const hipError_t e = c->lic_field.ensure((size_t)L.field_bytes);
+            if (e == hipErrorOutOfMemory) {
+                (void)hipGetLastError();
+            } else {
+                HIPCHK(c, e);
+                HIPCHK(c, launch_pack_lic_field4(c->field.p, c->noise.p, c->fdims, c->lic_field.p, c->stream));
+                c->lic_field_ok = true;
+                c->lic_field_brick = false;
+            }
+        }
+        if (c->lic_field_ok) {
+            L.field.p = c->lic_field.p;
+            L.field_has_noise = 1;
+        }
+    }
+    if (L.cache && !L.speed && nc == 1 && !L.gate && L.freq == 1.0f && grid) {
         long long nb[3];
         brick_counts(c->fdims, nb);
         const size_t brick_bytes = (size_t)(nb[0] * nb[1] * nb[2] * 512) * 16;

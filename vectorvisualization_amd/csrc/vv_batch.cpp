@@ -127,10 +127,9 @@ vv_status build_lic_launch(vv_ctx* c, BatchStep* st, LicLaunch& L)
                     st->dims[0], st->dims[1], st->dims[2]);
     if (p.speed_of_flow) {
         // SPEED_OF_FLOW reads the magnitude channel of the encoded field: the
-        // one-lane-per-voxel kernel on the field itself, not the LIC copy
+        // field itself, not the LIC copy
         L.field = make_clamp_desc(st->field.p, st->dims);
         L.field_has_noise = 0;
-        L.cache = 0;
         L.speed = 1;
     }
     return VV_OK;
@@ -554,7 +553,7 @@ vv_status vv_batch_run(vv_batch* b)
         const bool speed = c->params.speed_of_flow != 0;
         key.push_back(speed);
         if (speed) {
-            // the uncached LIC kernels take their arguments by value: a graph
+            // the single-volume LIC kernels take their arguments by value: a graph
             // holds the arguments it was captured with
             for (size_t i = 0; i + 8 <= b->host_jobs.size(); i += 8) {
                 long long w;

@@ -58,12 +58,30 @@ struct LicLaunch {
     VolDesc out;       // REPEAT layout, float (nc 1) or float4 (nc 4)
     int tile[3];       // threads per block along x,y,z
     int super_tile[3]; // tiles per super-tile along x,y,z (tile order)
-    int cache;         // 1: per-lane cell caches (scalar noise, no gate)
+    int cache;         // 1: per-lane cell caches (every volume within 32-bit byte offsets)
     unsigned long long field_bytes, noise_bytes;  // padded buffer sizes
-    int field_has_noise; // field is the LIC copy: channel 3 = noise byte (same grid)
+    int field_has_noise; // field is the LIC copy: channel 3 = noise byte(s) (same grid)
     int speed;         // SPEED_OF_FLOW: Heun displacements scaled by the field's channel 3
     const void* field_brick;  // float4 LIC copy in 8^3 bricks (launch_pack_lic_field_brick), or null
 };
+
+// Which LIC code a launch takes.
+enum class LicKind {
+    Copy,    // scalar noise in the LIC copy of the field (lic_point_cached SAME)
+    Grid,    // scalar noise on its own grid or frequency (lic_point_cached)
+    Copy4,   // RGBA noise in the LIC copy of an FP32 field (lic_point_cells SAME4)
+    Cells,   // RGBA noise, scalar gate or SPEED_OF_FLOW (lic_point_cells)
+    Direct   // no cell caches (lic_point): tuning, or volumes past 32-bit byte offsets
+};
+
+inline LicKind lic_kind(const LicLaunch& L)
+{
+    if (!L.cache) return LicKind::Direct;
+    const bool grid = L.noise.n[0] == L.field.n[0] && L.noise.n[1] == L.field.n[1] && L.noise.n[2] == L.field.n[2];
+    if (L.speed || L.gate) return LicKind::Cells;
+    if (L.nc == 4) return L.field_has_noise && grid ? LicKind::Copy4 : LicKind::Cells;
+    return L.field_has_noise && grid && L.freq == 1.0f ? LicKind::Copy : LicKind::Grid;
+}
 
 // 8^3-brick order of a CLAMP-padded volume of d + 2 texels per axis: texel
 // (x, y, z) at element ((bz * nby + by) * nbx + bx) * 512 + (lz * 8 + ly) * 8
@@ -269,6 +287,8 @@ hipError_t launch_field_decode(const void* field, int field_type, const int dims
 // texel (p - 1) mod n of CLAMP-padded texel p
 hipError_t launch_pack_lic_field(const void* field, int field_type, const uint8_t* noise, const int dims[3],
                                  void* out, hipStream_t s);
+// the LIC copy of an FP32 field for RGBA noise on its grid: channel 3 = the four noise bytes
+hipError_t launch_pack_lic_field4(const void* field, const void* noise, const int dims[3], void* out, hipStream_t s);
 hipError_t launch_noise_gen(uint64_t seed, int kind, uint64_t thr, const int dims[3],
                             uint8_t* out, hipStream_t s);
 hipError_t launch_noise_grad_raw(const uint8_t* noise, const int dims[3], const float sd[3],

@@ -202,6 +202,20 @@ __global__ void __launch_bounds__(kThreads) k_pack_lic_field(const T* field, con
     }
 }
 
+// the same for RGBA noise (FP32 fields): channel 3 holds the four noise bytes
+__global__ void __launch_bounds__(kThreads) k_pack_lic_field4(const float4* field, const uint32_t* noise, int nx, int ny,
+                                                              int nz, float4* out)
+{
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y, z = blockIdx.z;
+    if (x >= nx + 2 || y >= ny + 2) return;
+    const int ix = x == 0 ? nx - 1 : x - 1, iy = y == 0 ? ny - 1 : y - 1, iz = z == 0 ? nz - 1 : z - 1;
+    const long long q = ((long long)z * (ny + 2) + y) * (nx + 2) + x;
+    float4 v = field[q];
+    // the REPEAT layout holds texel n as a copy of texel 0
+    v.w = __uint_as_float(noise[((long long)iz * (ny + 1) + iy) * (nx + 1) + ix]);
+    out[q] = v;
+}
+
 // the float4 LIC copy reordered into 8^3 bricks (brick_counts): texel (x, y,
 // z) of the padded copy to element ((bz * nby + by) * nbx + bx) * 512 +
 // (lz * 8 + ly) * 8 + lx; elements of bricks past the padded volume are not
@@ -508,23 +522,33 @@ __global__ void __launch_bounds__(kThreads) k_lic_batch(const LicArgs* __restric
     if (tile < a.nblocks) lic_cached_tile<FT, SAME>(a, tile);
 }
 
-template <typename FT, int NC, bool GATE>
-__global__ void __launch_bounds__(kThreads) k_lic(LicArgs a)
+// voxel of this thread in the XCD-ordered tile of its block; false outside the
+// volume
+__device__ __forceinline__ bool lic_voxel(const LicArgs& a, int& x, int& y, int& z)
 {
     // XCD-aware tile order: hardware block b runs on XCD b % 8; give each
     // XCD a contiguous run of tiles so streamlines of neighbouring tiles
     // share that XCD's L2.
     const int b = blockIdx.x;
     const int tile = (b & 7) * a.per_xcd + (b >> 3);
-    if (tile >= a.nblocks) return;
+    if (tile >= a.nblocks) return false;
     int bx, by, bz;
     tile_coords(a, tile, bx, by, bz);
     const int t = threadIdx.x;
-    const int x = bx * a.tx + t % a.tx;
-    const int y = by * a.ty + (t / a.tx) % a.ty;
-    const int z = bz * a.tz + t / (a.tx * a.ty);
+    x = bx * a.tx + t % a.tx;
+    y = by * a.ty + (t / a.tx) % a.ty;
+    z = bz * a.tz + t / (a.tx * a.ty);
+    return x < a.field.n[0] && y < a.field.n[1] && z < a.field.n[2];
+}
+
+// one lane per voxel without cell caches (lic_point): "lic.cache" 0 and
+// volumes past 32-bit byte offsets
+template <typename FT, int NC, bool GATE>
+__global__ void __launch_bounds__(kThreads) k_lic(LicArgs a)
+{
+    int x, y, z;
+    if (!lic_voxel(a, x, y, z)) return;
     const int nx = a.field.n[0], ny = a.field.n[1], nz = a.field.n[2];
-    if (x >= nx || y >= ny || z >= nz) return;
 
     // voxel-centre seed (VV/renderer.cpp:1353-1358, lic3d_volume_fragment.glsl:4-5)
     const float sx = ((float)x + 0.5f) / (float)nx * a.sc0;
@@ -532,6 +556,27 @@ __global__ void __launch_bounds__(kThreads) k_lic(LicArgs a)
     const float sz = ((float)z + 0.5f) / (float)nz * a.sc2;
 
     const float4 acc = lic_point<FT, NC, GATE>(a, sx, sy, sz);
+    if constexpr (NC == 1) {
+        store_repeat<float>(a.out, a.osy, a.osz, x, y, z, nx, ny, nz, acc.x * a.scl);  // lic3d_volume_fragment.glsl:15
+    } else {
+        store_repeat<float4>(reinterpret_cast<float4*>(a.out), a.osy, a.osz, x, y, z, nx, ny, nz,
+                             make_float4(acc.x, acc.y, acc.z, acc.w * a.scl));
+    }
+}
+
+// k_lic with per-lane cell caches (lic_point_cells)
+template <typename FT, int NC, bool GATE, bool SPEED, bool SAME4>
+__global__ void __launch_bounds__(kThreads) k_lic_cells(LicArgs a)
+{
+    int x, y, z;
+    if (!lic_voxel(a, x, y, z)) return;
+    const int nx = a.field.n[0], ny = a.field.n[1], nz = a.field.n[2];
+    // voxel-centre seed (VV/renderer.cpp:1353-1358, lic3d_volume_fragment.glsl:4-5)
+    const float sx = ((float)x + 0.5f) / (float)nx * a.sc0;
+    const float sy = ((float)y + 0.5f) / (float)ny * a.sc1;
+    const float sz = ((float)z + 0.5f) / (float)nz * a.sc2;
+    const CachedArgs c = cached_args(a);
+    const float4 acc = lic_point_cells<FT, NC, GATE, SPEED, SAME4>(a, c, sx, sy, sz);
     if constexpr (NC == 1) {
         store_repeat<float>(a.out, a.osy, a.osz, x, y, z, nx, ny, nz, acc.x * a.scl);  // lic3d_volume_fragment.glsl:15
     } else {
@@ -585,6 +630,14 @@ hipError_t launch_field_decode(const void* field, int field_type, const int d[3]
         hipLaunchKernelGGL(k_field_decode<FT>, dim3(blocks_for(n)), dim3(kThreads), 0, s, (const FT*)field, d[0],
                            d[1], d[2], (float4*)out4);
     });
+}
+
+hipError_t launch_pack_lic_field4(const void* field, const void* noise, const int d[3], void* out, hipStream_t s)
+{
+    const dim3 block(64, 4), grid((d[0] + 2 + 63) / 64, (d[1] + 2 + 3) / 4, d[2] + 2);
+    hipLaunchKernelGGL(k_pack_lic_field4, grid, block, 0, s, (const float4*)field, (const uint32_t*)noise, d[0], d[1], d[2],
+                       (float4*)out);
+    return hipGetLastError();
 }
 
 hipError_t launch_pack_lic_field(const void* field, int field_type, const uint8_t* noise, const int d[3], void* out,
@@ -756,15 +809,11 @@ hipError_t launch_lic(const LicLaunch& L, hipStream_t s)
     if (e != hipSuccess) return e;
     dim3 grid((unsigned)(a.per_xcd * 8));
     dim3 block(kThreads);
-    const bool g = L.gate != 0;
-    const bool cached = L.cache && L.nc == 1 && !g;
-    // the SAME kernels read the noise from channel 3 of the LIC field copy
-    const bool same = L.field_has_noise && L.freq == 1.0f && L.noise.n[0] == L.field.n[0] &&
-                      L.noise.n[1] == L.field.n[1] && L.noise.n[2] == L.field.n[2];
+    const LicKind v = lic_kind(L);
     return with_field_type(L.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
         if constexpr (std::is_same<FT, float4>::value) {
-            if (cached && same && L.field_brick) {
+            if (v == LicKind::Copy && L.field_brick) {
                 // the LIC volume kernel alone reads the brick copy
                 long long nb[3];
                 const int d[3] = {L.field.n[0], L.field.n[1], L.field.n[2]};
@@ -777,16 +826,28 @@ hipError_t launch_lic(const LicLaunch& L, hipStream_t s)
                 return;
             }
         }
-        if (cached && same)
-            hipLaunchKernelGGL((k_lic_cached<FT, true>), grid, block, 0, s, a);
-        else if (cached)
-            hipLaunchKernelGGL((k_lic_cached<FT, false>), grid, block, 0, s, a);
-        else if (L.nc == 4)
-            hipLaunchKernelGGL((k_lic<FT, 4, false>), grid, block, 0, s, a);
-        else if (g)
-            hipLaunchKernelGGL((k_lic<FT, 1, true>), grid, block, 0, s, a);
-        else
-            hipLaunchKernelGGL((k_lic<FT, 1, false>), grid, block, 0, s, a);
+        auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
+        const bool g = L.gate != 0;
+        switch (v) {
+        case LicKind::Copy: run(k_lic_cached<FT, true>); break;
+        case LicKind::Grid: run(k_lic_cached<FT, false>); break;
+        case LicKind::Copy4:
+            if constexpr (std::is_same<FT, float4>::value) run(k_lic_cells<FT, 4, false, false, true>);
+            break;
+        case LicKind::Cells:
+            if (L.speed)
+                L.nc == 4 ? run(k_lic_cells<FT, 4, false, true, false>)
+                : g       ? run(k_lic_cells<FT, 1, true, true, false>)
+                          : run(k_lic_cells<FT, 1, false, true, false>);
+            else if (L.nc == 4)
+                run(k_lic_cells<FT, 4, false, false, false>);
+            else
+                run(k_lic_cells<FT, 1, true, false, false>);
+            break;
+        case LicKind::Direct:
+            L.nc == 4 ? run(k_lic<FT, 4, false>) : g ? run(k_lic<FT, 1, true>) : run(k_lic<FT, 1, false>);
+            break;
+        }
     });
 }
 

@@ -254,6 +254,33 @@ struct FieldCache<float4, 4> {
     }
 };
 
+// FP32 texels read as four plain floats (SPEED_OF_FLOW: the magnitude), and
+// the LIC copy of an FP32 field for RGBA noise on its grid, whose channel 3
+// holds the four noise bytes of the texel
+struct plain4_t {};
+struct copy4_t {};
+
+template <>
+struct FieldCache<copy4_t, 4> {
+    float kx, ky, kz;
+    bool same;
+    float v0[3][4], dx[3][4];
+    unsigned w0[4], w1[4];  // noise bytes of the texels at x0 and x1
+    __device__ __forceinline__ void reset() { kx = ky = kz = __builtin_nanf(""); same = false; }
+    template <int CH>
+    __device__ __forceinline__ float xlerp(int k, float fx) const { return fmaf(fx, dx[CH][k], v0[CH][k]); }
+    __device__ __forceinline__ void set_row(int k, const float* t0, const float* t1)
+    {
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) {
+            v0[ch][k] = t0[ch];
+            dx[ch][k] = t1[ch] - t0[ch];
+        }
+        w0[k] = __float_as_uint(t0[3]);
+        w1[k] = __float_as_uint(t1[3]);
+    }
+};
+
 // FP16 texels: the x0 texel of each corner row stays as the two words the
 // row load returned (channels 0|1 and 2|3, low half first), the differences
 // are floats; x-lerps and differences read the halves with fma_half and
@@ -388,6 +415,25 @@ struct FieldLoad<float4> {
     }
 };
 
+// two 16-byte loads (x0 and x1)
+struct Load4x2 {
+    static constexpr unsigned kShift = 4;
+    template <int NCH>
+    __device__ static __forceinline__ void pair(const char* base, unsigned off, float* t0, float* t1)
+    {
+        const gfloat* q = (const gfloat*)((gchar)base + off);
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            t0[ch] = q[ch];
+            t1[ch] = q[4 + ch];
+        }
+    }
+};
+template <>
+struct FieldLoad<plain4_t> : Load4x2 {};
+template <>
+struct FieldLoad<copy4_t> : Load4x2 {};
+
 // half4 texels: one 16-byte load holds x0 and x1, kept as the raw words for
 // the FP16 cell cache
 template <>
@@ -498,6 +544,15 @@ __device__ __forceinline__ unsigned repeat_corner(const LicArgs& a, const Cached
 // arithmetic are those of noise_at_cell.  field_at sets fc.same for a cell
 // whose three floors lie in that range.
 
+// rgb of the cached cell at fractions f
+template <typename FT, int NCH>
+__device__ __forceinline__ float3 field_rgb_of(const FieldCache<FT, NCH>& fc, const P3& f)
+{
+    return make_float3(FieldScale<FT>::apply(tri_fc<0>(fc, f.x, f.y, f.z)),
+                       FieldScale<FT>::apply(tri_fc<1>(fc, f.x, f.y, f.z)),
+                       FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z)));
+}
+
 template <typename FT, int NCH, bool BRICK = false>
 __device__ __forceinline__ float3 field_at(const CachedArgs& c, FieldCache<FT, NCH>& fc, const P3& t, P3& f)
 {
@@ -541,12 +596,80 @@ __device__ __forceinline__ float3 field_at(const CachedArgs& c, FieldCache<FT, N
             }
         }
     }
-    float3 r;
-    r.x = FieldScale<FT>::apply(tri_fc<0>(fc, f.x, f.y, f.z));
-    r.y = FieldScale<FT>::apply(tri_fc<1>(fc, f.x, f.y, f.z));
-    r.z = FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z));
-    return r;
+    return field_rgb_of(fc, f);
 }
+
+// A field fill in two steps, so that a noise fill can be issued between its
+// loads and their first use: issue() rekeys the cache to t's cell and starts
+// the loads, finish() makes the cache's values of them.  Float caches hold the
+// raw x1 texel in dx meanwhile, the FP16 cache takes its raw rows.
+template <typename FT, int NCH>
+struct FieldFill {
+    __device__ __forceinline__ void issue(const CachedArgs& c, FieldCache<FT, NCH>& fc, const P3& t, P3& f)
+    {
+        cell_rekey(fc, t, f);
+        const unsigned boff = clamp_corner(c, clamp_floors(c, fc.kx, fc.ky, fc.kz)) << FieldLoad<FT>::kShift;
+        const size_t off[4] = {0u, (size_t)c.fsy << FieldLoad<FT>::kShift, (size_t)c.fsz << FieldLoad<FT>::kShift,
+                               (size_t)(c.fsz + c.fsy) << FieldLoad<FT>::kShift};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float t0[NCH], t1[NCH];
+            FieldLoad<FT>::template pair<NCH>(c.fr + off[k], boff, t0, t1);
+#pragma unroll
+            for (int ch = 0; ch < NCH; ++ch) {
+                fc.v0[ch][k] = t0[ch];
+                fc.dx[ch][k] = t1[ch];
+            }
+        }
+    }
+    __device__ __forceinline__ void finish(FieldCache<FT, NCH>& fc)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int ch = 0; ch < NCH; ++ch) fc.dx[ch][k] = fc.dx[ch][k] - fc.v0[ch][k];
+    }
+};
+
+template <int NCH>
+struct FieldFill<half4_t, NCH> {
+    RowLoad<half4_t, NCH> rows[4];
+    __device__ __forceinline__ void issue(const CachedArgs& c, FieldCache<half4_t, NCH>& fc, const P3& t, P3& f)
+    {
+        cell_rekey(fc, t, f);
+        const unsigned boff = clamp_corner(c, clamp_floors(c, fc.kx, fc.ky, fc.kz)) << FieldLoad<half4_t>::kShift;
+        const size_t off[4] = {0u, (size_t)c.fsy << 3, (size_t)c.fsz << 3, (size_t)(c.fsz + c.fsy) << 3};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) rows[k].load(c.fr + off[k], boff);
+    }
+    __device__ __forceinline__ void finish(FieldCache<half4_t, NCH>& fc)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) rows[k].store(fc, k);
+    }
+};
+
+// the noise fill of a scalar cell in the same two steps
+struct NoiseFill {
+    unsigned short raw[4];
+    __device__ __forceinline__ void issue(const LicArgs& a, const CachedArgs& c, NoiseCache& nc, const P3& q, P3& g)
+    {
+        cell_rekey(nc, q, g);
+        const unsigned nb = repeat_corner(a, c, nc);
+        const unsigned off[4] = {0u, c.nsy, c.nsz, c.nsz + c.nsy};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) raw[k] = (unsigned short)noise_pair(c.nr, nb + off[k]);
+    }
+    __device__ __forceinline__ void finish(NoiseCache& nc) const
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float t0 = (float)(raw[k] & 0xffu), t1 = (float)(raw[k] >> 8);
+            nc.v0[k] = t0;
+            nc.dx[k] = t1 - t0;
+        }
+    }
+};
 
 // corrector sample: the field cell (texel position t) and the noise cell
 // (texel position q) of the same position.  Both fills are issued before
@@ -560,62 +683,14 @@ __device__ __forceinline__ float3 field_and_noise(const LicArgs& a, const Cached
     P3 f, g;
     const bool fmiss = !cell_hit(fc, t, f);
     const bool nmiss = !cell_hit(nc, q, g);
-    unsigned short nraw[4];
-    constexpr bool kHalf = std::is_same<FT, half4_t>::value;
-    RowLoad<half4_t, 3> hrows[kHalf ? 4 : 1];  // FP16: the raw rows until both fills are in flight
-    if (fmiss) {
-        cell_rekey(fc, t, f);
-        const unsigned boff = clamp_corner(c, clamp_floors(c, fc.kx, fc.ky, fc.kz)) << FieldLoad<FT>::kShift;
-        const size_t off[4] = {0u, (size_t)c.fsy << FieldLoad<FT>::kShift, (size_t)c.fsz << FieldLoad<FT>::kShift,
-                               (size_t)(c.fsz + c.fsy) << FieldLoad<FT>::kShift};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if constexpr (kHalf) {
-                hrows[k].load(c.fr + off[k], boff);
-            } else {
-                // float caches hold the raw x1 texel in dx until both fills are in flight
-                float t0[3], t1[3];
-                FieldLoad<FT>::template pair<3>(c.fr + off[k], boff, t0, t1);
-#pragma unroll
-                for (int ch = 0; ch < 3; ++ch) {
-                    fc.v0[ch][k] = t0[ch];
-                    fc.dx[ch][k] = t1[ch];
-                }
-            }
-        }
-    }
-    if (nmiss) {
-        cell_rekey(nc, q, g);
-        const unsigned nb = repeat_corner(a, c, nc);
-        const unsigned off[4] = {0u, c.nsy, c.nsz, c.nsz + c.nsy};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) nraw[k] = (unsigned short)noise_pair(c.nr, nb + off[k]);
-    }
-    if (fmiss) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if constexpr (kHalf) {
-                hrows[k].store(fc, k);
-            } else {
-#pragma unroll
-                for (int ch = 0; ch < 3; ++ch) fc.dx[ch][k] = fc.dx[ch][k] - fc.v0[ch][k];
-            }
-        }
-    }
-    if (nmiss) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float t0 = (float)(nraw[k] & 0xffu), t1 = (float)(nraw[k] >> 8);
-            nc.v0[k] = t0;
-            nc.dx[k] = t1 - t0;
-        }
-    }
+    FieldFill<FT, 3> ff;
+    NoiseFill nf;
+    if (fmiss) ff.issue(c, fc, t, f);
+    if (nmiss) nf.issue(a, c, nc, q, g);
+    if (fmiss) ff.finish(fc);
+    if (nmiss) nf.finish(nc);
     noise = tri_cached(nc.v0, nc.dx, g.x, g.y, g.z);
-    float3 r;
-    r.x = FieldScale<FT>::apply(tri_fc<0>(fc, f.x, f.y, f.z));
-    r.y = FieldScale<FT>::apply(tri_fc<1>(fc, f.x, f.y, f.z));
-    r.z = FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z));
-    return r;
+    return field_rgb_of(fc, f);
 }
 
 __device__ __forceinline__ float noise_at_cell(const LicArgs& a, const CachedArgs& c, NoiseCache& nc, const P3& t)
@@ -775,6 +850,216 @@ __device__ __forceinline__ CachedArgs cached_args(const LicArgs& a)
     c.nsy = (unsigned)a.noise.sy;
     c.nsz = (unsigned)a.noise.sz;
     return c;
+}
+
+// ---- cell caches for RGBA noise, the scalar gate and SPEED_OF_FLOW -----------
+//
+// lic_point_cells is lic_point with the field, noise and gate cells of each
+// streamline kept in registers as in lic_point_cached; values and order of the
+// arithmetic are lic_point's.  Of an RGBA noise cell it keeps the eight texels
+// as loaded and converts their bytes where they are blended: some lane of a
+// wave enters a new cell on nearly every step, so converting on the fill
+// would not be rarer, and 8 words take the registers of 32 floats.  An FP32
+// field with the noise on its grid reads the bytes from channel 3 of its LIC
+// copy (SAME4), which spares the L1 the noise loads.  Bound by the vector ALU
+// (RGBA: the four blends; gate: three cells' hits) and, in FP32, by the L1.
+// LIC volume at 128^3, 20+20 steps, without and with the caches: FP32 RGBA
+// .91 -> .42 ms (.48 with the noise from its volume), gate 1.11 -> .53,
+// SPEED_OF_FLOW .87 -> .43; FP16 .71 -> .51, .89 -> .46, .68 -> .49; UNORM8
+// .70 -> .52, .86 -> .45, .68 -> .47.
+
+// blended noise bytes (0..255) of a cell: channel CH of w0/w1
+template <int CH>
+__device__ __forceinline__ float tri_bytes(const unsigned* w0, const unsigned* w1, const P3& f)
+{
+    float x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float a = (float)((w0[k] >> (8 * CH)) & 0xffu), b = (float)((w1[k] >> (8 * CH)) & 0xffu);
+        x[k] = lerpf(a, b, f.x);
+    }
+    return lerpf(lerpf(x[0], x[1], f.y), lerpf(x[2], x[3], f.y), f.z);
+}
+
+__device__ __forceinline__ float4 rgba_bytes(const unsigned* w0, const unsigned* w1, const P3& f)
+{
+    return make_float4(tri_bytes<0>(w0, w1, f) * kInv255, tri_bytes<1>(w0, w1, f) * kInv255,
+                       tri_bytes<2>(w0, w1, f) * kInv255, tri_bytes<3>(w0, w1, f) * kInv255);
+}
+
+// four rows of an RGBA noise cell from texel `corner`
+__device__ __forceinline__ void load_rgba_rows(const CachedArgs& c, unsigned corner, unsigned* w0, unsigned* w1)
+{
+    const unsigned off[4] = {0u, c.nsy, c.nsz, c.nsz + c.nsy};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const gu32* q = (const gu32*)((gchar)(const char*)c.nr + ((corner + off[k]) << 2));
+        w0[k] = q[0];
+        w1[k] = q[1];
+    }
+}
+
+struct RgbaCache {
+    float kx, ky, kz;
+    unsigned w0[4], w1[4];
+    __device__ __forceinline__ void reset() { kx = ky = kz = __builtin_nanf(""); }
+};
+
+// byte of the scalar gate volume (CLAMP layout), blended, at its texel position
+struct GateCache : NoiseCache {
+    __device__ __forceinline__ float at(const Vol<uint8_t>& v, const P3& t)
+    {
+        P3 f;
+        if (!cell_hit(*this, t, f)) {
+            cell_rekey(*this, t, f);
+            const int x = (int)__builtin_amdgcn_fmed3f(kx, -1.0f, (float)(v.n[0] - 1)) + 1;
+            const int y = (int)__builtin_amdgcn_fmed3f(ky, -1.0f, (float)(v.n[1] - 1)) + 1;
+            const int z = (int)__builtin_amdgcn_fmed3f(kz, -1.0f, (float)(v.n[2] - 1)) + 1;
+            const unsigned base = (unsigned)z * (unsigned)v.sz + (unsigned)y * (unsigned)v.sy + (unsigned)x;
+            const unsigned off[4] = {0u, (unsigned)v.sy, (unsigned)v.sz, (unsigned)(v.sz + v.sy)};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const unsigned u = noise_pair(v.p, base + off[k]);
+                const float t0 = (float)(u & 0xffu), t1 = (float)(u >> 8);
+                v0[k] = t0;
+                dx[k] = t1 - t0;
+            }
+        }
+        return tri_cached(v0, dx, f.x, f.y, f.z);
+    }
+};
+
+template <typename FT, int NC, bool GATE, bool SPEED, bool SAME4>
+struct LicCells {
+    static_assert(!SAME4 || (NC == 4 && !SPEED && std::is_same<FT, float4>::value), "FP32 LIC copy with RGBA noise");
+    using T32 = typename std::conditional<SAME4, copy4_t, plain4_t>::type;
+    using T = typename std::conditional<std::is_same<FT, float4>::value && (SAME4 || SPEED), T32, FT>::type;
+    static constexpr int NCH = SAME4 || SPEED ? 4 : 3;
+    FieldCache<T, NCH> fc;
+    NoiseCache nc;
+    RgbaCache rc;
+    GateCache gc;
+
+    __device__ __forceinline__ void reset()
+    {
+        fc.reset();
+        nc.reset();
+        rc.reset();
+        gc.reset();
+    }
+
+    // direction, and the magnitude in w with SPEED
+    __device__ __forceinline__ float4 with_magnitude(const float3& s, const P3& f) const
+    {
+        float w = 1.0f;
+        if constexpr (SPEED) w = FieldScale<FT>::apply(tri_fc<3>(fc, f.x, f.y, f.z));
+        return make_float4(s.x, s.y, s.z, w);
+    }
+
+    // the field at texel position t and the noise at texture position p
+    __device__ __forceinline__ float4 field_noise(const LicArgs& a, const CachedArgs& c, const P3& t, float px, float py,
+                                                  float pz, float4& n)
+    {
+        P3 f, g;
+        n = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (SAME4) {
+            const float3 s = field_at<T, NCH>(c, fc, t, f);
+            if (fc.same) {
+                n = rgba_bytes(fc.w0, fc.w1, f);
+            } else {
+                unsigned w0[4], w1[4];
+                load_rgba_rows(c, __umul24(repeat_idx(fc.kz, a.noise.n[2]), c.nsz) +
+                                      __umul24(repeat_idx(fc.ky, a.noise.n[1]), c.nsy) + repeat_idx(fc.kx, a.noise.n[0]),
+                               w0, w1);
+                n = rgba_bytes(w0, w1, f);
+            }
+            return make_float4(s.x, s.y, s.z, 1.0f);
+        } else {
+            const bool fmiss = !cell_hit(fc, t, f);
+            FieldFill<T, NCH> ff;
+            if constexpr (NC == 4) {
+                const P3 q{texel(px, a.noise.n[0]), texel(py, a.noise.n[1]), texel(pz, a.noise.n[2])};
+                const bool nmiss = !cell_hit(rc, q, g);
+                if (fmiss) ff.issue(c, fc, t, f);
+                if (nmiss) {
+                    cell_rekey(rc, q, g);
+                    load_rgba_rows(c, __umul24(repeat_idx(rc.kz, a.noise.n[2]), c.nsz) +
+                                          __umul24(repeat_idx(rc.ky, a.noise.n[1]), c.nsy) +
+                                          repeat_idx(rc.kx, a.noise.n[0]),
+                                   rc.w0, rc.w1);
+                }
+                if (fmiss) ff.finish(fc);
+                n = rgba_bytes(rc.w0, rc.w1, g);
+            } else {
+                bool open = true;
+                if constexpr (GATE) {
+                    const float s = gc.at(a.scalar, P3{texel(px, a.scalar.n[0]), texel(py, a.scalar.n[1]),
+                                                       texel(pz, a.scalar.n[2])}) * kInv255;
+                    open = s > a.gate_lo && s < a.gate_hi;
+                }
+                const P3 q{texel(px * a.freq, a.noise.n[0]), texel(py * a.freq, a.noise.n[1]),
+                           texel(pz * a.freq, a.noise.n[2])};
+                const bool nmiss = open && !cell_hit(nc, q, g);
+                NoiseFill nf;
+                if (fmiss) ff.issue(c, fc, t, f);
+                if (nmiss) nf.issue(a, c, nc, q, g);
+                if (fmiss) ff.finish(fc);
+                if (nmiss) nf.finish(nc);
+                if (open) n.x = tri_cached(nc.v0, nc.dx, g.x, g.y, g.z) * kInv255;
+            }
+            return with_magnitude(field_rgb_of(fc, f), f);
+        }
+    }
+};
+
+// step of one axis: decode_step, or with SPEED the shader's ((2s - 1) a) h
+template <bool SPEED>
+__device__ __forceinline__ float cell_step(float s, float a, float h)
+{
+    return SPEED ? (fmaf(2.0f, s, -1.0f) * a) * h : decode_step(s, h);
+}
+
+template <typename FT, int NC, bool GATE, bool SPEED, bool SAME4>
+__device__ __forceinline__ float4 lic_point_cells(const LicArgs& a, const CachedArgs& c, float sx, float sy, float sz)
+{
+    const int nx = a.field.n[0], ny = a.field.n[1], nz = a.field.n[2];
+    LicCells<FT, NC, GATE, SPEED, SAME4> cells;
+    cells.reset();
+    float4 n;
+    const float4 s0 = cells.field_noise(a, c, P3{texel(sx, nx), texel(sy, ny), texel(sz, nz)}, sx, sy, sz, n);
+    const gfloat* w = (const gfloat*)a.w;
+    float4 acc = make_float4(n.x * w[0], n.y * w[0], n.z * w[0], n.w * w[0]);
+#pragma unroll 1
+    for (int dirn = 0; dirn < 2; ++dirn) {
+        const int steps = dirn == 0 ? a.B : a.F;
+        const float h = dirn == 0 ? -a.he : a.he;
+        const gfloat* wk = dirn == 0 ? w + 1 : w + 1 + a.B;
+        float px = sx, py = sy, pz = sz;
+        float4 s = s0;
+#pragma unroll 1
+        for (int i = 0; i < steps; ++i) {
+            // singleLICstep (inc_lic.glsl:93-145), Heun predictor/corrector
+            const float d1x = cell_step<SPEED>(s.x, s.w, h);
+            const float d1y = cell_step<SPEED>(s.y, s.w, h);
+            const float d1z = cell_step<SPEED>(s.z, s.w, h);
+            const float qx = px + d1x, qy = py + d1y, qz = pz + d1z;
+            P3 f;
+            const float3 s2 = field_at<typename decltype(cells)::T, decltype(cells)::NCH>(
+                c, cells.fc, P3{texel(qx, nx), texel(qy, ny), texel(qz, nz)}, f);
+            px = fmaf(0.5f, d1x + cell_step<SPEED>(s2.x, s.w, h), px);
+            py = fmaf(0.5f, d1y + cell_step<SPEED>(s2.y, s.w, h), py);
+            pz = fmaf(0.5f, d1z + cell_step<SPEED>(s2.z, s.w, h), pz);
+            s = cells.field_noise(a, c, P3{texel(px, nx), texel(py, ny), texel(pz, nz)}, px, py, pz, n);
+            const float wi = wk[i];
+            acc.x = acc.x + n.x * wi;
+            if constexpr (NC == 4) {
+                acc.y = acc.y + n.y * wi;
+                acc.z = acc.z + n.z * wi;
+                acc.w = acc.w + n.w * wi;
+            }
+        }
+    }
+    return acc;
 }
 
 // LIC of one seed, any noise (scalar or RGBA) and the optional scalar gate:

@@ -1646,6 +1646,32 @@ __device__ __forceinline__ float tf_alpha(const float* tf, float u)
     return lerpf(tf[4 * p.i + 3], tf[4 * p.i + 7], p.f);
 }
 
+// LIC of one sample of the on-the-fly casters, scaled, in l4 (NC values).  The
+// cell caches live for one sample: consecutive samples of a lane are G steps
+// apart, so the previous streamline's last cell rarely serves the next one,
+// and the caches' registers are free while shading.
+template <typename FT, int NC, bool GATE, int MODE>
+__device__ __forceinline__ void sample_lic(const LicArgs& L, const CachedArgs& c, const float pos[3], float l4[4])
+{
+    if constexpr (MODE > 0 && NC == 1 && !GATE) {
+        LicFieldCache<FT, MODE == 2> fc;
+        fc.reset();
+        NoiseCache nc;
+        nc.reset();
+        l4[0] = lic_point_cached<FT, MODE == 2>(L, c, fc, nc, pos[0], pos[1], pos[2]) * L.scl;
+    } else {
+        float4 acc;
+        if constexpr (MODE > 0)
+            acc = lic_point_cells<FT, NC, GATE, false, MODE == 2>(L, c, pos[0], pos[1], pos[2]);
+        else
+            acc = lic_point<FT, NC, GATE>(L, pos[0], pos[1], pos[2]);
+        l4[0] = NC == 1 ? acc.x * L.scl : acc.x;
+        l4[1] = acc.y;
+        l4[2] = acc.z;
+        l4[3] = acc.w * L.scl;
+    }
+}
+
 // ---- fused on-the-fly LIC ray caster --------------------------------------
 //
 // lic3d_fragment.glsl:5-99 (the reference's default VOLIC_RAYCAST mode): no
@@ -1677,21 +1703,7 @@ k_render_fused(RenderLaunch a, LicArgs L)
             float pos[3] = {r.pos[0], r.pos[1], r.pos[2]};
             for (long long k = 0; k < a.max_samples; ++k) {
                 float l4[4];
-                if constexpr (MODE > 0) {
-                    // cell caches per sample (their registers are free while shading)
-                    LicFieldCache<FT, MODE == 2> fc;
-                    fc.reset();
-                    NoiseCache nc;
-                    nc.reset();
-                    const float acc = lic_point_cached<FT, MODE == 2>(L, c, fc, nc, pos[0], pos[1], pos[2]);
-                    l4[0] = acc * L.scl;
-                } else {
-                    const float4 acc = lic_point<FT, NC, GATE>(L, pos[0], pos[1], pos[2]);
-                    l4[0] = NC == 1 ? acc.x * L.scl : acc.x;
-                    l4[1] = acc.y;
-                    l4[2] = acc.z;
-                    l4[3] = acc.w * L.scl;
-                }
+                sample_lic<FT, NC, GATE, MODE>(L, c, pos, l4);
                 const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
                 Sample s;
                 shade_sample<FT, NC>(a, tf, op, r, pos, fv, cf, tri_ch(fv, cf, a.tf_ch), l4, s);
@@ -1800,21 +1812,7 @@ k_render_slices(RenderLaunch a, LicArgs L, SliceSetup S)
             const float tfu = tri_ch(fv, cf, a.tf_ch);
             if (!(tf_alpha(tf, tfu) > 0.05f)) continue;
             float l4[4];
-            if constexpr (MODE > 0) {
-                // cell caches per sample (their registers are free while shading)
-                LicFieldCache<FT, MODE == 2> fc;
-                fc.reset();
-                NoiseCache nc;
-                nc.reset();
-                const float acc = lic_point_cached<FT, MODE == 2>(L, c, fc, nc, pos[0], pos[1], pos[2]);
-                l4[0] = acc * L.scl;
-            } else {
-                const float4 acc = lic_point<FT, NC, GATE>(L, pos[0], pos[1], pos[2]);
-                l4[0] = NC == 1 ? acc.x * L.scl : acc.x;
-                l4[1] = acc.y;
-                l4[2] = acc.z;
-                l4[3] = acc.w * L.scl;
-            }
+            sample_lic<FT, NC, GATE, MODE>(L, c, pos, l4);
             Sample s;
             shade_sample<FT, NC>(a, tf, op, r, pos, fv, cf, tfu, l4, s);
             if (S.blend) {
@@ -1953,23 +1951,7 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
             }
             if (visible) {
                 float l4[4];
-                if constexpr (MODE > 0) {
-                    // cell caches per sample: consecutive samples of a lane are G steps
-                    // apart, so the previous streamline's last cell rarely serves the
-                    // next one, and the caches' registers are free while shading
-                    LicFieldCache<FT, MODE == 2> fc;
-                    fc.reset();
-                    NoiseCache nc;
-                    nc.reset();
-                    const float acc = lic_point_cached<FT, MODE == 2>(L, c, fc, nc, pos[0], pos[1], pos[2]);
-                    l4[0] = acc * L.scl;
-                } else {
-                    const float4 acc = lic_point<FT, NC, GATE>(L, pos[0], pos[1], pos[2]);
-                    l4[0] = NC == 1 ? acc.x * L.scl : acc.x;
-                    l4[1] = acc.y;
-                    l4[2] = acc.z;
-                    l4[3] = acc.w * L.scl;
-                }
+                sample_lic<FT, NC, GATE, MODE>(L, c, pos, l4);
                 Sample sm;
                 if constexpr (!SLICES) tfu = tri_ch(fv, cf, a.tf_ch);
                 shade_sample<FT, NC>(a, tf, op, rs, pos, fv, cf, tfu, l4, sm);
@@ -2092,8 +2074,13 @@ hipError_t launch_render_rg(const RenderLaunch& R, int G, hipStream_t s)
 
 namespace {
 
-// LIC variant of the on-the-fly casters: 2 cached with the noise cell on
-// the field grid, 1 cached, 0 uncached (RGBA noise or the scalar gate)
+// LIC code of the on-the-fly casters (their MODE): 0 lic_point, 1 the cell
+// caches, 2 the same with the noise in the LIC copy of the field.  The caches
+// pay for every noise, gate and caster (128^3, 20+20 steps, 512 x 512, without
+// and with them: RGBA FP32 fused 6.8 -> 2.0 ms, slices 3.5 -> 1.5; FP16 4.2 ->
+// 2.2, 3.0 -> 2.2; UNORM8 4.1 -> 2.3, 2.9 -> 2.3; gate FP32 7.2 -> 2.9, FP16
+// slices 3.8 -> 2.4), also where a kernel then passes 128 registers.
+// SPEED_OF_FLOW takes 0.
 struct LicVariant {
     bool gate;
     int nc;
@@ -2105,12 +2092,35 @@ LicVariant lic_variant(const LicLaunch& L)
     LicVariant v;
     v.gate = L.gate != 0;
     v.nc = L.nc;
-    const bool cached = L.cache && L.nc == 1 && !v.gate;
-    // the SAME kernels read the noise from channel 3 of the LIC field copy
-    const bool same = L.field_has_noise && L.freq == 1.0f && L.noise.n[0] == L.field.n[0] &&
-                      L.noise.n[1] == L.field.n[1] && L.noise.n[2] == L.field.n[2];
-    v.mode = cached ? (same ? 2 : 1) : 0;
+    const LicKind k = lic_kind(L);
+    v.mode = k == LicKind::Direct || L.speed ? 0 : k == LicKind::Copy || k == LicKind::Copy4 ? 2 : 1;
     return v;
+}
+
+// fn(integral_constant NC, GATE, MODE) of a variant; MODE 2 with RGBA noise
+// is FP32's alone
+template <typename FT, typename Fn>
+void with_lic_variant(const LicVariant& v, Fn&& fn)
+{
+    using std::integral_constant;
+    auto call = [&](auto nc, auto gate, auto mode) { fn(nc, gate, mode); };
+    auto modes = [&](auto nc, auto gate) {
+        if (v.mode == 1)
+            call(nc, gate, integral_constant<int, 1>{});
+        else
+            call(nc, gate, integral_constant<int, 0>{});
+    };
+    using F = integral_constant<bool, false>;
+    using T = integral_constant<bool, true>;
+    if (v.mode == 2 && v.nc == 1) return call(integral_constant<int, 1>{}, F{}, integral_constant<int, 2>{});
+    if constexpr (std::is_same<FT, float4>::value)
+        if (v.mode == 2) return call(integral_constant<int, 4>{}, F{}, integral_constant<int, 2>{});
+    if (v.nc == 4)
+        modes(integral_constant<int, 4>{}, F{});
+    else if (v.gate)
+        modes(integral_constant<int, 1>{}, T{});
+    else
+        modes(integral_constant<int, 1>{}, F{});
 }
 
 }  // namespace
@@ -2128,16 +2138,9 @@ hipError_t launch_render_fused(const RenderLaunch& R, const LicLaunch& L, hipStr
     const LicVariant v = lic_variant(L);
     return with_field_type(R.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
-        if (v.mode == 2)
-            hipLaunchKernelGGL((k_render_fused<FT, 1, false, 2>), grid, block, 0, s, R, A);
-        else if (v.mode == 1)
-            hipLaunchKernelGGL((k_render_fused<FT, 1, false, 1>), grid, block, 0, s, R, A);
-        else if (v.nc == 4)
-            hipLaunchKernelGGL((k_render_fused<FT, 4, false, 0>), grid, block, 0, s, R, A);
-        else if (v.gate)
-            hipLaunchKernelGGL((k_render_fused<FT, 1, true, 0>), grid, block, 0, s, R, A);
-        else
-            hipLaunchKernelGGL((k_render_fused<FT, 1, false, 0>), grid, block, 0, s, R, A);
+        with_lic_variant<FT>(v, [&](auto nc, auto gate, auto mode) {
+            hipLaunchKernelGGL((k_render_fused<FT, nc.value, gate.value, mode.value>), grid, block, 0, s, R, A);
+        });
     });
 }
 
@@ -2154,16 +2157,9 @@ hipError_t launch_render_slices(const RenderLaunch& R, const LicLaunch& L, const
     const LicVariant v = lic_variant(L);
     return with_field_type(R.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
-        if (v.mode == 2)
-            hipLaunchKernelGGL((k_render_slices<FT, 1, false, 2>), grid, block, 0, s, R, A, S);
-        else if (v.mode == 1)
-            hipLaunchKernelGGL((k_render_slices<FT, 1, false, 1>), grid, block, 0, s, R, A, S);
-        else if (v.nc == 4)
-            hipLaunchKernelGGL((k_render_slices<FT, 4, false, 0>), grid, block, 0, s, R, A, S);
-        else if (v.gate)
-            hipLaunchKernelGGL((k_render_slices<FT, 1, true, 0>), grid, block, 0, s, R, A, S);
-        else
-            hipLaunchKernelGGL((k_render_slices<FT, 1, false, 0>), grid, block, 0, s, R, A, S);
+        with_lic_variant<FT>(v, [&](auto nc, auto gate, auto mode) {
+            hipLaunchKernelGGL((k_render_slices<FT, nc.value, gate.value, mode.value>), grid, block, 0, s, R, A, S);
+        });
     });
 }
 
@@ -2183,27 +2179,17 @@ hipError_t launch_render_group(const RenderLaunch& R, const LicLaunch& L, const 
     if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
     dim3 grid((unsigned)nblocks), block(kRThreads);
     const LicVariant v = lic_variant(L);
-#define VV_GROUP_LAUNCH(FT, NC, GATE, MODE)                                                                 \
-    do {                                                                                                   \
-        if (slices)                                                                                        \
-            hipLaunchKernelGGL((k_render_group<FT, NC, GATE, MODE, true>), grid, block, 0, s, R, A, S, G);  \
-        else                                                                                               \
-            hipLaunchKernelGGL((k_render_group<FT, NC, GATE, MODE, false>), grid, block, 0, s, R, A, S, G); \
-    } while (0)
     return with_field_type(R.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
-        if (v.mode == 2)
-            VV_GROUP_LAUNCH(FT, 1, false, 2);
-        else if (v.mode == 1)
-            VV_GROUP_LAUNCH(FT, 1, false, 1);
-        else if (v.nc == 4)
-            VV_GROUP_LAUNCH(FT, 4, false, 0);
-        else if (v.gate)
-            VV_GROUP_LAUNCH(FT, 1, true, 0);
-        else
-            VV_GROUP_LAUNCH(FT, 1, false, 0);
+        with_lic_variant<FT>(v, [&](auto nc, auto gate, auto mode) {
+            if (slices)
+                hipLaunchKernelGGL((k_render_group<FT, nc.value, gate.value, mode.value, true>), grid, block, 0, s, R, A, S,
+                                   G);
+            else
+                hipLaunchKernelGGL((k_render_group<FT, nc.value, gate.value, mode.value, false>), grid, block, 0, s, R, A, S,
+                                   G);
+        });
     });
-#undef VV_GROUP_LAUNCH
 }
 
 // ---- scratch of the allocation-free adjoint ---------------------------------
