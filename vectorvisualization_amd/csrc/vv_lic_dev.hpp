@@ -553,11 +553,39 @@ __device__ __forceinline__ float3 field_rgb_of(const FieldCache<FT, NCH>& fc, co
                        FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z)));
 }
 
+// The hit test of field_at: with FP32 texels by floors, elsewhere by fractions
+// (cell_hit).  An FP32 fill waits on the L1, and floors taken before the test
+// start it sooner: slices of 124 x 32 x 154 voxels at 302 x 174, 31+31 steps,
+// 479 us by fractions, 463 by floors; the LIC volume takes the same by either.
+template <typename FT, int NCH>
+__device__ __forceinline__ bool fill_hit(const FieldCache<FT, NCH>& fc, const P3& t, P3& f)
+{
+    if constexpr (std::is_same<FT, float4>::value) {
+        const P3 k{floorf(t.x), floorf(t.y), floorf(t.z)};
+        f = P3{t.x - k.x, t.y - k.y, t.z - k.z};
+        return k.x == fc.kx && k.y == fc.ky && k.z == fc.kz;
+    } else {
+        return cell_hit(fc, t, f);
+    }
+}
+
+template <typename FT, int NCH>
+__device__ __forceinline__ void fill_rekey(FieldCache<FT, NCH>& fc, const P3& t, P3& f)
+{
+    if constexpr (std::is_same<FT, float4>::value) {
+        fc.kx = floorf(t.x);
+        fc.ky = floorf(t.y);
+        fc.kz = floorf(t.z);
+    } else {
+        cell_rekey(fc, t, f);
+    }
+}
+
 template <typename FT, int NCH, bool BRICK = false>
 __device__ __forceinline__ float3 field_at(const CachedArgs& c, FieldCache<FT, NCH>& fc, const P3& t, P3& f)
 {
-    if (!cell_hit(fc, t, f)) {
-        cell_rekey(fc, t, f);
+    if (!fill_hit(fc, t, f)) {
+        fill_rekey(fc, t, f);
         // clamped floors; a floor the clamp leaves unchanged lies in [-1, n-1]
         const P3 m = clamp_floors(c, fc.kx, fc.ky, fc.kz);
         if constexpr (NCH == 4) fc.same = m.x == fc.kx && m.y == fc.ky && m.z == fc.kz;
