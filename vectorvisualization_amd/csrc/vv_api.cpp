@@ -240,37 +240,33 @@ vv_status build_noise_tex(vv_ctx* c, const uint8_t* d_noise, const int dims[3], 
 {
     const long long n = nvox(dims);
     const int nc = with_gradients ? 4 : 1;
-    const uint8_t* d_rgb = nullptr;
-    if (with_gradients) {
-        if (grad_rgb) {
+    if (with_gradients && !grad_rgb) {
+        // computeGradients -> filterGradients -> quantizeGradients
+        // (VV/dataset.cpp:1241-1252) on the GPU; the noise VolumeData's
+        // sliceDist is 1 by default.  filterGradients kernel weights:
+        // exp(-(i^2+j^2+k^2)/SIGMA2) over i,j,k in [-2,0], normalised
+        // (VV/gradient.cpp:394-409)
+        float w[27], sum = 0.0f;
+        for (int k = -2; k < 1; ++k)
+            for (int j = -2; j < 1; ++j)
+                for (int i = -2; i < 1; ++i) {
+                    float v = std::exp(-(float)(i * i + j * j + k * k) / 5.0f);
+                    w[((k + 2) * 3 + (j + 2)) * 3 + (i + 2)] = v;
+                    sum += v;
+                }
+        for (float& v : w) v /= sum;
+        HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims)));
+        HIPCHK(c, launch_noise_grad_tex(d_noise, dims, w, c->noise.p, c->stream));
+    } else {
+        const uint8_t* d_rgb = nullptr;
+        if (with_gradients) {
             vv_status st = upload(c, c->stage2, grad_rgb, 3 * (size_t)n, grad_on_device);
             if (st) return st;
             d_rgb = (const uint8_t*)c->stage2.p;
-        } else {
-            // computeGradients -> filterGradients -> quantizeGradients
-            // (VV/dataset.cpp:1241-1252) on the GPU
-            HIPCHK(c, c->stage2.ensure(sizeof(float) * 3 * (size_t)n + 3 * (size_t)n));
-            float* g = (float*)c->stage2.p;
-            uint8_t* rgb = (uint8_t*)(g + 3 * n);
-            const float sd[3] = {1.0f, 1.0f, 1.0f};  // noise VolumeData sliceDist default
-            HIPCHK(c, launch_noise_grad_raw(d_noise, dims, sd, g, c->stream));
-            // filterGradients kernel weights: exp(-(i^2+j^2+k^2)/SIGMA2) over
-            // i,j,k in [-2,0], normalised (VV/gradient.cpp:394-409)
-            float w[27], sum = 0.0f;
-            for (int k = -2; k < 1; ++k)
-                for (int j = -2; j < 1; ++j)
-                    for (int i = -2; i < 1; ++i) {
-                        float v = std::exp(-(float)(i * i + j * j + k * k) / 5.0f);
-                        w[((k + 2) * 3 + (j + 2)) * 3 + (i + 2)] = v;
-                        sum += v;
-                    }
-            for (float& v : w) v /= sum;
-            HIPCHK(c, launch_noise_grad_filter(g, dims, w, rgb, c->stream));
-            d_rgb = rgb;
         }
+        HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims)));
+        HIPCHK(c, launch_noise_tex(d_noise, d_rgb, dims, c->noise.p, nc, c->stream));
     }
-    HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims)));
-    HIPCHK(c, launch_noise_tex(d_noise, d_rgb, dims, c->noise.p, nc, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int a = 0; a < 3; ++a) c->ndims[a] = dims[a];
     c->nch = nc;

@@ -291,10 +291,8 @@ hipError_t launch_pack_lic_field(const void* field, int field_type, const uint8_
 hipError_t launch_pack_lic_field4(const void* field, const void* noise, const int dims[3], void* out, hipStream_t s);
 hipError_t launch_noise_gen(uint64_t seed, int kind, uint64_t thr, const int dims[3],
                             uint8_t* out, hipStream_t s);
-hipError_t launch_noise_grad_raw(const uint8_t* noise, const int dims[3], const float sd[3],
-                                 float* g, hipStream_t s);
-hipError_t launch_noise_grad_filter(const float* g, const int dims[3], const float w27[27],
-                                    uint8_t* rgb, hipStream_t s);
+// RGBA noise texture (REPEAT layout) of scalar noise: filtered gradients in rgb, noise in alpha
+hipError_t launch_noise_grad_tex(const uint8_t* noise, const int dims[3], const float w27[27], void* tex, hipStream_t s);
 hipError_t launch_noise_tex(const uint8_t* noise, const uint8_t* rgb, const int dims[3],
                             void* tex, int nc, hipStream_t s);
 hipError_t launch_noise_untex(const void* tex, int nc, const int dims[3], uint8_t* out,

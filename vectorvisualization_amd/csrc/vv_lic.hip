@@ -251,45 +251,6 @@ __global__ void __launch_bounds__(kThreads) k_noise_gen(uint64_t seed, int kind,
     out[i] = kind == 0 ? (((u >> 32) < thr) ? 255 : 0) : (uint8_t)(u >> 56);
 }
 
-// computeGradients, SOBEL == 1 (VV/gradient.cpp:199-307)
-__constant__ signed char c_sobel[3][3][3][3] = {
-    {{{-1, -3, -1}, {-3, -6, -3}, {-1, -3, -1}},
-     {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}},
-     {{1, 3, 1}, {3, 6, 3}, {1, 3, 1}}},
-    {{{-1, -3, -1}, {0, 0, 0}, {1, 3, 1}},
-     {{-3, -6, -3}, {0, 0, 0}, {3, 6, 3}},
-     {{-1, -3, -1}, {0, 0, 0}, {1, 3, 1}}},
-    {{{-1, 0, 1}, {-3, 0, 3}, {-1, 0, 1}},
-     {{-3, 0, 3}, {-6, 0, 6}, {-3, 0, 3}},
-     {{-1, 0, 1}, {-3, 0, 3}, {-1, 0, 1}}}};
-
-__global__ void __launch_bounds__(kThreads) k_noise_grad_raw(const uint8_t* v, int nx, int ny, int nz,
-                                                             float sd0, float sd1, float sd2, float* g)
-{
-    long long n = (long long)nx * ny * nz;
-    long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    int x = (int)(q % nx), y = (int)((q / nx) % ny), z = (int)(q / ((long long)nx * ny));
-    auto vox = [&](int a, int b, int c) -> float {
-        return (float)v[((long long)c * ny + b) * nx + a];
-    };
-    float sd[3] = {sd0, sd1, sd2};
-    float* gp = g + 3 * q;
-    if (x > 0 && x < nx - 1 && y > 0 && y < ny - 1 && z > 0 && z < nz - 1) {
-        for (int d = 0; d < 3; ++d) {
-            float acc = 0.0f;
-            for (int i = -1; i < 2; ++i)
-                for (int j = -1; j < 2; ++j)
-                    for (int k = -1; k < 2; ++k)
-                        acc += (float)c_sobel[d][i + 1][j + 1][k + 1] * vox(x + i, y + j, z + k);
-            gp[d] = acc / (2.0f * sd[d]);
-        }
-    } else {
-        gp[0] = (x < 1) ? (vox(x + 1, y, z) - vox(x, y, z)) / sd[0] : (vox(x, y, z) - vox(x - 1, y, z)) / sd[0];
-        gp[1] = (y < 1) ? (vox(x, y + 1, z) - vox(x, y, z)) / sd[1] : (vox(x, y, z) - vox(x, y - 1, z)) / sd[1];
-        gp[2] = (z < 1) ? (vox(x, y, z + 1) - vox(x, y, z)) / sd[2] : (vox(x, y, z) - vox(x, y, z - 1)) / sd[2];
-    }
-}
 
 struct W27 {
     float w[27];
@@ -313,40 +274,6 @@ __device__ __forceinline__ uint8_t quantize8(float f)
     return (uint8_t)fminf(fmaxf(k, 0.0f), 255.0f);
 }
 
-// filterGradients (VV/gradient.cpp:377-459: window [-fw, fw-2], fw shrinking
-// at the border) followed by quantize8 (:462-478)
-__global__ void __launch_bounds__(kThreads) k_noise_grad_filter(const float* g, int nx, int ny, int nz,
-                                                                W27 fw27, uint8_t* rgb)
-{
-    long long n = (long long)nx * ny * nz;
-    long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    int x = (int)(q % nx), y = (int)((q / nx) % ny), z = (int)(q / ((long long)nx * ny));
-    int bx = min(x, nx - x - 1), by = min(y, ny - y - 1), bz = min(z, nz - z - 1);
-    int w = min(2, min(min(bx, by), bz));
-    float f[3];
-    for (int c = 0; c < 3; ++c) {
-        float acc = 0.0f;
-        for (int k = -w; k < w - 1; ++k)
-            for (int j = -w; j < w - 1; ++j)
-                for (int i = -w; i < w - 1; ++i) {
-                    long long o = 3 * (((long long)(z + k) * ny + (y + j)) * nx + (x + i)) + c;
-                    acc += fw27.w[((w + k) * 3 + (w + j)) * 3 + (w + i)] * g[o];
-                }
-        f[c] = acc;
-    }
-    float len = sqrtf(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]);
-    if (len < 1e-5f) {
-        f[0] = f[1] = f[2] = 0.0f;
-    } else {
-        f[0] /= len;
-        f[1] /= len;
-        f[2] /= len;
-    }
-    for (int c = 0; c < 3; ++c) rgb[3 * q + c] = quantize8(f[c]);
-}
-
-// raw noise (+ quantised gradients) -> REPEAT-padded texture
 __global__ void __launch_bounds__(kThreads) k_noise_tex(const uint8_t* noise, const uint8_t* rgb,
                                                         int nx, int ny, int nz, void* tex, int nc)
 {
@@ -462,6 +389,113 @@ __global__ void __launch_bounds__(kThreads) k_sample_pair(const T* field, int ch
 
 // ---- LIC ---------------------------------------------------------------------
 #include "vv_lic_dev.hpp"
+
+// RGBA noise texture of scalar noise in one pass: computeGradients with SOBEL
+// == 1 (VV/gradient.cpp:199-307; one-sided differences in the border voxels),
+// filterGradients (:377-459: window [-fw, fw-2], fw shrinking at the border),
+// quantize8 (:462-478), and the noise byte in alpha.
+//
+// A block takes a column of kGradX x kGradY voxels through zc slices.  Four
+// noise slices and two slices of raw gradients, each with its halo, stay in
+// LDS, and a thread carries the filter sums of the three outputs that a raw
+// slice reaches: their taps arrive in the order of the filter's loops (z, y,
+// x), so the sums round as theirs do, and the raw gradients (integers in a
+// Sobel sum) are exact in any order.  Bound by the vector ALU (81 products and
+// sums per voxel and the Sobel sums).  192^3: 112 us; 400 us in three kernels
+// whose raw gradients went through memory, 81 loads a voxel.
+constexpr int kGradX = 32, kGradY = 8;
+
+__global__ void __launch_bounds__(kThreads) k_noise_grad_tex(const uint8_t* __restrict__ v, int nx, int ny, int nz, int zc,
+                                                             W27 fw, uchar4* __restrict__ tex)
+{
+    constexpr int kNX = kGradX + 4, kNY = kGradY + 4;  // noise of a slice: -3 .. +1
+    constexpr int kRX = kGradX + 2, kRY = kGradY + 2;  // raw gradients: -2 .. 0
+    __shared__ uint8_t vox[4][kNY][kNX + 4];
+    __shared__ float raw[2][3][kRY][kRX];
+    const int t = threadIdx.x;
+    const int tx = t % kGradX, ty = t / kGradX;
+    const int x0 = blockIdx.x * kGradX, y0 = blockIdx.y * kGradY, z0 = blockIdx.z * zc;
+    const int x = x0 + tx, y = y0 + ty, z1 = min(z0 + zc, nz);
+    const int bxy = min(min(x, nx - x - 1), min(y, ny - y - 1));
+    // positions outside the volume hold copies that no voxel uses
+    auto load = [&](int s) {
+        const int z = min(max(s, 0), nz - 1);
+        for (int e = t; e < kNX * kNY; e += kThreads) {
+            const int X = min(max(x0 - 3 + e % kNX, 0), nx - 1), Y = min(max(y0 - 3 + e / kNX, 0), ny - 1);
+            vox[s & 3][e / kNX][e % kNX] = v[(z * ny + Y) * nx + X];  // below 2^29
+        }
+    };
+    const int first = max(z0 - 2, 0);
+    load(first - 1);
+    load(first);
+    float a1[3] = {0.f, 0.f, 0.f}, a2[3] = {0.f, 0.f, 0.f}, one[3] = {0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = first; s < z1; ++s) {
+        load(s + 1);
+        __syncthreads();
+        for (int e = t; e < kRX * kRY; e += kThreads) {
+            const int lx = e % kRX, ly = e / kRX;
+            const int X = x0 - 2 + lx, Y = y0 - 2 + ly;
+            auto at = [&](int i, int j, int k) -> int { return vox[(s + k) & 3][ly + 1 + j][lx + 1 + i]; };
+            float g[3];
+            if (X > 0 && X < nx - 1 && Y > 0 && Y < ny - 1 && s > 0 && s < nz - 1) {
+                int sum[3] = {0, 0, 0};
+#pragma unroll
+                for (int p = -1; p < 2; ++p)
+#pragma unroll
+                    for (int q = -1; q < 2; ++q) {
+                        const int w = p == 0 && q == 0 ? 6 : (p == 0 || q == 0 ? 3 : 1);
+                        sum[0] += w * (at(1, p, q) - at(-1, p, q));
+                        sum[1] += w * (at(p, 1, q) - at(p, -1, q));
+                        sum[2] += w * (at(p, q, 1) - at(p, q, -1));
+                    }
+                for (int c = 0; c < 3; ++c) g[c] = (float)sum[c] * 0.5f;  // 2 x slice distance 1
+            } else {
+                const int m = at(0, 0, 0);
+                g[0] = (float)(X < 1 ? at(1, 0, 0) - m : m - at(-1, 0, 0));
+                g[1] = (float)(Y < 1 ? at(0, 1, 0) - m : m - at(0, -1, 0));
+                g[2] = (float)(s < 1 ? at(0, 0, 1) - m : m - at(0, 0, -1));
+            }
+            for (int c = 0; c < 3; ++c) raw[s & 1][c][ly][lx] = g[c];
+        }
+        __syncthreads();
+        // taps of slice s: the last of output s, the second of s + 1, the
+        // first of s + 2
+        float f[3] = {a1[0], a1[1], a1[2]}, n1[3] = {a2[0], a2[1], a2[2]}, n2[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const float g = raw[s & 1][c][ty + j][tx + i];
+                    f[c] += fw.w[18 + 3 * j + i] * g;
+                    n1[c] += fw.w[9 + 3 * j + i] * g;
+                    n2[c] += fw.w[3 * j + i] * g;
+                }
+        const int w = min(2, min(bxy, min(s, nz - s - 1)));
+        if (w < 2)  // next to the border the window is one tap, on it empty
+            for (int c = 0; c < 3; ++c) f[c] = w == 1 ? one[c] : 0.0f;
+        for (int c = 0; c < 3; ++c) {
+            one[c] = 0.0f + fw.w[0] * raw[s & 1][c][ty + 1][tx + 1];
+            a1[c] = n1[c];
+            a2[c] = n2[c];
+        }
+        if (s < z0 || x >= nx || y >= ny) continue;
+        const float len = sqrtf(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]);
+        if (len < 1e-5f) {
+            f[0] = f[1] = f[2] = 0.0f;
+        } else {
+            f[0] /= len;
+            f[1] /= len;
+            f[2] /= len;
+        }
+        store_repeat<uchar4>(tex, nx + 1, (nx + 1) * (ny + 1), x, y, s, nx, ny, nz,
+                             make_uchar4(quantize8(f[0]), quantize8(f[1]), quantize8(f[2]), vox[s & 3][ty + 3][tx + 3]));
+    }
+}
+
+// raw noise (+ quantised gradients) -> REPEAT-padded texture
 
 template <typename FT, bool SAME, bool BRICK = false>
 __device__ __forceinline__ void lic_cached_tile(const LicArgs& a, int tile)
@@ -669,23 +703,16 @@ hipError_t launch_noise_gen(uint64_t seed, int kind, uint64_t thr, const int d[3
     return hipGetLastError();
 }
 
-hipError_t launch_noise_grad_raw(const uint8_t* noise, const int d[3], const float sd[3], float* g,
-                                 hipStream_t s)
+hipError_t launch_noise_grad_tex(const uint8_t* noise, const int d[3], const float w27[27], void* tex, hipStream_t s)
 {
-    long long n = (long long)d[0] * d[1] * d[2];
-    hipLaunchKernelGGL(k_noise_grad_raw, dim3(blocks_for(n)), dim3(kThreads), 0, s, noise, d[0], d[1],
-                       d[2], sd[0], sd[1], sd[2], g);
-    return hipGetLastError();
-}
-
-hipError_t launch_noise_grad_filter(const float* g, const int d[3], const float w27[27], uint8_t* rgb,
-                                    hipStream_t s)
-{
-    long long n = (long long)d[0] * d[1] * d[2];
     W27 w;
     for (int i = 0; i < 27; ++i) w.w[i] = w27[i];
-    hipLaunchKernelGGL(k_noise_grad_filter, dim3(blocks_for(n)), dim3(kThreads), 0, s, g, d[0], d[1],
-                       d[2], w, rgb);
+    const unsigned gx = (unsigned)((d[0] + kGradX - 1) / kGradX), gy = (unsigned)((d[1] + kGradY - 1) / kGradY);
+    // 16 slices a block repeat two slices' work in eighteen; where that is
+    // fewer than four blocks a CU, 4 slices (64^3: 18 us; the three kernels 31)
+    const int zc = (long long)gx * gy * ((d[2] + 15) / 16) >= 1024 ? 16 : 4;
+    hipLaunchKernelGGL(k_noise_grad_tex, dim3(gx, gy, (unsigned)((d[2] + zc - 1) / zc)), dim3(kThreads), 0, s, noise, d[0],
+                       d[1], d[2], zc, w, (uchar4*)tex);
     return hipGetLastError();
 }
 
