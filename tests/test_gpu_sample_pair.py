@@ -107,3 +107,26 @@ def test_groups_with_values_that_are_not_finite(ctx, bad):
     for G, (im, n) in img.items():
         np.testing.assert_array_equal(im, img[1][0], err_msg=str(G))
         assert n == img[1][1]
+
+
+@pytest.mark.parametrize("storage", [vv.STORE_FP32, vv.STORE_FP16, vv.STORE_UNORM8])
+@pytest.mark.parametrize("dims,spacing", [((40, 33, 37), (1.0, 1.5, 2.0)), ((36, 40, 44), (0.5, 1.0, 0.7))])
+def test_rgba_frames_equal(ctx, storage, dims, spacing):
+    """An RGBA LIC volume with the field's channel from its plane."""
+    ctx.upload_field(_field(dims, 1), dims, spacing=spacing, storage=storage)
+    ctx.generate_noise(3, vv.NOISE_UNIFORM, 0.0, dims, with_gradients=True)
+    p = vv.default_lic_params()
+    p.steps_forward = p.steps_backward = 4
+    p.gradient_scale = 4.0
+    p.illum_mode = vv.ILLUM_GRADIENT
+    ctx.set_lic_params(p)
+    ctx.set_tf(*fields.tf_magnitude(0.05, 0.2))
+    ctx.compute_lic()
+    _same(ctx, adjoint=True)
+    p.tf_index = vv.TF_INDEX_MAG
+    ctx.set_lic_params(p)
+    _same(ctx)
+    ctx.set_opacity_scale(np.random.default_rng(5).uniform(0.5, 1.5, dims[0] * dims[1] * dims[2]).astype(np.float32))
+    _same(ctx, adjoint=True)
+    ctx.upload_field(_field(dims, 2), dims, spacing=spacing, storage=storage)
+    _same(ctx)

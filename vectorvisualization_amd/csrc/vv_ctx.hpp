@@ -449,29 +449,31 @@ inline void drop_pair(vv_ctx* c)
     c->pair_used = 0.0;
 }
 
-// room for a LIC volume of d voxels and, behind a scalar one, for its sample
-// volume (pair stays null where memory does not suffice)
+// room for a LIC volume of d voxels and, behind it, for its sample volume
+// (pair stays null where memory does not suffice): two floats per texel with
+// scalar LIC, one with RGBA
 inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
 {
     const size_t lic = (sizeof(float) * channels * (size_t)repeat_elems(d) + 255) / 256 * 256;
-    const size_t pair = channels == 1 ? sizeof(float) * 2 * (size_t)clamp_elems(d) : 0;
+    const size_t pair = sizeof(float) * (channels == 1 ? 2 : 1) * (size_t)clamp_elems(d);
     drop_pair(c);
     c->pair = nullptr;
     const hipError_t e = c->lic.ensure(lic + pair);
-    if (e == hipErrorOutOfMemory && pair) {
+    if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
         return c->lic.ensure(lic);
     }
-    if (e == hipSuccess && pair) c->pair = (char*)c->lic.p + lic;
+    if (e == hipSuccess) c->pair = (char*)c->lic.p + lic;
     return e;
 }
 
-// R.pair: the sample volume of the context's scalar LIC volume and field, made
-// here once the frames drawn since they changed are worth the pass
-// (kPairSamplesPerVoxel).  Without it the ray caster samples both volumes.
+// R.pair: the sample volume of the context's LIC volume and field, made here
+// once the frames drawn since they changed are worth the pass
+// (kPairSamplesPerVoxel, kPlaneSamplesPerVoxel).  Without it the ray caster samples both volumes.
 inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
 {
-    if (!c->pair || R.illum >= VV_ILLUM_MALLO || !sample_pair_ok(R.view.tex_max, c->fdims)) return VV_OK;
+    const bool rgba = c->lch == 4;
+    if (!c->pair || R.illum >= VV_ILLUM_MALLO || (!rgba && !sample_pair_ok(R.view.tex_max, c->fdims))) return VV_OK;
     for (int a = 0; a < 3; ++a)
         if (c->ldims[a] != c->fdims[a]) return VV_OK;
     if (!pair_allowed(c)) return VV_OK;
@@ -479,9 +481,12 @@ inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
         if (c->pair_ch != R.tf_ch) drop_pair(c);
         c->pair_ch = R.tf_ch;
         c->pair_used += pair_samples(R.view.width, R.view.height, R.step);
-        if (c->pair_used < kPairSamplesPerVoxel * (double)nvox(c->fdims)) return VV_OK;
-        HIPCHK(c, launch_sample_pair(c->field.p, c->storage, R.tf_ch, (const float*)c->lic.p, c->fdims, (float*)c->pair,
-                                     c->stream));
+        if (c->pair_used < (rgba ? kPlaneSamplesPerVoxel : kPairSamplesPerVoxel) * (double)nvox(c->fdims)) return VV_OK;
+        if (rgba)
+            HIPCHK(c, launch_sample_plane(c->field.p, c->storage, R.tf_ch, c->fdims, (float*)c->pair, c->stream));
+        else
+            HIPCHK(c, launch_sample_pair(c->field.p, c->storage, R.tf_ch, (const float*)c->lic.p, c->fdims,
+                                         (float*)c->pair, c->stream));
         c->pair_ok = true;
     }
     R.pair = (const float*)c->pair;

@@ -387,6 +387,15 @@ __global__ void __launch_bounds__(kThreads) k_sample_pair(const T* field, int ch
     pair[q] = make_float2(lic[((long long)iz * (ny + 1) + iy) * (nx + 1) + ix], ld1(field + q, 0, ch));
 }
 
+// one channel of the field as floats, for the casters of RGBA LIC volumes;
+// bound by its reads of whole texels
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_sample_plane(const T* field, int ch, long long n, float* plane)
+{
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < n) plane[q] = ld1(field + q, 0, ch);
+}
+
 // ---- LIC ---------------------------------------------------------------------
 #include "vv_lic_dev.hpp"
 
@@ -773,6 +782,15 @@ hipError_t launch_sample_pair(const void* field, int field_type, int tf_ch, cons
         using FT = typename decltype(tag)::type;
         hipLaunchKernelGGL(k_sample_pair<FT>, grid, block, 0, s, (const FT*)field, tf_ch, lic, d[0], d[1], d[2],
                            (float2*)pair);
+    });
+}
+
+hipError_t launch_sample_plane(const void* field, int field_type, int tf_ch, const int d[3], float* plane, hipStream_t s)
+{
+    const long long n = clamp_elems(d);
+    return with_field_type(field_type, [&](auto tag) {
+        using FT = typename decltype(tag)::type;
+        hipLaunchKernelGGL(k_sample_plane<FT>, dim3(blocks_for(n)), dim3(kThreads), 0, s, (const FT*)field, tf_ch, n, plane);
     });
 }
 

@@ -53,6 +53,12 @@ struct Ray {
 // 211 us, FP16 468 -> 217, UNORM8 555 -> 220.
 struct pair_t {};
 
+// The same with an RGBA LIC volume: its REPEAT volume for the LIC value, and
+// the TF coordinate from RenderLaunch::pair as a plane of one float per texel
+// (four 8-byte loads instead of eight strided ones of 4).  LIC and 512^2 frame of
+// 64^3 FP32: 179 -> 156 us with the plane made each time.
+struct plane_t {};
+
 __device__ __forceinline__ void normalize3(const float v[3], float o[3])
 {
     float d = sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
@@ -255,7 +261,7 @@ __device__ __forceinline__ void shade_sample(const RenderLaunch& a, const float*
     s.l = l;
     constexpr bool kPair = std::is_same<FT, pair_t>::value;
     bool shaded = false;
-    if constexpr (!kPair) shaded = shade_line<FT>(a, r, fv, cf, t4, l, s);
+    if constexpr (!kPair && !std::is_same<FT, plane_t>::value) shaded = shade_line<FT>(a, r, fv, cf, t4, l, s);
     if (shaded) {
     } else if (LC == 1 || a.illum == 0) {
         // illumLIC: rgb = illum * tf.rgb * gradient.g
@@ -357,7 +363,20 @@ __device__ __forceinline__ void eval_sample(const RenderLaunch& a, const float* 
             l4[2] = q.z;
             l4[3] = q.w;
         }
-        shade_sample<FT, LC>(a, tf, op, r, pos, fv, cf, tri_ch(fv, cf, a.tf_ch), l4, s);
+        float v;
+        if constexpr (std::is_same<FT, plane_t>::value) {
+            typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+            typedef const __attribute__((address_space(1))) f2* gf2;
+            const char* p = reinterpret_cast<const char*>(a.pair);
+            const unsigned off = (unsigned)cf.base << 2;
+            const f2 r00 = *(gf2)((gchar)p + off), r10 = *(gf2)((gchar)(p + (size_t)fv.sy * 4) + off);
+            const f2 r01 = *(gf2)((gchar)(p + (size_t)fv.sz * 4) + off);
+            const f2 r11 = *(gf2)((gchar)(p + ((size_t)fv.sz + fv.sy) * 4) + off);
+            v = tri(r00.x, r00.y, r10.x, r10.y, r01.x, r01.y, r11.x, r11.y, cf) * a.pair_scale;
+        } else {
+            v = tri_ch(fv, cf, a.tf_ch);
+        }
+        shade_sample<FT, LC>(a, tf, op, r, pos, fv, cf, v, l4, s);
     }
 }
 
@@ -2069,12 +2088,16 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
 
 // Host-side dispatch of the LIC-volume ray casters: fn(TypeTag<source>{},
 // integral_constant<int, LC>{}).  A scalar LIC volume with its sample volume
-// takes pair_t unless a line mode needs the field's direction.
+// takes pair_t, or plane_t with an RGBA LIC volume, unless a line mode needs the field's direction.
 template <typename Fn>
 hipError_t with_sample_type(const RenderLaunch& R, Fn&& fn)
 {
     if (R.pair && R.lc == 1 && R.illum < 2) {
         fn(TypeTag<pair_t>{}, std::integral_constant<int, 1>{});
+        return hipGetLastError();
+    }
+    if (R.pair && R.lc == 4 && R.illum < 2) {
+        fn(TypeTag<plane_t>{}, std::integral_constant<int, 4>{});
         return hipGetLastError();
     }
     return with_field_type(R.field_type, [&](auto tag) {
