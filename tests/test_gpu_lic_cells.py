@@ -5,6 +5,7 @@ off the field's grid, a gate volume of other dims, steps that jump several
 cells, leave the volume or end a hundred million volumes away."""
 import numpy as np
 import pytest
+import torch
 
 import vectorvisualization_amd as vv
 from vectorvisualization_amd import fields
@@ -70,3 +71,21 @@ def test_on_the_fly_bits(ctx, storage, kind, group):
         a, b = _both(ctx, lambda: render(cam))
         assert np.abs(np.asarray(a)).max() > 0
         np.testing.assert_array_equal(np.asarray(a), np.asarray(b))
+
+
+def test_captured_lic_reads_later_fields(ctx):
+    """A captured LIC with RGBA noise is the LIC of the field at each replay."""
+    dims = (13, 11, 7)
+    _scene(ctx, dims, vv.STORE_FP32, "rgba", 0.03, 0)
+    ctx.compute_lic()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=ctx._torch_stream()):
+        ctx.compute_lic()
+    for seed in (1, 2):
+        v = np.random.default_rng(seed).normal(size=dims[::-1] + (3,)).astype(np.float32)
+        ctx.upload_field(v, dims)
+        g.replay()
+        torch.cuda.synchronize()
+        got = ctx.download_lic()
+        ctx.compute_lic()
+        np.testing.assert_array_equal(got, ctx.download_lic())

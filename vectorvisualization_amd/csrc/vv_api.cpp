@@ -548,9 +548,12 @@ vv_status fill_lic_launch(vv_ctx* c, LicLaunch& L, void* out)
     // room for the four bytes, and the volume at 128^3 with 20+20 steps takes
     // .42 ms with the copy, .48 without; in FP16 and UNORM8 the copy would be
     // wider than the field).  Without memory for the copy it reads the noise
-    // volume.
+    // volume; so does a call under capture with RGBA noise, whose graph then
+    // reads what later uploads put into the field.
     const bool grid = c->ndims[0] == c->fdims[0] && c->ndims[1] == c->fdims[1] && c->ndims[2] == c->fdims[2];
-    if (L.cache && !L.speed && nc == 4 && c->storage == VV_STORE_FP32 && grid) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (L.cache && !L.speed && nc == 4 && c->storage == VV_STORE_FP32 && grid &&
+        hipStreamIsCapturing(c->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
         if (!c->lic_field_ok) {
             const hipError_t e = c->lic_field.ensure((size_t)L.field_bytes);
             if (e == hipErrorOutOfMemory) {
