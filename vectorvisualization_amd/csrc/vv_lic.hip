@@ -53,16 +53,43 @@ __device__ __forceinline__ float field_len(const float* v0, const float* v1, flo
     return len < 1e-5f ? 0.0f : len;
 }
 
+// Largest |v|, as its bits.  Bound by memory: a thread takes four vectors at a
+// time in three 16-byte loads (VEC: both arrays aligned to 16 bytes; else one
+// vector), reads a lone field once, and takes the root (and its limit) of the
+// largest square alone, both being monotone.  One atomic per block on one
+// address, so the grid is four blocks a CU.  192^3: 24 us, 3.5 TB/s; 55 with a
+// vector and a root at a time, both reads and 4096 blocks.
+template <bool VEC>
 __global__ void __launch_bounds__(kThreads) k_field_maxlen(const float* v0, const float* v1,
                                                            float t, long long n, uint32_t* maxbits)
 {
     __shared__ float red[kThreads / 64];
     float m = 0.0f;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x) {
+    auto square = [&](const float* a, const float* b) {
         float tv[3];
-        m = fmaxf(m, field_len(v0, v1, t, i, tv));
+        for (int c = 0; c < 3; ++c) tv[c] = a[c] + t * (b[c] - a[c]);
+        m = fmaxf(m, tv[0] * tv[0] + tv[1] * tv[1] + tv[2] * tv[2]);
+    };
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    long long done = 0;
+    if constexpr (VEC) {
+        const long long quads = n / 4;
+        const float4 *p0 = reinterpret_cast<const float4*>(v0), *p1 = reinterpret_cast<const float4*>(v1);
+        for (long long i = i0; i < quads; i += stride) {
+            float a[12], b[12];
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<float4*>(a + 4 * k) = p0[3 * i + k];
+            if (v0 == v1)
+                for (int k = 0; k < 12; ++k) b[k] = a[k];
+            else
+                for (int k = 0; k < 3; ++k) *reinterpret_cast<float4*>(b + 4 * k) = p1[3 * i + k];
+            for (int k = 0; k < 4; ++k) square(a + 3 * k, b + 3 * k);
+        }
+        done = 4 * quads;
     }
+    for (long long i = done + i0; i < n; i += stride) square(v0 + 3 * i, v1 + 3 * i);
+    m = sqrtf(m);
+    if (m < 1e-5f) m = 0.0f;
     m = wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -649,8 +676,11 @@ hipError_t launch_field_maxlen(const float* v0, const float* v1, float t, long l
                                uint32_t* maxbits, hipStream_t s)
 {
     unsigned g = blocks_for(n);
-    if (g > 4096) g = 4096;
-    hipLaunchKernelGGL(k_field_maxlen, dim3(g), dim3(kThreads), 0, s, v0, v1, t, n, maxbits);
+    if (g > 1024) g = 1024;
+    if ((reinterpret_cast<uintptr_t>(v0) | reinterpret_cast<uintptr_t>(v1)) % 16 == 0)
+        hipLaunchKernelGGL(k_field_maxlen<true>, dim3(g), dim3(kThreads), 0, s, v0, v1, t, n, maxbits);
+    else
+        hipLaunchKernelGGL(k_field_maxlen<false>, dim3(g), dim3(kThreads), 0, s, v0, v1, t, n, maxbits);
     return hipGetLastError();
 }
 
