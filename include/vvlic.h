@@ -504,8 +504,8 @@ vv_status vv_anim_destroy(vv_anim* a);
  * 64; 1 = one lane per pixel; 0 = the power of two, at most 16, below
  * 16 / (step_size_vol sqrt(width height)), at least 1; the forward pass of
  * vv_render_record and of the adjoints and the adjoints' backward walk take
- * 4, or the set value if it is smaller;
- * gradients do not depend on it), "render.block_x", "render.block_y" (pixel
+ * 4, or the set value if it is smaller; with 0 the forward pass takes 2 from
+ * 2^19 rays and 1 from 3 2^19; gradients do not depend on it), "render.block_x", "render.block_y" (pixel
  * tile of vv_render with one lane per pixel, 64 to 256 threads in
  * multiples of 64), "render.ray_group" (lanes per ray of vv_render_fused /
  * vv_render_slices, a power of two up to 64; 0 = enough lanes for about

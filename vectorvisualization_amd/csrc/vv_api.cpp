@@ -996,6 +996,14 @@ static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A
     // both walks take 4 lanes per ray unless the tuning asks for fewer (with 2
     // the voxel boxes of the opacity-scale windows overflow on oblique views)
     A.group = c->volume_group > 0 && c->volume_group < 4 ? c->volume_group : 4;
+    // a large view has rays enough without lanes for each: recorded frame of
+    // 128^3 at 1/128, 1, 2 and 4 lanes, on an oblique view: 512^2 .130, .125,
+    // .116 ms; 768^2 .127, .134, .153; 1024^2 .142, .162, .207; 1536^2 .182,
+    // .257, .375; of 256^3 at 1/256: 768^2 .246, .237, .248; 1024^2 .351, .290,
+    // .354; 1536^2 .402, .484, .658
+    const long long rays = (long long)cam->width * cam->height;
+    const int most = rays < (1ll << 19) ? 4 : rays < 3 * (1ll << 19) ? 2 : 1;
+    A.fwd_group = c->volume_group > 0 || A.group < most ? A.group : most;
     return VV_OK;
 }
 

@@ -247,7 +247,8 @@ struct AdjointLaunch {
     long long* dsigma_fx;         // sigma voxel accumulators, or null
     int use_window;               // accumulate dsigma in an LDS window per segment
     int full_col;                 // the full layout: a column per segment, no checkpoints
-    int group;                    // lanes per ray of the forward pass: 2 or 4, else one lane per pixel
+    int group;                    // lanes per ray of both walks: 2 or 4, else one lane per pixel
+    int fwd_group;                // the forward pass's own with full_col: its entries do not depend on it
 };
 
 // Scratch of vv_render_adjoint_noalloc: one static device array per GPU

@@ -2295,8 +2295,8 @@ hipError_t noalloc_scratch(int device, void** ptr)
 
 hipError_t launch_adjoint_forward(const AdjointLaunch& A, hipStream_t s)
 {
-    if (A.group == 2 || A.group == 4) {
-        const int G = A.group;
+    const int G = A.full_col ? A.fwd_group : A.group;
+    if (G == 2 || G == 4) {
         const long long nblocks = rg_blocks(G, A.r.view.width, A.r.view.height);
         if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
         dim3 grid((unsigned)nblocks), block(kRThreads);
