@@ -68,7 +68,7 @@ vv_status vv_destroy(vv_ctx* c)
         (void)hipStreamSynchronize(c->stream);
         DevBuf* bufs[] = {&c->field, &c->noise, &c->scalar, &c->tf_dev, &c->lic, &c->weights,
                           &c->sigma, &c->stage, &c->stage2, &c->image, &c->counter, &c->adj_ckpt,
-                          &c->adj_dimg, &c->adj_out, &c->lic_field, &c->illum_luts};
+                          &c->adj_dimg, &c->adj_out, &c->lic_field, &c->illum_luts, &c->pair};
         for (DevBuf* b : bufs) b->release();
         (void)hipStreamDestroy(c->stream);
         delete c;
@@ -614,7 +614,6 @@ vv_status vv_compute_lic(vv_ctx* c)
         const int nc = c->nch;
         HIPCHK(c, lic_buffer(c, nc, c->fdims));
         L.out = make_repeat_desc(c->lic.p, c->fdims);
-        (void)pair_allowed(c);  // notes a capture
         HIPCHK(c, launch_lic(L, c->stream));  // also writes the REPEAT halo planes
         // the opacity scale lives on the LIC grid: drop it when that grid changes
         if (c->ldims[0] != c->fdims[0] || c->ldims[1] != c->fdims[1] || c->ldims[2] != c->fdims[2])

@@ -102,9 +102,11 @@ struct vv_ctx {
 
     // the ray casters' sample volume of lic and the field's channel pair_ch
     // (RenderLaunch::pair), made once the frames since either changed are
-    // worth it; pair_used counts their samples.  It lies behind the LIC volume
-    // in `lic` (lic_buffer), so no frame allocates.
-    void* pair = nullptr;
+    // worth it; pair_used counts their samples.  Its buffer comes with the LIC
+    // volume's (lic_buffer), so no frame allocates, and may be missing:
+    // pair_denied is the smallest size that memory did not suffice for.
+    DevBuf pair;
+    size_t pair_denied = 0;
     bool pair_ok = false;
     int pair_ch = 0;
     double pair_used = 0.0;
@@ -449,21 +451,31 @@ inline void drop_pair(vv_ctx* c)
     c->pair_used = 0.0;
 }
 
-// room for a LIC volume of d voxels and, behind it, for its sample volume
-// (pair stays null where memory does not suffice): two floats per texel with
-// scalar LIC, one with RGBA
+// bytes of the sample volume of a LIC volume of d voxels: two floats per texel
+// with scalar LIC, one with RGBA
+inline size_t pair_bytes(int channels, const int d[3])
+{
+    return sizeof(float) * (channels == 1 ? 2 : 1) * (size_t)clamp_elems(d);
+}
+
+// Room for a LIC volume of d voxels, and for its sample volume where memory
+// suffices.  They are two buffers, and a size that was refused is not asked
+// for again: a LIC volume of the same size as before allocates nothing and
+// stays where a captured graph has it.
 inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
 {
-    const size_t lic = (sizeof(float) * channels * (size_t)repeat_elems(d) + 255) / 256 * 256;
-    const size_t pair = sizeof(float) * (channels == 1 ? 2 : 1) * (size_t)clamp_elems(d);
+    const size_t lic = sizeof(float) * channels * (size_t)repeat_elems(d), pair = pair_bytes(channels, d);
     drop_pair(c);
-    c->pair = nullptr;
-    const hipError_t e = c->lic.ensure(lic + pair);
+    if (c->lic.bytes < lic) c->has_lic = false;  // no frame of a buffer that could not grow
+    hipError_t e = c->lic.ensure(lic);
+    const bool refused = c->pair_denied && pair >= c->pair_denied;
+    if (e != hipSuccess || !pair_allowed(c) || refused || (channels == 1 && !pair_addressable(d))) return e;
+    e = c->pair.ensure(pair);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        return c->lic.ensure(lic);
+        c->pair_denied = pair;
+        e = hipSuccess;
     }
-    if (e == hipSuccess) c->pair = (char*)c->lic.p + lic;
     return e;
 }
 
@@ -473,7 +485,9 @@ inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
 inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
 {
     const bool rgba = c->lch == 4;
-    if (!c->pair || R.illum >= VV_ILLUM_MALLO || (!rgba && !sample_pair_ok(R.view.tex_max, c->fdims))) return VV_OK;
+    if (c->pair.bytes < pair_bytes(c->lch, c->ldims) || R.illum >= VV_ILLUM_MALLO ||
+        (!rgba && !sample_pair_ok(R.view.tex_max, c->fdims)))
+        return VV_OK;
     for (int a = 0; a < 3; ++a)
         if (c->ldims[a] != c->fdims[a]) return VV_OK;
     if (!pair_allowed(c)) return VV_OK;
@@ -483,13 +497,13 @@ inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
         c->pair_used += pair_samples(R.view.width, R.view.height, R.step);
         if (c->pair_used < (rgba ? kPlaneSamplesPerVoxel : kPairSamplesPerVoxel) * (double)nvox(c->fdims)) return VV_OK;
         if (rgba)
-            HIPCHK(c, launch_sample_plane(c->field.p, c->storage, R.tf_ch, c->fdims, (float*)c->pair, c->stream));
+            HIPCHK(c, launch_sample_plane(c->field.p, c->storage, R.tf_ch, c->fdims, (float*)c->pair.p, c->stream));
         else
             HIPCHK(c, launch_sample_pair(c->field.p, c->storage, R.tf_ch, (const float*)c->lic.p, c->fdims,
-                                         (float*)c->pair, c->stream));
+                                         (float*)c->pair.p, c->stream));
         c->pair_ok = true;
     }
-    R.pair = (const float*)c->pair;
+    R.pair = (const float*)c->pair.p;
     R.pair_scale = pair_scale(c->storage);
     return VV_OK;
 }

@@ -103,10 +103,15 @@ struct ViewBlock {
 // texel coordinate must stay below n (a spacing below 1 on the longest axis
 // stretches the texture range past the volume, where the LIC volume repeats
 // and the field clamps).  Its texels are addressed with 32-bit byte offsets
-// and 24-bit row numbers.
+// and 24-bit row numbers (pair_addressable).
+inline bool pair_addressable(const int n[3])
+{
+    return clamp_elems(n) * 8 < (1ll << 32) && (long long)(n[1] + 2) * (n[2] + 2) < (1ll << 24);
+}
+
 inline bool sample_pair_ok(const float tex_max[3], const int n[3])
 {
-    if (clamp_elems(n) * 8 >= (1ll << 32) || (long long)(n[1] + 2) * (n[2] + 2) >= (1ll << 24)) return false;
+    if (!pair_addressable(n)) return false;
     for (int a = 0; a < 3; ++a)
         if (!(tex_max[a] * (float)n[a] - 0.5f < (float)n[a] - 0.25f)) return false;
     return true;
