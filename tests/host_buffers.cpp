@@ -157,8 +157,28 @@ static void refused_lic_volume_is_gone()
     CHECK(!a.c.has_lic);
 }
 
+// what does not fit beside the sample volume takes its memory, for good
+static void sample_volume_gives_way()
+{
+    Scene a(1u << 20);
+    CHECK(a.lic() == hipSuccess && a.frame());
+    const void* p = a.c.lic.p;
+    CHECK(a.c.adj_ckpt.ensure(900u << 10) == hipSuccess && hipGetLastError() == hipSuccess);
+    CHECK(!a.frame());
+    const int n = g_mallocs, f = g_frees;
+    CHECK(a.lic() == hipSuccess && a.c.lic.p == p && !a.frame() && g_mallocs == n && g_frees == f);
+    CHECK(a.c.image.ensure(900u << 10) == hipErrorOutOfMemory);
+
+    // a larger LIC volume does too
+    Scene b(1u << 20);
+    CHECK(b.lic() == hipSuccess && b.frame());
+    g_limit = lic_size(4) + 256;
+    CHECK(b.lic(4) == hipSuccess && !b.frame());
+}
+
 int main()
 {
+    sample_volume_gives_way();
     lic_buffer_stays();
     capture_allocates_nothing();
     refused_lic_volume_is_gone();

@@ -66,10 +66,8 @@ vv_status vv_destroy(vv_ctx* c)
         if (!c) return VV_OK;
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
-        DevBuf* bufs[] = {&c->field, &c->noise, &c->scalar, &c->tf_dev, &c->lic, &c->weights,
-                          &c->sigma, &c->stage, &c->stage2, &c->image, &c->counter, &c->adj_ckpt,
-                          &c->adj_dimg, &c->adj_out, &c->lic_field, &c->illum_luts, &c->pair};
-        for (DevBuf* b : bufs) b->release();
+        for (DevBuf* b : c->required()) b->release();
+        c->pair.release();
         (void)hipStreamDestroy(c->stream);
         delete c;
         return VV_OK;
@@ -798,6 +796,8 @@ vv_status vv_render(vv_ctx* c, const vv_camera* cam, float* image, int on_device
             R.counter = (unsigned long long*)((char*)c->counter.p + 8);
             HIPCHK(c, launch_fill_u32((uint32_t*)R.counter, 0u, 2, c->stream));
         }
+        st = ensure_pair(c, R);
+        if (st) return st;
         const int G = volume_group_for(c, cam);
         if (G > 1)
             HIPCHK(c, launch_render_rg(R, G, c->stream));
@@ -977,10 +977,10 @@ vv_status vv_set_opacity_scale(vv_ctx* c, const float* sigma, int on_device)
 // Launch descriptor and checkpoint count of an adjoint call.  Samples per ray
 // are bounded by the box diagonal in texture space over the shortest
 // per-step displacement (|dir| >= min scale).
-static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A, bool allow_pair = true)
+static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A)
 {
     std::memset(&A, 0, sizeof(A));
-    vv_status st = fill_render_launch(c, cam, A.r, true, allow_pair);
+    vv_status st = fill_render_launch(c, cam, A.r);
     if (st) return st;
     double diag = 0.0, smin = 1e30;
     for (int a = 0; a < 3; ++a) {
@@ -1089,7 +1089,8 @@ vv_status vv_render_record(vv_ctx* c, const vv_camera* cam, float* image, int on
             HIPCHK(c, launch_fill_u32((uint32_t*)A.r.counter, 0u, 2, c->stream));
         }
         adjoint_bind(A, (char*)c->adj_ckpt.p, SL, false);
-        st = adjoint_forward(c, A);
+        st = ensure_pair(c, A.r);
+        if (!st) st = adjoint_forward(c, A);
         if (st) return st;
         if (!on_device) HIPCHK(c, hipMemcpyAsync(image, dst, bytes, hipMemcpyDeviceToHost, c->stream));
         if (samples_out) {
@@ -1166,6 +1167,8 @@ vv_status vv_render_adjoint(vv_ctx* c, const vv_camera* cam, const float* dimage
             d_dsigma = dsigma ? d_dtf + 1024 : nullptr;
         }
         adjoint_bind(A, (char*)c->adj_ckpt.p, SL, dsigma != nullptr);
+        st = ensure_pair(c, A.r);
+        if (st) return st;
         if (!reuse) {
             st = adjoint_forward(c, A);
             if (st) return st;
@@ -1195,8 +1198,8 @@ vv_status vv_render_adjoint_noalloc(vv_ctx* c, const vv_camera* cam, const float
                         "line-illumination tables are not on the device: render once with this material first");
         HIPCHK(c, hipSetDevice(c->device));
         AdjointLaunch A;
-        // no sample volume: it may need an allocation, and a captured call would read a stale one
-        vv_status st = adjoint_setup(c, cam, A, false);
+        // no sample volume (ensure_pair): a captured call would read a stale one
+        vv_status st = adjoint_setup(c, cam, A);
         if (st) return st;
         const long long nrays = (long long)cam->width * cam->height;
         const long long nv = nvox(c->ldims);

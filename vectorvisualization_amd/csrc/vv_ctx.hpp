@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -24,6 +25,11 @@ inline thread_local std::string g_create_error;
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    // buffers that are given up where memory for this one is short
+    // (vv_ctx::optional), and of such a buffer the smallest size that memory
+    // did not suffice for (0: none)
+    std::vector<DevBuf*>* spare = nullptr;
+    size_t denied = 0;
     void release()
     {
         if (p) (void)hipFree(p);
@@ -35,11 +41,39 @@ struct DevBuf {
         if (n <= bytes && p) return hipSuccess;
         release();
         hipError_t e = hipMalloc(&p, n ? n : 1);
+        if (e == hipErrorOutOfMemory && spare && give_up(*spare)) {
+            (void)hipGetLastError();
+            e = hipMalloc(&p, n ? n : 1);
+        }
         if (e != hipSuccess) {
             p = nullptr;
             return e;
         }
         bytes = n;
+        return hipSuccess;
+    }
+    // releases optional buffers (hipFree waits for the kernels that read
+    // them); false when none was there
+    static bool give_up(std::vector<DevBuf*>& optional)
+    {
+        bool any = false;
+        for (DevBuf* b : optional)
+            if (b->p) {
+                b->denied = b->denied && b->denied < b->bytes ? b->denied : b->bytes;
+                b->release();
+                any = true;
+            }
+        return any;
+    }
+    // ensure of an optional buffer: a size that was refused, or given up, is
+    // not asked for again, and no memory is no error
+    hipError_t ensure_optional(size_t n)
+    {
+        if (denied && n >= denied) return hipSuccess;
+        const hipError_t e = ensure(n);
+        if (e != hipErrorOutOfMemory) return e;
+        (void)hipGetLastError();
+        denied = n;
         return hipSuccess;
     }
 };
@@ -103,10 +137,8 @@ struct vv_ctx {
     // the ray casters' sample volume of lic and the field's channel pair_ch
     // (RenderLaunch::pair), made once the frames since either changed are
     // worth it; pair_used counts their samples.  Its buffer comes with the LIC
-    // volume's (lic_buffer), so no frame allocates, and may be missing:
-    // pair_denied is the smallest size that memory did not suffice for.
+    // volume's (lic_buffer), so no frame allocates, and may be missing.
     DevBuf pair;
-    size_t pair_denied = 0;
     bool pair_ok = false;
     int pair_ch = 0;
     double pair_used = 0.0;
@@ -151,6 +183,20 @@ struct vv_ctx {
     // staging / scratch
     DevBuf stage, stage2, image, counter, adj_ckpt, adj_dimg, adj_out;
     void* noalloc_scratch = nullptr;  // this device's scratch array (vv_render_adjoint_noalloc)
+
+    // the buffers of this context and its batches that may be missing, and are
+    // given up where memory for another one is short
+    std::vector<DevBuf*> optional{&pair};
+
+    std::array<DevBuf*, 16> required()
+    {
+        return {&field, &noise, &scalar, &tf_dev, &lic, &weights, &sigma, &stage, &stage2, &image, &counter, &adj_ckpt,
+                &adj_dimg, &adj_out, &lic_field, &illum_luts};
+    }
+    vv_ctx()
+    {
+        for (DevBuf* b : required()) b->spare = &optional;
+    }
 };
 
 namespace vv_host {
@@ -459,29 +505,23 @@ inline size_t pair_bytes(int channels, const int d[3])
 }
 
 // Room for a LIC volume of d voxels, and for its sample volume where memory
-// suffices.  They are two buffers, and a size that was refused is not asked
-// for again: a LIC volume of the same size as before allocates nothing and
+// suffices.  A LIC volume of the same size as before allocates nothing and
 // stays where a captured graph has it.
 inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
 {
     const size_t lic = sizeof(float) * channels * (size_t)repeat_elems(d), pair = pair_bytes(channels, d);
     drop_pair(c);
     if (c->lic.bytes < lic) c->has_lic = false;  // no frame of a buffer that could not grow
-    hipError_t e = c->lic.ensure(lic);
-    const bool refused = c->pair_denied && pair >= c->pair_denied;
-    if (e != hipSuccess || !pair_allowed(c) || refused || (channels == 1 && !pair_addressable(d))) return e;
-    e = c->pair.ensure(pair);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        c->pair_denied = pair;
-        e = hipSuccess;
-    }
-    return e;
+    const hipError_t e = c->lic.ensure(lic);
+    if (e != hipSuccess || !pair_allowed(c) || (channels == 1 && !pair_addressable(d))) return e;
+    return c->pair.ensure_optional(pair);
 }
 
 // R.pair: the sample volume of the context's LIC volume and field, made here
 // once the frames drawn since they changed are worth the pass
-// (kPairSamplesPerVoxel, kPlaneSamplesPerVoxel).  Without it the ray caster samples both volumes.
+// (kPairSamplesPerVoxel, kPlaneSamplesPerVoxel).  Without it the ray caster
+// samples both volumes.  Called right before the launch: an allocation in
+// between could give the sample volume up.
 inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
 {
     const bool rgba = c->lch == 4;
@@ -510,9 +550,7 @@ inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
 
 // need_lic: the LIC-volume ray caster; without it (the fused caster) the
 // shading channels are those of the noise
-// (allow_pair: it may sample through ensure_pair's volume)
-inline vv_status fill_render_launch(vv_ctx* c, const vv_camera* cam, RenderLaunch& R, bool need_lic = true,
-                                    bool allow_pair = true)
+inline vv_status fill_render_launch(vv_ctx* c, const vv_camera* cam, RenderLaunch& R, bool need_lic = true)
 {
     if (!c->has_field) return fail(c, VV_ESTATE, "no vector field uploaded");
     if (need_lic && !c->has_lic) return fail(c, VV_ESTATE, "no LIC volume (call vv_compute_lic or vv_upload_lic)");
@@ -564,7 +602,7 @@ inline vv_status fill_render_launch(vv_ctx* c, const vv_camera* cam, RenderLaunc
     if (nt > 256 || nt % 64)
         return fail(c, VV_EINVAL, "render block %dx%d must hold 64, 128, 192 or 256 threads", R.block[0],
                     R.block[1]);
-    return need_lic && allow_pair ? ensure_pair(c, R) : VV_OK;
+    return VV_OK;
 }
 
 }  // namespace vv_host
