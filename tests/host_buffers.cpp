@@ -1,9 +1,11 @@
-// Host checks of the context's buffers (vv_ctx.hpp) against a device memory of
-// a set size: hipMalloc and hipFree are counted here instead of calling the
-// runtime.  Prints one line per failed check; the exit code is their number.
+// Host checks of the library's device buffers (vv_ctx.hpp, vv_api.cpp,
+// vv_batch.cpp) against a device memory of a set size: hipMalloc and hipFree
+// are counted here instead of calling the runtime, and the kernels' launchers
+// check that what they are given lies in a live buffer.  Prints one line per
+// failed check; the exit code is their number.
 #include "vv_ctx.hpp"
 
-#include <cstdlib>
+#include <iterator>
 #include <map>
 
 using namespace vv_host;
@@ -11,6 +13,7 @@ using namespace vv_host;
 static size_t g_limit = 0, g_held = 0;
 static int g_mallocs = 0, g_frees = 0, g_failed = 0;
 static std::map<void*, size_t> g_blocks;
+static char* g_next = (char*)(1ull << 40);
 static hipStreamCaptureStatus g_capture = hipStreamCaptureStatusNone;
 static hipError_t g_query = hipSuccess, g_last = hipSuccess;
 
@@ -19,7 +22,8 @@ extern "C" hipError_t hipMalloc(void** p, size_t n)
     if (g_capture != hipStreamCaptureStatusNone) return g_last = hipErrorStreamCaptureUnsupported;
     if (g_held + n > g_limit) return g_last = hipErrorOutOfMemory;
     ++g_mallocs;
-    *p = std::malloc(1);
+    *p = g_next;  // addresses alone: nothing is read or written
+    g_next += (n + 4095) / 4096 * 4096 + 4096;
     g_blocks[*p] = n;
     g_held += n;
     return hipSuccess;
@@ -30,7 +34,6 @@ extern "C" hipError_t hipFree(void* p)
     ++g_frees;
     g_held -= g_blocks.at(p);
     g_blocks.erase(p);
-    std::free(p);
     return hipSuccess;
 }
 
@@ -44,15 +47,8 @@ extern "C" hipError_t hipGetLastError(void)
 extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
 {
     *s = g_capture;
-    return g_last = g_query;
+    return g_query == hipSuccess ? hipSuccess : (g_last = g_query);
 }
-
-extern "C" const char* hipGetErrorString(hipError_t) { return "error"; }
-
-namespace vv {
-hipError_t launch_sample_pair(const void*, int, int, const float*, const int*, float*, hipStream_t) { return hipSuccess; }
-hipError_t launch_sample_plane(const void*, int, int, const int*, float*, hipStream_t) { return hipSuccess; }
-}  // namespace vv
 
 #define CHECK(x)                                             \
     do {                                                     \
@@ -61,6 +57,103 @@ hipError_t launch_sample_plane(const void*, int, int, const int*, float*, hipStr
             ++g_failed;                                      \
         }                                                    \
     } while (0)
+
+extern "C" {
+const char* hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = nullptr, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+}
+
+namespace vv_host {
+vv_status ensure_illum_luts(vv_ctx*) { return VV_OK; }
+}  // namespace vv_host
+
+extern "C" void vv_default_line_material(vv_line_material*) {}
+
+// the kernels: whether each buffer that is given holds what they touch
+static bool live(const void* p, size_t n)
+{
+    const auto b = g_blocks.upper_bound((char*)p);
+    if (b == g_blocks.begin()) return false;
+    const auto& [base, size] = *std::prev(b);
+    return (char*)p + n <= (char*)base + size;
+}
+
+static size_t field_size(const int* d, int type) { return field_texel_bytes(type) * (size_t)clamp_elems(d); }
+
+static hipError_t check_lic(const LicLaunch& L)
+{
+    CHECK(live(L.field.p, field_size(L.field.n, L.field_type)));
+    CHECK(live(L.noise.p, L.nc * (size_t)repeat_elems(L.noise.n)));
+    if (L.gate) CHECK(live(L.scalar.p, (size_t)clamp_elems(L.scalar.n)));
+    return hipSuccess;
+}
+
+static hipError_t check_frame(const RenderLaunch& R)
+{
+    CHECK(live(R.field.p, field_size(R.field.n, R.field_type)));
+    if (R.lic.p) CHECK(live(R.lic.p, sizeof(float) * R.lc * (size_t)repeat_elems(R.lic.n)));
+    if (R.pair) CHECK(live(R.pair, pair_bytes(R.lc, R.lic.n)));
+    if (R.sigma.p) CHECK(live(R.sigma.p, sizeof(float) * (size_t)clamp_elems(R.sigma.n)));
+    CHECK(live(R.image, sizeof(float) * 4 * R.view.width * R.view.height));
+    return hipSuccess;
+}
+
+namespace vv {
+hipError_t noalloc_scratch(int, void** p) { return *p = nullptr, hipSuccess; }
+hipError_t launch_fill_u32(uint32_t*, uint32_t, long long, hipStream_t) { return hipSuccess; }
+hipError_t launch_fill_i64(long long*, long long, long long, hipStream_t) { return hipSuccess; }
+hipError_t launch_field_maxlen(const float*, const float*, float, long long, uint32_t*, hipStream_t) { return hipSuccess; }
+hipError_t launch_field_encode(const float*, const float*, float, const int d[3], const uint32_t*, void* f, int type,
+                               hipStream_t, int)
+{
+    CHECK(live(f, field_size(d, type)));
+    return hipSuccess;
+}
+hipError_t launch_noise_gen(uint64_t, int, uint64_t, const int*, uint8_t*, hipStream_t) { return hipSuccess; }
+hipError_t launch_noise_tex(const uint8_t*, const uint8_t*, const int d[3], void* tex, int nc, hipStream_t)
+{
+    CHECK(live(tex, nc * (size_t)repeat_elems(d)));
+    return hipSuccess;
+}
+hipError_t launch_noise_grad_tex(const uint8_t*, const int d[3], const float*, void* tex, hipStream_t)
+{
+    CHECK(live(tex, 4 * (size_t)repeat_elems(d)));
+    return hipSuccess;
+}
+hipError_t launch_pack_lic_field(const void*, int type, const uint8_t*, const int d[3], void* out, hipStream_t)
+{
+    CHECK(live(out, field_size(d, type)));
+    return hipSuccess;
+}
+hipError_t launch_pack_lic_field4(const void*, const void*, const int d[3], void* out, hipStream_t)
+{
+    CHECK(live(out, field_size(d, 0)));
+    return hipSuccess;
+}
+hipError_t launch_pad_clamp_u8(const uint8_t*, const int*, uint8_t*, hipStream_t) { return hipSuccess; }
+hipError_t launch_pad_clamp_f32(const float*, const int*, float*, hipStream_t) { return hipSuccess; }
+hipError_t launch_pad_repeat_f32(const float*, int, const int*, float*, hipStream_t) { return hipSuccess; }
+hipError_t launch_sample_pair(const void*, int, int, const float*, const int*, float*, hipStream_t) { return hipSuccess; }
+hipError_t launch_sample_plane(const void*, int, int, const int*, float*, hipStream_t) { return hipSuccess; }
+hipError_t launch_lic(const LicLaunch& L, hipStream_t)
+{
+    CHECK(live(L.out.p, sizeof(float) * L.nc * (size_t)repeat_elems(L.out.n)));
+    return check_lic(L);
+}
+hipError_t launch_render(const RenderLaunch& R, hipStream_t) { return check_frame(R); }
+hipError_t launch_render_rg(const RenderLaunch& R, int, hipStream_t) { return check_frame(R); }
+hipError_t launch_render_fused(const RenderLaunch& R, const LicLaunch& L, hipStream_t) { return (void)check_lic(L), check_frame(R); }
+hipError_t launch_render_group(const RenderLaunch& R, const LicLaunch& L, const SliceSetup&, int, int, hipStream_t)
+{
+    return (void)check_lic(L), check_frame(R);
+}
+hipError_t launch_adjoint_forward(const AdjointLaunch& A, hipStream_t) { return check_frame(A.r); }
+}  // namespace vv
 
 static const int kDims[3] = {30, 31, 32};
 
@@ -72,11 +165,9 @@ struct Scene {
     explicit Scene(size_t room, int channels = 1)
     {
         g_limit = lic_size(channels) + 256 + room;
-        g_held = 0;
-        g_mallocs = g_frees = 0;
+        g_held = g_mallocs = g_frees = 0;
         g_capture = hipStreamCaptureStatusNone;
         g_query = g_last = hipSuccess;
-        g_blocks.clear();
         c.has_field = true;
         for (int a = 0; a < 3; ++a) c.fdims[a] = kDims[a];
         c.lch = channels;
@@ -176,8 +267,57 @@ static void sample_volume_gives_way()
     CHECK(b.lic(4) == hipSuccess && !b.frame());
 }
 
+static size_t free_memory(size_t n) { return g_limit = g_held + n; }
+
+// the library's entry points on a context with a field, noise and LIC volume of kDims
+struct Api {
+    vv_ctx* c = nullptr;
+    float* data = (float*)(1ull << 20);  // inputs and images: device pointers
+    explicit Api(int with_gradients = 0)
+    {
+        g_capture = hipStreamCaptureStatusNone;
+        g_limit = 1ull << 40;
+        CHECK(vv_create(&c, 0) == VV_OK);
+        CHECK(vv_upload_field(c, data, nullptr, 0.0f, kDims, nullptr, VV_STORE_FP32, 1) == VV_OK);
+        CHECK(vv_generate_noise(c, 1, VV_NOISE_UNIFORM, 0.0, kDims, with_gradients) == VV_OK);
+        CHECK(vv_compute_lic(c) == VV_OK);
+    }
+    ~Api() { CHECK(vv_destroy(c) == VV_OK && g_blocks.empty()); }
+};
+
+// no kernel runs on a volume whose buffer could not grow
+static void refused_volumes_are_gone()
+{
+    const int big[3] = {40, 40, 40};
+    for (int kind = 0; kind < 3; ++kind) {
+        Api a;
+        vv_ctx* c = a.c;
+        CHECK(vv_upload_scalar(c, (const uint8_t*)a.data, kDims, 1) == VV_OK);
+        c->params.gate_enable = 1;
+        CHECK(vv_compute_lic(c) == VV_OK);
+        CHECK(c->stage.ensure((size_t)nvox(big)) == hipSuccess);
+        c->pair.release();
+        free_memory(0);
+        if (kind == 0)
+            CHECK(vv_upload_field(c, a.data, nullptr, 0.0f, big, nullptr, VV_STORE_FP32, 1) == VV_ENOMEM);
+        else if (kind == 1)
+            CHECK(vv_generate_noise(c, 1, VV_NOISE_UNIFORM, 0.0, big, 0) == VV_ENOMEM);
+        else
+            CHECK(vv_upload_scalar(c, (const uint8_t*)a.data, big, 1) == VV_ENOMEM);
+        CHECK(vv_compute_lic(c) == VV_ESTATE);
+        // the refusal is reported once, and the next volume is taken
+        CHECK(hipGetLastError() == hipSuccess);
+        free_memory(1u << 22);
+        CHECK(vv_upload_field(c, a.data, nullptr, 0.0f, kDims, nullptr, VV_STORE_FP32, 1) == VV_OK);
+        CHECK(vv_generate_noise(c, 1, VV_NOISE_UNIFORM, 0.0, kDims, 0) == VV_OK);
+        CHECK(vv_upload_scalar(c, (const uint8_t*)a.data, kDims, 1) == VV_OK);
+        CHECK(vv_compute_lic(c) == VV_OK);
+    }
+}
+
 int main()
 {
+    refused_volumes_are_gone();
     sample_volume_gives_way();
     lic_buffer_stays();
     capture_allocates_nothing();

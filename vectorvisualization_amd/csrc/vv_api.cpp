@@ -167,7 +167,7 @@ vv_status vv_upload_field_ex(vv_ctx* c, const float* v0, const float* v1, float 
             }
         }
         drop_pair(c);
-        HIPCHK(c, c->field.ensure((size_t)field_texel_bytes(storage) * (size_t)clamp_elems(dims)));
+        HIPCHK(c, c->field.ensure((size_t)field_texel_bytes(storage) * (size_t)clamp_elems(dims), c->has_field));
         HIPCHK(c, c->counter.ensure(64));
         uint32_t* maxbits = (uint32_t*)c->counter.p;
         HIPCHK(c, launch_fill_u32(maxbits, 0u, 1, c->stream));
@@ -253,7 +253,7 @@ vv_status build_noise_tex(vv_ctx* c, const uint8_t* d_noise, const int dims[3], 
                     sum += v;
                 }
         for (float& v : w) v /= sum;
-        HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims)));
+        HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims), c->has_noise));
         HIPCHK(c, launch_noise_grad_tex(d_noise, dims, w, c->noise.p, c->stream));
     } else {
         const uint8_t* d_rgb = nullptr;
@@ -262,7 +262,7 @@ vv_status build_noise_tex(vv_ctx* c, const uint8_t* d_noise, const int dims[3], 
             if (st) return st;
             d_rgb = (const uint8_t*)c->stage2.p;
         }
-        HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims)));
+        HIPCHK(c, c->noise.ensure((size_t)nc * (size_t)repeat_elems(dims), c->has_noise));
         HIPCHK(c, launch_noise_tex(d_noise, d_rgb, dims, c->noise.p, nc, c->stream));
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -448,7 +448,7 @@ vv_status vv_upload_scalar(vv_ctx* c, const uint8_t* scalar, const int dims[3], 
         HIPCHK(c, hipSetDevice(c->device));
         vv_status st = upload(c, c->stage, scalar, (size_t)nvox(dims), on_device);
         if (st) return st;
-        HIPCHK(c, c->scalar.ensure((size_t)clamp_elems(dims)));
+        HIPCHK(c, c->scalar.ensure((size_t)clamp_elems(dims), c->has_scalar));
         HIPCHK(c, launch_pad_clamp_u8((const uint8_t*)c->stage.p, dims, (uint8_t*)c->scalar.p, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         for (int a = 0; a < 3; ++a) c->sdims[a] = dims[a];
@@ -966,7 +966,7 @@ vv_status vv_set_opacity_scale(vv_ctx* c, const float* sigma, int on_device)
         const long long n = nvox(c->ldims);
         vv_status st = upload(c, c->stage, sigma, sizeof(float) * (size_t)n, on_device);
         if (st) return st;
-        HIPCHK(c, c->sigma.ensure(sizeof(float) * (size_t)clamp_elems(c->ldims)));
+        HIPCHK(c, c->sigma.ensure(sizeof(float) * (size_t)clamp_elems(c->ldims), c->has_sigma));
         HIPCHK(c, launch_pad_clamp_f32((const float*)c->stage.p, c->ldims, (float*)c->sigma.p, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         c->has_sigma = true;

@@ -41,9 +41,10 @@ struct DevBuf {
         if (n <= bytes && p) return hipSuccess;
         release();
         hipError_t e = hipMalloc(&p, n ? n : 1);
+        if (e != hipSuccess) (void)hipGetLastError();  // the next launch's check is its own
         if (e == hipErrorOutOfMemory && spare && give_up(*spare)) {
-            (void)hipGetLastError();
             e = hipMalloc(&p, n ? n : 1);
+            if (e != hipSuccess) (void)hipGetLastError();
         }
         if (e != hipSuccess) {
             p = nullptr;
@@ -51,6 +52,13 @@ struct DevBuf {
         }
         bytes = n;
         return hipSuccess;
+    }
+    // ensure of a buffer whose contents `valid` announces: a buffer that could
+    // not grow holds none
+    hipError_t ensure(size_t n, bool& valid)
+    {
+        if (n > bytes) valid = false;
+        return ensure(n);
     }
     // releases optional buffers (hipFree waits for the kernels that read
     // them); false when none was there
@@ -72,7 +80,6 @@ struct DevBuf {
         if (denied && n >= denied) return hipSuccess;
         const hipError_t e = ensure(n);
         if (e != hipErrorOutOfMemory) return e;
-        (void)hipGetLastError();
         denied = n;
         return hipSuccess;
     }
@@ -461,6 +468,7 @@ inline vv_status ensure_weights(vv_ctx* c)
     std::vector<float> w;
     lic_weights(c, w);
     if (w != c->weights_host) {
+        c->weights_host.clear();
         HIPCHK(c, c->weights.ensure(sizeof(float) * w.size()));
         HIPCHK(c, hipMemcpyAsync(c->weights.p, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice,
                                  c->stream));
@@ -511,8 +519,7 @@ inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
 {
     const size_t lic = sizeof(float) * channels * (size_t)repeat_elems(d), pair = pair_bytes(channels, d);
     drop_pair(c);
-    if (c->lic.bytes < lic) c->has_lic = false;  // no frame of a buffer that could not grow
-    const hipError_t e = c->lic.ensure(lic);
+    const hipError_t e = c->lic.ensure(lic, c->has_lic);
     if (e != hipSuccess || !pair_allowed(c) || (channels == 1 && !pair_addressable(d))) return e;
     return c->pair.ensure_optional(pair);
 }
