@@ -99,7 +99,7 @@ static hipError_t check_frame(const RenderLaunch& R)
     if (R.lic.p) CHECK(live(R.lic.p, sizeof(float) * R.lc * (size_t)repeat_elems(R.lic.n)));
     if (R.pair) CHECK(live(R.pair, pair_bytes(R.lc, R.lic.n)));
     if (R.sigma.p) CHECK(live(R.sigma.p, sizeof(float) * (size_t)clamp_elems(R.sigma.n)));
-    CHECK(live(R.image, sizeof(float) * 4 * R.view.width * R.view.height));
+    CHECK(live(R.image, (size_t)4 * R.view.width * R.view.height));
     return hipSuccess;
 }
 
@@ -315,8 +315,37 @@ static void refused_volumes_are_gone()
     }
 }
 
+// RGBA noise on an FP32 field: the LIC copy gives way too, also in the middle
+// of the call that would have read it
+static void rgba_copy_gives_way()
+{
+    Api a(1);
+    vv_ctx* c = a.c;
+    vv_camera cam;
+    CHECK(vv_default_camera(&cam, 64, 48, nullptr) == VV_OK);
+    std::vector<float> image(4 * 64 * 48);
+    std::vector<uint8_t> bytes(4 * 64 * 48);
+    for (int call = 0; call < 3; ++call) {
+        CHECK(vv_upload_noise(c, (const uint8_t*)a.data, kDims, 1, nullptr, 1) == VV_OK);
+        g_limit = 1ull << 40;
+        for (DevBuf* b : c->optional) b->denied = 0;
+        CHECK(vv_compute_lic(c) == VV_OK && vv_render_fused(c, &cam, image.data(), 0, nullptr) == VV_OK);
+        (call == 0 ? c->lic : c->image).release();
+        c->pair.release();
+        free_memory(0);
+        if (call == 0)
+            CHECK(vv_compute_lic(c) == VV_OK);
+        else if (call == 1)
+            CHECK(vv_render_fused(c, &cam, image.data(), 0, nullptr) == VV_OK);
+        else
+            CHECK(vv_render_slices_blend(c, &cam, bytes.data(), 0, nullptr) == VV_OK);
+        CHECK(vv_compute_lic(c) == VV_OK);
+    }
+}
+
 int main()
 {
+    rgba_copy_gives_way();
     refused_volumes_are_gone();
     sample_volume_gives_way();
     lic_buffer_stays();

@@ -67,7 +67,7 @@ vv_status vv_destroy(vv_ctx* c)
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
         for (DevBuf* b : c->required()) b->release();
-        c->pair.release();
+        for (DevBuf* b : c->optional) b->release();
         (void)hipStreamDestroy(c->stream);
         delete c;
         return VV_OK;
@@ -192,7 +192,7 @@ vv_status vv_upload_field_ex(vv_ctx* c, const float* v0, const float* v1, float 
         }
         c->storage = storage;
         c->has_field = true;
-        c->lic_field_ok = false;
+        c->lic_field_ok = c->lic_field4_ok = false;
         ++c->scene_version;
         return VV_OK;
     });
@@ -269,7 +269,8 @@ vv_status build_noise_tex(vv_ctx* c, const uint8_t* d_noise, const int dims[3], 
     for (int a = 0; a < 3; ++a) c->ndims[a] = dims[a];
     c->nch = nc;
     c->has_noise = true;
-    c->lic_field_ok = false;
+    c->lic_field_ok = c->lic_field4_ok = false;
+    if (nc == 1) c->lic_field4.release();
     return VV_OK;
 }
 
@@ -552,19 +553,14 @@ vv_status fill_lic_launch(vv_ctx* c, LicLaunch& L, void* out)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (L.cache && !L.speed && nc == 4 && c->storage == VV_STORE_FP32 && grid &&
         hipStreamIsCapturing(c->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-        if (!c->lic_field_ok) {
-            const hipError_t e = c->lic_field.ensure((size_t)L.field_bytes);
-            if (e == hipErrorOutOfMemory) {
-                (void)hipGetLastError();
-            } else {
-                HIPCHK(c, e);
-                HIPCHK(c, launch_pack_lic_field4(c->field.p, c->noise.p, c->fdims, c->lic_field.p, c->stream));
-                c->lic_field_ok = true;
-                c->lic_field_brick = false;
-            }
+        if (!c->lic_field4_ok || !c->lic_field4.p) {
+            HIPCHK(c, c->lic_field4.ensure_optional((size_t)L.field_bytes));
+            c->lic_field4_ok = c->lic_field4.bytes >= L.field_bytes;
+            if (c->lic_field4_ok)
+                HIPCHK(c, launch_pack_lic_field4(c->field.p, c->noise.p, c->fdims, c->lic_field4.p, c->stream));
         }
-        if (c->lic_field_ok) {
-            L.field.p = c->lic_field.p;
+        if (c->lic_field4_ok) {
+            L.field.p = c->lic_field4.p;
             L.field_has_noise = 1;
         }
     }
@@ -599,6 +595,15 @@ vv_status fill_lic_launch(vv_ctx* c, LicLaunch& L, void* out)
     return VV_OK;
 }
 
+// The copy of fill_lic_launch for RGBA noise, if an allocation since gave it
+// up: the LIC reads the field.
+void drop_lost_copy(const vv_ctx* c, LicLaunch& L)
+{
+    if (L.nc != 4 || !L.field_has_noise || c->lic_field4.p) return;
+    L.field.p = c->field.p;
+    L.field_has_noise = 0;
+}
+
 }  // namespace
 
 vv_status vv_compute_lic(vv_ctx* c)
@@ -611,6 +616,7 @@ vv_status vv_compute_lic(vv_ctx* c)
         if (st) return st;
         const int nc = c->nch;
         HIPCHK(c, lic_buffer(c, nc, c->fdims));
+        drop_lost_copy(c, L);
         L.out = make_repeat_desc(c->lic.p, c->fdims);
         HIPCHK(c, launch_lic(L, c->stream));  // also writes the REPEAT halo planes
         // the opacity scale lives on the LIC grid: drop it when that grid changes
@@ -855,6 +861,7 @@ vv_status vv_render_fused(vv_ctx* c, const vv_camera* cam, float* image, int on_
             R.counter = (unsigned long long*)((char*)c->counter.p + 8);
             HIPCHK(c, launch_fill_u32((uint32_t*)R.counter, 0u, 2, c->stream));
         }
+        drop_lost_copy(c, L);
         const int G = ray_group_for(c, cam);
         if (G > 1) {
             SliceSetup S;
@@ -923,6 +930,7 @@ static vv_status render_slices(vv_ctx* c, const vv_camera* cam, void* image, int
         R.counter = (unsigned long long*)((char*)c->counter.p + 8);
         HIPCHK(c, launch_fill_u32((uint32_t*)R.counter, 0u, 2, c->stream));
     }
+    drop_lost_copy(c, L);
     const int G = ray_group_for(c, cam);
     if (G > 1)
         HIPCHK(c, launch_render_group(R, L, S, 1, G, c->stream));

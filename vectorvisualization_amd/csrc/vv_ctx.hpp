@@ -116,6 +116,10 @@ struct vv_ctx {
     // either input changes
     DevBuf lic_field;
     bool lic_field_ok = false;
+    // the same for RGBA noise on the grid of an FP32 field
+    // (launch_pack_lic_field4); it may be missing
+    DevBuf lic_field4;
+    bool lic_field4_ok = false;
 
     // scalar gate volume
     bool has_scalar = false;
@@ -193,7 +197,7 @@ struct vv_ctx {
 
     // the buffers of this context and its batches that may be missing, and are
     // given up where memory for another one is short
-    std::vector<DevBuf*> optional{&pair};
+    std::vector<DevBuf*> optional{&pair, &lic_field4};
 
     std::array<DevBuf*, 16> required()
     {
