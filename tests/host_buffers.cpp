@@ -3,7 +3,8 @@
 // are counted here instead of calling the runtime, and the kernels' launchers
 // check that what they are given lies in a live buffer.  Prints one line per
 // failed check; the exit code is their number.
-#include "vv_ctx.hpp"
+#include "vv_api.cpp"
+#include "vv_batch.cpp"
 
 #include <iterator>
 #include <map>
@@ -13,6 +14,7 @@ using namespace vv_host;
 static size_t g_limit = 0, g_held = 0;
 static int g_mallocs = 0, g_frees = 0, g_failed = 0;
 static std::map<void*, size_t> g_blocks;
+static int g_graph, g_pair_passes = 0, g_frames = 0, g_pair_frames = 0;
 static char* g_next = (char*)(1ull << 40);
 static hipStreamCaptureStatus g_capture = hipStreamCaptureStatusNone;
 static hipError_t g_query = hipSuccess, g_last = hipSuccess;
@@ -65,6 +67,21 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = nullptr, hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return *g = (hipGraph_t)&g_graph, hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t)
+{
+    return *e = (hipGraphExec_t)&g_graph, hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = nullptr, hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.0f, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
 }
 
@@ -97,6 +114,8 @@ static hipError_t check_frame(const RenderLaunch& R)
 {
     CHECK(live(R.field.p, field_size(R.field.n, R.field_type)));
     if (R.lic.p) CHECK(live(R.lic.p, sizeof(float) * R.lc * (size_t)repeat_elems(R.lic.n)));
+    ++g_frames;
+    g_pair_frames += R.pair != nullptr;
     if (R.pair) CHECK(live(R.pair, pair_bytes(R.lc, R.lic.n)));
     if (R.sigma.p) CHECK(live(R.sigma.p, sizeof(float) * (size_t)clamp_elems(R.sigma.n)));
     CHECK(live(R.image, (size_t)4 * R.view.width * R.view.height));
@@ -138,7 +157,14 @@ hipError_t launch_pack_lic_field4(const void*, const void*, const int d[3], void
 hipError_t launch_pad_clamp_u8(const uint8_t*, const int*, uint8_t*, hipStream_t) { return hipSuccess; }
 hipError_t launch_pad_clamp_f32(const float*, const int*, float*, hipStream_t) { return hipSuccess; }
 hipError_t launch_pad_repeat_f32(const float*, int, const int*, float*, hipStream_t) { return hipSuccess; }
-hipError_t launch_sample_pair(const void*, int, int, const float*, const int*, float*, hipStream_t) { return hipSuccess; }
+hipError_t launch_sample_pair(const void* f, int type, int, const float* lic, const int d[3], float* pair, hipStream_t)
+{
+    ++g_pair_passes;
+    CHECK(live(f, field_size(d, type)));
+    CHECK(live(lic, sizeof(float) * (size_t)repeat_elems(d)));
+    CHECK(live(pair, pair_bytes(1, d)));
+    return hipSuccess;
+}
 hipError_t launch_sample_plane(const void*, int, int, const int*, float*, hipStream_t) { return hipSuccess; }
 hipError_t launch_lic(const LicLaunch& L, hipStream_t)
 {
@@ -152,6 +178,16 @@ hipError_t launch_render_group(const RenderLaunch& R, const LicLaunch& L, const 
 {
     return (void)check_lic(L), check_frame(R);
 }
+size_t lic_args_size() { return 64; }
+hipError_t lic_args_fill(const LicLaunch& L, void* args, int* ntiles)
+{
+    std::memset(args, 0, 64);
+    return *ntiles = 1, check_lic(L);
+}
+hipError_t launch_lic_batch(const LicBatchLaunch&, hipStream_t) { return hipSuccess; }
+hipError_t launch_render_batch(const RenderBatchLaunch&, hipStream_t) { return hipSuccess; }
+hipError_t launch_stamp(unsigned long long*, hipStream_t) { return hipSuccess; }
+int render_batch_blocks_per_cu(int, int, int, int, int) { return 1; }
 hipError_t launch_adjoint_forward(const AdjointLaunch& A, hipStream_t) { return check_frame(A.r); }
 }  // namespace vv
 
@@ -164,13 +200,20 @@ struct Scene {
     vv_ctx c;
     explicit Scene(size_t room, int channels = 1)
     {
-        g_limit = lic_size(channels) + 256 + room;
-        g_held = g_mallocs = g_frees = 0;
         g_capture = hipStreamCaptureStatusNone;
         g_query = g_last = hipSuccess;
+        g_limit = 1ull << 40;
+        CHECK(c.field.ensure(field_size(kDims, c.storage)) == hipSuccess);
+        g_limit = g_held + lic_size(channels) + room;
+        g_mallocs = g_frees = 0;
         c.has_field = true;
         for (int a = 0; a < 3; ++a) c.fdims[a] = kDims[a];
         c.lch = channels;
+    }
+    ~Scene()
+    {
+        for (DevBuf* b : c.required()) b->release();
+        for (DevBuf* b : *c.optional) b->release();
     }
     hipError_t lic(int channels = 1)
     {
@@ -263,7 +306,7 @@ static void sample_volume_gives_way()
     // a larger LIC volume does too
     Scene b(1u << 20);
     CHECK(b.lic() == hipSuccess && b.frame());
-    g_limit = lic_size(4) + 256;
+    g_limit = g_held - b.c.lic.bytes - b.c.pair.bytes + lic_size(4);
     CHECK(b.lic(4) == hipSuccess && !b.frame());
 }
 
@@ -328,7 +371,7 @@ static void rgba_copy_gives_way()
     for (int call = 0; call < 3; ++call) {
         CHECK(vv_upload_noise(c, (const uint8_t*)a.data, kDims, 1, nullptr, 1) == VV_OK);
         g_limit = 1ull << 40;
-        for (DevBuf* b : c->optional) b->denied = 0;
+        for (DevBuf* b : *c->optional) b->denied = 0;
         CHECK(vv_compute_lic(c) == VV_OK && vv_render_fused(c, &cam, image.data(), 0, nullptr) == VV_OK);
         (call == 0 ? c->lic : c->image).release();
         c->pair.release();
@@ -343,8 +386,66 @@ static void rgba_copy_gives_way()
     }
 }
 
+// a batch step's sample volume comes with the views that are worth it, serves
+// run and autotune alike, and gives way to another step
+static void batch_sample_volumes()
+{
+    Api a;
+    vv_batch* b = nullptr;
+    CHECK(vv_batch_create(a.c, &b) == VV_OK);
+    auto add_step = [&] {
+        return vv_batch_add_timestep(b, a.data, kDims, nullptr, VV_STORE_FP32, 1, VV_NOISE_UNIFORM, 0.0, 1);
+    };
+    void* image = nullptr;
+    CHECK(hipMalloc(&image, 16 << 20) == hipSuccess);
+    auto add_view = [&](int step, int width) {
+        vv_camera cam;
+        CHECK(vv_default_camera(&cam, width, width, nullptr) == VV_OK);
+        return vv_batch_add_view(b, step, &cam, (float*)image);
+    };
+    // every view that a run shows reads live memory; their number through a sample volume
+    auto run = [&] {
+        CHECK(vv_batch_run(b) == VV_OK);
+        const int frames = g_pair_frames;
+        for (const RenderLaunch& R : b->host_views) CHECK(check_frame(R) == hipSuccess);
+        return g_pair_frames - frames;
+    };
+    auto autotune = [&] {
+        const int frames = g_pair_frames;
+        CHECK(vv_batch_autotune(b) == VV_OK);
+        return g_pair_frames - frames;
+    };
+    CHECK(add_step() == VV_OK && add_view(0, 8) == VV_OK);
+    CHECK(!b->steps[0]->pair.p && run() == 0 && autotune() == 0);
+    CHECK(add_view(0, 512) == VV_OK);
+    CHECK(b->steps[0]->pair.p && run() == 2 && autotune() > 0);
+    int passes = g_pair_passes;
+    CHECK(run() == 2 && g_pair_passes == passes + 1);  // autotune drops the graph
+
+    // the line modes read both volumes
+    a.c->params.illum_mode = VV_ILLUM_MALLO;
+    CHECK(run() == 0);
+    a.c->params.illum_mode = VV_ILLUM_LIC;
+    CHECK(run() == 2);
+
+    // a step that does not fit beside it, with the context's own still there
+    const size_t step = 2 * 16 * (size_t)clamp_elems(kDims) + 5 * (size_t)repeat_elems(kDims);
+    a.c->pair.denied = 0;
+    CHECK(vv_compute_lic(a.c) == VV_OK && a.c->pair.p);
+    free_memory(step - (1u << 16));
+    CHECK(add_step() == VV_OK && add_view(1, 512) == VV_OK);
+    CHECK(!b->steps[0]->pair.p && !a.c->pair.p && b->steps[1]->pair.p);
+    free_memory(1u << 30);
+    CHECK(run() == 1);
+
+    CHECK(vv_batch_destroy(b) == VV_OK);
+    CHECK(hipFree(image) == hipSuccess);
+    CHECK(vv_compute_lic(a.c) == VV_OK && a.c->optional->size() == 2);
+}
+
 int main()
 {
+    batch_sample_volumes();
     rgba_copy_gives_way();
     refused_volumes_are_gone();
     sample_volume_gives_way();

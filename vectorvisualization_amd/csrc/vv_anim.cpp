@@ -48,7 +48,7 @@ vv_status anim_alloc(vv_ctx* c, int nsteps, const int dims[3], const float spaci
     a->storage = storage;
     const size_t bytes = sizeof(float) * 3 * (size_t)nvox(dims);
     for (DevBuf& d : a->steps) {
-        d.spare = &c->optional;
+        d.spare = c->optional.get();
         hipError_t e = d.ensure(bytes);
         if (e) {
             for (DevBuf& x : a->steps) x.release();

@@ -67,7 +67,8 @@ vv_status vv_destroy(vv_ctx* c)
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
         for (DevBuf* b : c->required()) b->release();
-        for (DevBuf* b : c->optional) b->release();
+        c->pair.release();
+        c->lic_field4.release();
         (void)hipStreamDestroy(c->stream);
         delete c;
         return VV_OK;

@@ -38,7 +38,8 @@ struct BatchStep {
     int storage;
     DevBuf field, noise, lic;
     DevBuf lic_field;  // field copy with the noise byte in channel 3 (launch_pack_lic_field)
-    DevBuf pair;       // sample volume of the ray caster (RenderLaunch::pair), made in each run
+    DevBuf pair;       // sample volume of the ray caster (RenderLaunch::pair), made in each run that
+                       // reads it; it may be missing (step_pair)
     int tile[3] = {16, 4, 4};
     int super[3] = {2, 8, 8};
 };
@@ -58,6 +59,7 @@ std::mutex g_tune_mu;
 
 struct vv_batch {
     vv_ctx* ctx = nullptr;
+    std::shared_ptr<std::vector<DevBuf*>> optional;  // the context's
     std::vector<BatchStep*> steps;
     std::vector<BatchView> views;
     DevBuf jobs, first, rviews, vfirst, ctr;
@@ -133,6 +135,26 @@ vv_status build_lic_launch(vv_ctx* c, BatchStep* st, LicLaunch& L)
         L.speed = 1;
     }
     return VV_OK;
+}
+
+// Whether the ray caster reads time step t through its sample volume: its views
+// are worth the pass that makes it, and memory suffices.  Its buffer is
+// allocated here, with the view or parameters that make it worthwhile.
+hipError_t step_pair(vv_batch* b, int t, bool& use)
+{
+    vv_ctx* c = b->ctx;
+    BatchStep* st = b->steps[t];
+    use = false;
+    float tex_max[3];
+    for (int a = 0; a < 3; ++a) tex_max[a] = (float)((double)st->extent[a] * (double)st->scale[a]);
+    if (c->params.illum_mode >= VV_ILLUM_MALLO || !sample_pair_ok(tex_max, st->dims)) return hipSuccess;
+    double samples = 0.0;
+    for (const BatchView& v : b->views)
+        if (v.step == t) samples += pair_samples(v.cam.width, v.cam.height, c->params.step_size_vol);
+    if (samples == 0.0 || samples < kPairSamplesPerVoxel * (double)nvox(st->dims)) return hipSuccess;
+    const hipError_t e = st->pair.ensure_optional(pair_bytes(1, st->dims));
+    use = st->pair.p != nullptr;
+    return e;
 }
 
 vv_status build_view_launch(vv_batch* b, const BatchView& v, RenderLaunch& R)
@@ -218,6 +240,7 @@ vv_status vv_batch_create(vv_ctx* ctx, vv_batch** out)
         vv_batch* b = new (std::nothrow) vv_batch();
         if (!b) return fail(ctx, VV_ENOMEM, "out of host memory");
         b->ctx = ctx;
+        b->optional = ctx->optional;
         *out = b;
         return VV_OK;
     });
@@ -236,6 +259,7 @@ vv_status vv_batch_destroy(vv_batch* b)
             st->lic.release();
             st->lic_field.release();
             st->pair.release();
+            b->optional->erase(std::remove(b->optional->begin(), b->optional->end(), &st->pair), b->optional->end());
             delete st;
         }
         DevBuf* bufs[] = {&b->jobs, &b->first, &b->rviews, &b->vfirst, &b->ctr};
@@ -289,10 +313,10 @@ vv_status vv_batch_add_timestep(vv_batch* b, const float* v0, const int dims[3],
             st->noise.release();
             st->lic.release();
             st->lic_field.release();
-            st->pair.release();
             delete st;
             return s;
         };
+        for (DevBuf* d : {&st->field, &st->noise, &st->lic, &st->lic_field}) d->spare = b->optional.get();
         const float* d0 = v0;
         if (!on_device) {
             vv_status s = upload(c, c->stage, v0, sizeof(float) * 3 * (size_t)n, 0);
@@ -303,14 +327,6 @@ vv_status vv_batch_add_timestep(vv_batch* b, const float* v0, const int dims[3],
         if (!e) e = st->noise.ensure((size_t)repeat_elems(dims));
         if (!e) e = st->lic.ensure(sizeof(float) * (size_t)repeat_elems(dims));
         if (!e) e = st->lic_field.ensure((size_t)field_texel_bytes(storage) * (size_t)clamp_elems(dims));
-        if (!e) {
-            // without memory for it the ray caster samples field and LIC volume
-            const hipError_t ep = st->pair.ensure(sizeof(float) * 2 * (size_t)clamp_elems(dims));
-            if (ep == hipErrorOutOfMemory)
-                (void)hipGetLastError();
-            else
-                e = ep;
-        }
         if (!e) e = c->counter.ensure(64);
         if (!e) e = launch_fill_u32((uint32_t*)c->counter.p, 0u, 1, c->stream);
         if (!e) e = launch_field_maxlen(d0, d0, 0.0f, n, (uint32_t*)c->counter.p, c->stream);
@@ -345,6 +361,7 @@ vv_status vv_batch_add_timestep(vv_batch* b, const float* v0, const int dims[3],
             st->center[a] = st->extent[a] / 2.0f;
         }
         st->storage = storage;
+        b->optional->push_back(&st->pair);
         b->steps.push_back(st);
         release_graph(b);
         b->ran = false;  // the last run's counters no longer match the batch
@@ -410,6 +427,8 @@ vv_status vv_batch_add_view(vv_batch* b, int timestep, const vv_camera* cam, flo
         b->views.push_back(v);
         release_graph(b);
         b->ran = false;
+        bool use;
+        (void)step_pair(b, timestep, use);  // its memory now rather than in the run
         return VV_OK;
     });
 }
@@ -487,17 +506,10 @@ vv_status vv_batch_run(vv_batch* b)
                 ++k;
             }
             gtiles[g] = b->host_vfirst.back();
-            // the step's sample volume, when its views are worth the pass
-            BatchStep* st = b->steps[t];
-            double samples = 0.0;
-            bool usable = st->pair.p && c->params.illum_mode < VV_ILLUM_MALLO && k > (size_t)b->gview[g];
-            for (size_t v = b->gview[g]; v < k; ++v) {
-                const ViewBlock& vb = b->host_views[v].view;
-                samples += pair_samples(vb.width, vb.height, c->params.step_size_vol);
-                usable = usable && sample_pair_ok(vb.tex_max, st->dims);
-            }
-            if (usable && samples >= kPairSamplesPerVoxel * (double)nvox(st->dims))
-                for (size_t v = b->gview[g]; v < k; ++v) b->host_views[v].pair = (const float*)st->pair.p;
+            bool use;
+            HIPCHK(c, step_pair(b, t, use));
+            if (use)
+                for (size_t v = b->gview[g]; v < k; ++v) b->host_views[v].pair = (const float*)b->steps[t]->pair.p;
         }
         b->gview[nsteps] = (int)k;
         b->ngroups = (int)nsteps;
@@ -549,6 +561,7 @@ vv_status vv_batch_run(vv_batch* b)
             // the sample volume's pass takes its arguments by value
             const RenderLaunch* R0 = b->gview[g + 1] > b->gview[g] ? &b->host_views[b->gview[g]] : nullptr;
             key.push_back(R0 && R0->pair ? R0->tf_ch : -1);
+            key.push_back(R0 ? (long long)(intptr_t)R0->pair : 0);
         }
         const bool speed = c->params.speed_of_flow != 0;
         key.push_back(speed);

@@ -12,6 +12,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <string>
 #include <vector>
@@ -196,8 +197,10 @@ struct vv_ctx {
     void* noalloc_scratch = nullptr;  // this device's scratch array (vv_render_adjoint_noalloc)
 
     // the buffers of this context and its batches that may be missing, and are
-    // given up where memory for another one is short
-    std::vector<DevBuf*> optional{&pair, &lic_field4};
+    // given up where memory for another one is short (shared with the batches,
+    // which take theirs out when they end, before or after the context)
+    std::shared_ptr<std::vector<DevBuf*>> optional = std::make_shared<std::vector<DevBuf*>>(
+        std::vector<DevBuf*>{&pair, &lic_field4});
 
     std::array<DevBuf*, 16> required()
     {
@@ -206,7 +209,7 @@ struct vv_ctx {
     }
     vv_ctx()
     {
-        for (DevBuf* b : required()) b->spare = &optional;
+        for (DevBuf* b : required()) b->spare = optional.get();
     }
 };
 
