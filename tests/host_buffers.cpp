@@ -428,6 +428,12 @@ static void batch_sample_volumes()
     a.c->params.illum_mode = VV_ILLUM_LIC;
     CHECK(run() == 2);
 
+    // few samples: neither is worth the pass
+    a.c->params.step_size_vol = 10.0f;
+    CHECK(run() == 0 && autotune() == 0);
+    a.c->params.step_size_vol = 1.0f / 128.0f;
+    CHECK(run() == 2 && autotune() > 0);
+
     // a step that does not fit beside it, with the context's own still there
     const size_t step = 2 * 16 * (size_t)clamp_elems(kDims) + 5 * (size_t)repeat_elems(kDims);
     a.c->pair.denied = 0;

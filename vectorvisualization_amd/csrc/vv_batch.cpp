@@ -774,13 +774,15 @@ vv_status vv_batch_autotune(vv_batch* b)
             static const int blocks[][2] = {{16, 16}, {32, 8}, {64, 4}, {16, 4}, {32, 4}};
             float best = 1e30f;
             int pick[3] = {16, 16, 4};
-            // as the batch renders: through the step's sample volume where it can
+            // as the batch renders: through the step's sample volume or not
             BatchStep* st0 = b->steps[b->views[0].step];
             RenderLaunch V;
             s = build_view_launch(b, b->views[0], V);
             if (s) return s;
             float* pair = nullptr;
-            if (st0->pair.p && V.illum < VV_ILLUM_MALLO && sample_pair_ok(V.view.tex_max, st0->dims)) {
+            bool use;
+            HIPCHK(c, step_pair(b, b->views[0].step, use));
+            if (use) {
                 pair = (float*)st0->pair.p;
                 HIPCHK(c, launch_sample_pair(V.field.p, st0->storage, V.tf_ch, (const float*)V.lic.p, st0->dims, pair,
                                              c->stream));
