@@ -239,6 +239,24 @@ struct Scene {
     }
 };
 
+static size_t free_memory(size_t n) { return g_limit = g_held + n; }
+
+// the library's entry points on a context with a field, noise and LIC volume of kDims
+struct Api {
+    vv_ctx* c = nullptr;
+    float* data = (float*)(1ull << 20);  // inputs and images: device pointers
+    explicit Api(int with_gradients = 0)
+    {
+        g_capture = hipStreamCaptureStatusNone;
+        g_limit = 1ull << 40;
+        CHECK(vv_create(&c, 0) == VV_OK);
+        CHECK(vv_upload_field(c, data, nullptr, 0.0f, kDims, nullptr, VV_STORE_FP32, 1) == VV_OK);
+        CHECK(vv_generate_noise(c, 1, VV_NOISE_UNIFORM, 0.0, kDims, with_gradients) == VV_OK);
+        CHECK(vv_compute_lic(c) == VV_OK);
+    }
+    ~Api() { CHECK(vv_destroy(c) == VV_OK && g_blocks.empty()); }
+};
+
 static void lic_buffer_stays()
 {
     // room for both: the second LIC volume allocates nothing
@@ -283,6 +301,24 @@ static void capture_allocates_nothing()
     CHECK(!b.frame());
 }
 
+// a failed query costs the call its sample volume, not the context, and leaves
+// no error behind
+static void failed_capture_query()
+{
+    for (int channels : {1, 4}) {
+        Scene a(1u << 20, channels);
+        CHECK(a.lic(channels) == hipSuccess && a.frame());
+        g_query = hipErrorUnknown;
+        CHECK(!a.frame() && hipGetLastError() == hipSuccess);
+        g_query = hipSuccess;
+        CHECK(a.frame());
+    }
+    Api b(1);
+    g_query = hipErrorUnknown;
+    CHECK(vv_compute_lic(b.c) == VV_OK && hipGetLastError() == hipSuccess);
+    g_query = hipSuccess;
+}
+
 static void refused_lic_volume_is_gone()
 {
     Scene a(0);
@@ -309,24 +345,6 @@ static void sample_volume_gives_way()
     g_limit = g_held - b.c.lic.bytes - b.c.pair.bytes + lic_size(4);
     CHECK(b.lic(4) == hipSuccess && !b.frame());
 }
-
-static size_t free_memory(size_t n) { return g_limit = g_held + n; }
-
-// the library's entry points on a context with a field, noise and LIC volume of kDims
-struct Api {
-    vv_ctx* c = nullptr;
-    float* data = (float*)(1ull << 20);  // inputs and images: device pointers
-    explicit Api(int with_gradients = 0)
-    {
-        g_capture = hipStreamCaptureStatusNone;
-        g_limit = 1ull << 40;
-        CHECK(vv_create(&c, 0) == VV_OK);
-        CHECK(vv_upload_field(c, data, nullptr, 0.0f, kDims, nullptr, VV_STORE_FP32, 1) == VV_OK);
-        CHECK(vv_generate_noise(c, 1, VV_NOISE_UNIFORM, 0.0, kDims, with_gradients) == VV_OK);
-        CHECK(vv_compute_lic(c) == VV_OK);
-    }
-    ~Api() { CHECK(vv_destroy(c) == VV_OK && g_blocks.empty()); }
-};
 
 // no kernel runs on a volume whose buffer could not grow
 static void refused_volumes_are_gone()
@@ -457,6 +475,7 @@ int main()
     sample_volume_gives_way();
     lic_buffer_stays();
     capture_allocates_nothing();
+    failed_capture_query();
     refused_lic_volume_is_gone();
     return g_failed;
 }

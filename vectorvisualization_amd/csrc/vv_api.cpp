@@ -551,9 +551,8 @@ vv_status fill_lic_launch(vv_ctx* c, LicLaunch& L, void* out)
     // volume; so does a call under capture with RGBA noise, whose graph then
     // reads what later uploads put into the field.
     const bool grid = c->ndims[0] == c->fdims[0] && c->ndims[1] == c->fdims[1] && c->ndims[2] == c->fdims[2];
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (L.cache && !L.speed && nc == 4 && c->storage == VV_STORE_FP32 && grid &&
-        hipStreamIsCapturing(c->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        capture_status(c) == hipStreamCaptureStatusNone) {
         if (!c->lic_field4_ok || !c->lic_field4.p) {
             HIPCHK(c, c->lic_field4.ensure_optional((size_t)L.field_bytes));
             c->lic_field4_ok = c->lic_field4.bytes >= L.field_bytes;

@@ -496,13 +496,24 @@ inline void illum_lut_ptrs(vv_ctx* c, RenderLaunch& R)
     R.lut_mallo_spec = base + 256 * 256 * 5;
 }
 
+// Whether the context's stream records a graph.  Invalidated where the runtime
+// does not say (the call then does without what a graph must not read, and the
+// error is not left for the next launch to report).
+inline hipStreamCaptureStatus capture_status(vv_ctx* c)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) == hipSuccess) return st;
+    (void)hipGetLastError();
+    return hipStreamCaptureStatusInvalidated;
+}
+
 // whether a sample volume may be used and kept: not while the context's
 // stream is being captured, nor after (vv_ctx::pair_off)
 inline bool pair_allowed(vv_ctx* c)
 {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) c->pair_off = true;
-    return !c->pair_off;
+    const hipStreamCaptureStatus st = capture_status(c);
+    if (st == hipStreamCaptureStatusActive) c->pair_off = true;
+    return st == hipStreamCaptureStatusNone && !c->pair_off;
 }
 
 // drops the sample volume of a LIC volume or field about to change
