@@ -510,7 +510,15 @@ vv_status vv_anim_destroy(vv_anim* a);
  * multiples of 64), "render.ray_group" (lanes per ray of vv_render_fused /
  * vv_render_slices, a power of two up to 64; 0 = enough lanes for about
  * 2^21 in total with an FP32 field and 2^22 with FP16 or UNORM8, at most 32
- * per ray).  Images and sample counts do not depend on the lanes per ray.
+ * per ray), "render.sample_volume" (0/1, 1 by default: with each LIC volume
+ * on the field's grid the context reserves a volume of LIC value and field
+ * channel, 8 bytes per voxel, 4 with RGBA noise, that vv_render,
+ * vv_render_record and vv_render_adjoint read in place of the two; memory that
+ * another buffer needs is taken back.  vv_compute_lic under stream capture
+ * sets it to 0, since that graph rewrites the LIC volume at each replay; set it
+ * to 1 again once the graph is no longer replayed.  Setting it releases the
+ * volume; the next LIC volume brings it).
+ * Images and sample counts do not depend on the lanes per ray.
  * Results do not depend on these settings. */
 vv_status vv_set_tuning(vv_ctx* ctx, const char* key, int value);
 vv_status vv_get_tuning(const vv_ctx* ctx, const char* key, int* value);

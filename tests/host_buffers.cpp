@@ -292,13 +292,35 @@ static void capture_allocates_nothing()
     g_capture = hipStreamCaptureStatusNone;
     CHECK(a.lic() == hipSuccess && a.c.lic.p == p && g_mallocs == n && g_frees == f);
 
-    // a graph replays without the context's flags: no sample volume after it
+    // no captured frame reads the sample volume; a captured LIC volume changes
+    // unseen, so no later frame does either
     Scene b(1u << 20);
     CHECK(b.lic() == hipSuccess && b.frame());
+    g_capture = hipStreamCaptureStatusActive;
+    CHECK(!b.frame());
+    g_capture = hipStreamCaptureStatusNone;
+    CHECK(b.frame());
     g_capture = hipStreamCaptureStatusActive;
     CHECK(b.lic() == hipSuccess && !b.frame());
     g_capture = hipStreamCaptureStatusNone;
     CHECK(!b.frame());
+
+    // until the caller says that none is replayed any more
+    int on = -1;
+    CHECK(vv_get_tuning(&b.c, "render.sample_volume", &on) == VV_OK && on == 0);
+    CHECK(vv_set_tuning(&b.c, "render.sample_volume", 1) == VV_OK && !b.c.pair.p && !b.frame());
+    CHECK(b.lic() == hipSuccess && b.frame());
+}
+
+// "render.sample_volume" 0: no memory for it
+static void switched_off()
+{
+    Scene a(1u << 20);
+    CHECK(vv_set_tuning(&a.c, "render.sample_volume", 2) == VV_EINVAL);
+    CHECK(vv_set_tuning(&a.c, "render.sample_volume", 0) == VV_OK);
+    CHECK(a.lic() == hipSuccess && !a.frame() && !a.c.pair.p);
+    CHECK(vv_set_tuning(&a.c, "render.sample_volume", 1) == VV_OK && a.lic() == hipSuccess && a.frame());
+    CHECK(vv_set_tuning(&a.c, "render.sample_volume", 0) == VV_OK && !a.c.pair.p && !a.frame());
 }
 
 // a failed query costs the call its sample volume, not the context, and leaves
@@ -475,6 +497,7 @@ int main()
     sample_volume_gives_way();
     lic_buffer_stays();
     capture_allocates_nothing();
+    switched_off();
     failed_capture_query();
     refused_lic_volume_is_gone();
     return g_failed;

@@ -704,14 +704,21 @@ vv_status vv_set_tuning(vv_ctx* c, const char* key, int value)
         else if (k == "render.block_y") slot = &c->render_block[1];
         else if (k == "render.ray_group") slot = &c->ray_group;
         else if (k == "render.volume_group") slot = &c->volume_group;
+        else if (k == "render.sample_volume") slot = &c->pair_on;
         else return fail(c, VV_EINVAL, "unknown tuning key '%s'", key);
-        if (k == "lic.cache" || k == "lic.brick" || k == "adjoint.window") {
+        if (k == "lic.cache" || k == "lic.brick" || k == "adjoint.window" || k == "render.sample_volume") {
             if (value != 0 && value != 1) return fail(c, VV_EINVAL, "%s must be 0 or 1", key);
         } else if (k == "render.ray_group" || k == "render.volume_group") {
             if (value < 0 || value > 64 || (value & (value - 1)))
                 return fail(c, VV_EINVAL, "%s must be 0 (automatic) or a power of two up to 64", key);
         } else if (value < 1 || value > 256 || (value & (value - 1))) {
             return fail(c, VV_EINVAL, "tile sizes must be powers of two in [1,256]");
+        }
+        if (slot == &c->pair_on) {
+            // made from the next LIC volume on, which brings its memory
+            drop_pair(c);
+            if (capture_status(c) == hipStreamCaptureStatusNone) c->pair.release();
+            c->pair.denied = 0;
         }
         *slot = value;  // render block pairs are checked when a frame is rendered
         return VV_OK;
@@ -736,6 +743,7 @@ vv_status vv_get_tuning(const vv_ctx* c, const char* key, int* value)
         else if (k == "render.block_y") *value = c->render_block[1];
         else if (k == "render.ray_group") *value = c->ray_group;
         else if (k == "render.volume_group") *value = c->volume_group;
+        else if (k == "render.sample_volume") *value = c->pair_on;
         else return VV_EINVAL;
         return VV_OK;
     });

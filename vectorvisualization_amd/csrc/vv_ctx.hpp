@@ -154,9 +154,10 @@ struct vv_ctx {
     bool pair_ok = false;
     int pair_ch = 0;
     double pair_used = 0.0;
-    // a graph that captured the context's LIC or frames replays without its
-    // flags: no sample volume from then on
-    bool pair_off = false;
+    // whether a sample volume may be used ("render.sample_volume").  A graph that
+    // captured vv_compute_lic changes the LIC volume without a word to the
+    // context, so that capture clears it; the caller sets it again.
+    int pair_on = 1;
 
     // launch tuning (vv_set_tuning)
     int lic_tile[3] = {16, 4, 4};
@@ -507,15 +508,6 @@ inline hipStreamCaptureStatus capture_status(vv_ctx* c)
     return hipStreamCaptureStatusInvalidated;
 }
 
-// whether a sample volume may be used and kept: not while the context's
-// stream is being captured, nor after (vv_ctx::pair_off)
-inline bool pair_allowed(vv_ctx* c)
-{
-    const hipStreamCaptureStatus st = capture_status(c);
-    if (st == hipStreamCaptureStatusActive) c->pair_off = true;
-    return st == hipStreamCaptureStatusNone && !c->pair_off;
-}
-
 // drops the sample volume of a LIC volume or field about to change
 inline void drop_pair(vv_ctx* c)
 {
@@ -538,7 +530,9 @@ inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
     const size_t lic = sizeof(float) * channels * (size_t)repeat_elems(d), pair = pair_bytes(channels, d);
     drop_pair(c);
     const hipError_t e = c->lic.ensure(lic, c->has_lic);
-    if (e != hipSuccess || !pair_allowed(c) || (channels == 1 && !pair_addressable(d))) return e;
+    const hipStreamCaptureStatus st = capture_status(c);
+    if (st == hipStreamCaptureStatusActive) c->pair_on = 0;
+    if (e != hipSuccess || !c->pair_on || st != hipStreamCaptureStatusNone || (channels == 1 && !pair_addressable(d))) return e;
     return c->pair.ensure_optional(pair);
 }
 
@@ -555,7 +549,8 @@ inline vv_status ensure_pair(vv_ctx* c, RenderLaunch& R)
         return VV_OK;
     for (int a = 0; a < 3; ++a)
         if (c->ldims[a] != c->fdims[a]) return VV_OK;
-    if (!pair_allowed(c)) return VV_OK;
+    // a captured frame would be drawn from it after it changed
+    if (!c->pair_on || capture_status(c) != hipStreamCaptureStatusNone) return VV_OK;
     if (!c->pair_ok || c->pair_ch != R.tf_ch) {
         if (c->pair_ch != R.tf_ch) drop_pair(c);
         c->pair_ch = R.tf_ch;
