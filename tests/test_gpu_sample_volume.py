@@ -1,5 +1,6 @@
-"""The ray casters' sample volume where a captured graph rewrites what it was
-made of."""
+"""The ray casters' sample volume against the two volumes it is made of, switched
+by "render.sample_volume": with an opacity scale, on stretched boxes, past
+2 GiB, and where a captured graph rewrites what it was made of."""
 import numpy as np
 import pytest
 import torch
@@ -66,3 +67,70 @@ def test_captured_lic_and_frame(ctx, grad):
         assert np.max(want) > 0
         np.testing.assert_array_equal(got, want)
         np.testing.assert_array_equal(plain, want)
+
+
+def _off_and_on(ctx, load, draw):
+    """draw() from the two volumes and through the sample volume, which frames of
+    this size have made by then."""
+    large = _cams(ctx)[0]
+    out = []
+    for on in (0, 1):
+        ctx.set_tuning("render.sample_volume", on)
+        load()
+        for _ in range(2):
+            ctx.render(large)
+        out.append(draw())
+    for a, b in zip(*out):
+        assert np.any(a != 0)
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", [vv.STORE_FP32, vv.STORE_FP16, vv.STORE_UNORM8])
+@pytest.mark.parametrize("dims,spacing", [((40, 33, 37), (1.0, 1.0, 1.0)), ((36, 40, 44), (1.3, 1.0, 1.1))])
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("index", [vv.TF_INDEX_B, vv.TF_INDEX_MAG])
+def test_opacity_scale(ctx, storage, dims, spacing, grad, index):
+    """Frame, recorded frame and both gradients with an opacity scale."""
+    p = _scene(ctx, dims, 4, grad, storage, spacing)
+    p.tf_index = index
+    ctx.set_lic_params(p)
+    cam = _cams(ctx)[1]
+    sigma = np.random.default_rng(5).uniform(0.5, 1.5, dims[0] * dims[1] * dims[2]).astype(np.float32)
+    dimg = np.random.default_rng(6).normal(size=cam.width * cam.height * 4).astype(np.float32)
+
+    def load():
+        ctx.compute_lic()
+        ctx.set_opacity_scale(sigma)
+
+    def draw():
+        return [ctx.render(cam), ctx.render_record(cam), *ctx.render_adjoint(cam, dimg)]
+
+    _off_and_on(ctx, load, draw)
+
+
+def test_past_2gib(ctx):
+    """A sample volume of 3.4 GB, read with 32-bit byte offsets."""
+    dims = (1024, 1024, 400)
+    assert 2 ** 31 < 8 * (dims[0] + 2) * (dims[1] + 2) * (dims[2] + 2) < 2 ** 32
+    z = torch.linspace(0.0, 9.0, dims[2], device="cuda").view(-1, 1, 1)
+    y = torch.linspace(0.0, 7.0, dims[1], device="cuda").view(1, -1, 1)
+    x = torch.linspace(0.0, 5.0, dims[0], device="cuda").view(1, 1, -1)
+    v = torch.empty(dims[::-1] + (3,), device="cuda")
+    v[..., 0], v[..., 1], v[..., 2] = torch.sin(z) + 0 * y + 0 * x, torch.cos(x) + 0 * y + 0 * z, torch.sin(y) * z + 0 * x
+    ctx.upload_field(v, dims, storage=vv.STORE_UNORM8)
+    del v
+    lic = torch.rand(dims[::-1], device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    p = vv.default_lic_params()
+    p.step_size_vol, p.num_iterations = 1.0 / 1024.0, 64
+    ctx.set_lic_params(p)
+    ctx.set_tf(*fields.tf_magnitude(0.02, 0.01))
+    cen = ctx.field_geometry()[2]
+    frames = []
+    for on in (0, 1):
+        ctx.set_tuning("render.sample_volume", on)
+        ctx.upload_lic(lic, 1, dims)
+        cams = [fields.orbit_camera(1024, 1024, cen, yaw, pitch) for yaw, pitch in ((0.4, 0.3), (2.8, -0.3))]
+        frames.append([ctx.render(c).copy() for c in cams])
+    for a, b in zip(*frames):
+        assert np.max(a) > 0.01
+        np.testing.assert_array_equal(a, b)
