@@ -1025,7 +1025,6 @@ __global__ void __launch_bounds__(kRThreads) k_adjoint_forward_rg(AdjointLaunch 
     float max_am = 0.0f, max_q = 0.0f, max_qr = 0.0f, gamma = 1.0f;
     unsigned mb[2] = {0u, 0u};  // clamp masks of the part, samples 0-7 and 8-15
     const int kmax = (int)a.max_samples;
-    bool finite_so_far = true;  // the same in every lane of the wave
     // bk, the round's first sample, is the same for all rays: a round lies in
     // one part of one segment
     for (int bk = 0; alive; bk += GT) {
@@ -1053,62 +1052,36 @@ __global__ void __launch_bounds__(kRThreads) k_adjoint_forward_rg(AdjointLaunch 
         group_gather<GT>(rsum, rs);
         const unsigned long long okb = __ballot((int)ok);
         // compositing in sample order; this lane keeps D before its own sample
-        const float d0[4] = {dest[0], dest[1], dest[2], dest[3]};
         float mine_d[4] = {0.f, 0.f, 0.f, 0.f};
         int ncomp = 0;
-        bool clamped = false;
-        auto round = [&](auto finite) {
+        unsigned m = 0;  // the round's clamp masks, 4 bits per sample
 #pragma unroll
-            for (int g = 0; g < GT; ++g) {
-                if (!group_bit<GT>(okb, g)) {
-                    alive = false;
-                    break;
-                }
-                if (g == sub)
-                    for (int q = 0; q < 4; ++q) mine_d[q] = dest[q];
-                const float sv[4] = {s0[g], s1[g], s2[g], s3[g]};
-                const float t = 1.0f - dest[3];
-                for (int q = 0; q < 4; ++q) {
-                    const float u = fmaf(t, sv[q], dest[q]);
-                    dest[q] = finite.value ? __builtin_amdgcn_fmed3f(u, 0.0f, 1.0f) : clamp01(u);
-                    clamped |= u < 0.0f || u > 1.0f;
-                }
-                gamma = fmaf(s3[g], rs[g], gamma);
-                ++ncomp;
-                if (dest[3] > 0.95f) {
-                    alive = false;
-                    break;
-                }
+        for (int g = 0; g < GT; ++g) {
+            if (!group_bit<GT>(okb, g)) {
+                alive = false;
+                break;
             }
-        };
-        if (finite_so_far && wave_finite(src)) {
-            round(std::true_type{});
-        } else {
-            finite_so_far = false;
-            round(std::false_type{});
-        }
-        // the round's clamp masks, 4 bits per sample: zero unless some lane
-        // clamped, then from the round's compositing again
-        if (__any(clamped)) {
-            float d[4] = {d0[0], d0[1], d0[2], d0[3]};
-            unsigned m = 0;
-#pragma unroll
-            for (int g = 0; g < GT; ++g) {
-                if (g >= ncomp) break;
-                const float sv[4] = {s0[g], s1[g], s2[g], s3[g]};
-                const float t = 1.0f - d[3];
-                for (int q = 0; q < 4; ++q) {
-                    const float u = fmaf(t, sv[q], d[q]);
-                    if (u < 0.0f || u > 1.0f) m |= 1u << (4 * g + q);
-                    d[q] = clamp01(u);
-                }
+            if (g == sub)
+                for (int q = 0; q < 4; ++q) mine_d[q] = dest[q];
+            const float sv[4] = {s0[g], s1[g], s2[g], s3[g]};
+            const float t = 1.0f - dest[3];
+            for (int q = 0; q < 4; ++q) {
+                const float u = fmaf(t, sv[q], dest[q]);
+                if (u < 0.0f || u > 1.0f) m |= 1u << (4 * g + q);
+                dest[q] = clamp01(u);
             }
-            const int at = bk % kSub;
-            if (at < 8)
-                mb[0] |= m << (4 * at);
-            else
-                mb[1] |= m << (4 * (at - 8));
+            gamma = fmaf(s3[g], rs[g], gamma);
+            ++ncomp;
+            if (dest[3] > 0.95f) {
+                alive = false;
+                break;
+            }
         }
+        const int at = bk % kSub;
+        if (at < 8)
+            mb[0] |= m << (4 * at);
+        else
+            mb[1] |= m << (4 * (at - 8));
         // this lane's sample, when composited: its column entries
         const int kk0 = bk % kSeg, c = bk / kSeg;
         const AdjColumn col = adj_column(A, nrays, c);
