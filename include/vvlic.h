@@ -502,11 +502,12 @@ vv_status vv_anim_destroy(vv_anim* a);
  * an LDS window per ray segment before the global integer atomics),
  * "render.volume_group" (lanes per ray of vv_render, a power of two up to
  * 64; 1 = one lane per pixel; 0 = the power of two, at most 16, below
- * 16 / (step_size_vol sqrt(width height)), at least 1; the forward pass of
- * vv_render_record and of the adjoints and the adjoints' backward walk take
- * 4, or the set value if it is smaller; with 0 the forward pass takes 2 from
- * 2^19 rays and 1 from 3 2^19; gradients do not depend on it), "render.block_x", "render.block_y" (pixel
- * tile of vv_render with one lane per pixel, 64 to 256 threads in
+ * 16 / (step_size_vol sqrt(width height)), at least 1, with line illumination
+ * at least 4 and 2^20 in all; the forward pass of vv_render_record and of the
+ * adjoints and the adjoints' backward walk take 4, or the set value if it is
+ * smaller; with 0 the forward pass takes fewer in views of more than 2^18 rays
+ * where its scratch keeps a column per 64 samples of a ray, at most 8 GiB;
+ * gradients do not depend on it), "render.block_x", "render.block_y" (pixel tile of vv_render with one lane per pixel, 64 to 256 threads in
  * multiples of 64), "render.ray_group" (lanes per ray of vv_render_fused /
  * vv_render_slices, a power of two up to 64; 0 = enough lanes for about
  * 2^21 in total with an FP32 field and 2^22 with FP16 or UNORM8, at most 32

@@ -489,8 +489,50 @@ static void batch_sample_volumes()
     CHECK(vv_compute_lic(a.c) == VV_OK && a.c->optional->size() == 2);
 }
 
+// lanes per ray: the measured best of each size, or what is within 5 % of it
+static void lanes_per_ray()
+{
+    Api a;
+    RenderLaunch R;
+    std::memset(&R, 0, sizeof(R));
+    auto view = [&](int n, int width, int illum, int lc, bool pair) {
+        R.view.width = R.view.height = width;
+        R.step = 1.0f / (float)n;
+        R.illum = illum;
+        R.lc = lc;
+        R.pair = pair ? (const float*)&R : nullptr;
+    };
+    const struct { int n, width, illum, lc, pair, lo, hi; } frames[] = {
+        {128, 256, 0, 1, 1, 8, 8},   {256, 256, 0, 1, 1, 16, 16}, {256, 1024, 0, 1, 1, 2, 4}, {128, 1448, 0, 1, 1, 1, 1},
+        {128, 256, 2, 1, 0, 16, 16}, {128, 512, 2, 1, 0, 4, 4},   {128, 768, 3, 1, 0, 4, 4},  {128, 1448, 3, 1, 0, 2, 4},
+        {256, 256, 3, 1, 0, 16, 16}, {256, 512, 3, 1, 0, 8, 8},   {256, 1024, 2, 1, 0, 4, 4}, {256, 1448, 2, 1, 0, 2, 4}};
+    for (const auto& f : frames) {
+        view(f.n, f.width, f.illum, f.lc, f.pair);
+        const int G = volume_group_for(a.c, R);
+        CHECK(G >= f.lo && G <= f.hi);
+    }
+    const struct { int n, width, illum, lc, pair, lo, hi; } records[] = {
+        {128, 512, 0, 1, 1, 2, 4},  {128, 768, 0, 1, 1, 1, 2},  {128, 1024, 0, 1, 1, 1, 1}, {256, 640, 0, 1, 1, 4, 4},
+        {256, 768, 0, 1, 1, 2, 2},  {256, 1024, 0, 1, 1, 2, 2}, {256, 1448, 0, 1, 1, 1, 1}, {512, 768, 0, 1, 1, 4, 4},
+        {512, 1448, 0, 1, 1, 2, 2}, {512, 2048, 0, 1, 1, 1, 2}, {128, 768, 1, 4, 1, 2, 2},  {128, 1448, 1, 4, 1, 1, 2},
+        {256, 768, 1, 4, 1, 4, 4},  {256, 1448, 1, 4, 1, 2, 2}, {256, 2048, 1, 4, 1, 1, 2}, {128, 1024, 0, 1, 0, 2, 2},
+        {128, 2048, 0, 1, 0, 1, 1}, {256, 768, 0, 1, 0, 4, 4},  {256, 1024, 0, 1, 0, 4, 4}, {256, 1448, 1, 4, 0, 2, 2},
+        {512, 1024, 0, 1, 0, 4, 4}, {128, 640, 2, 1, 0, 4, 4},  {128, 1448, 3, 1, 0, 2, 2}, {256, 768, 3, 1, 0, 4, 4},
+        {256, 1024, 2, 1, 0, 4, 4}, {256, 1448, 2, 1, 0, 2, 4}, {512, 1024, 2, 1, 0, 4, 4}, {512, 1448, 3, 1, 0, 4, 4}};
+    for (const auto& f : records) {
+        view(f.n, f.width, f.illum, f.lc, f.pair);
+        const int G = record_group_for(a.c, R, 4);
+        CHECK(G >= f.lo && G <= f.hi);
+        CHECK(record_group_for(a.c, R, 2) <= 2);
+        a.c->volume_group = 1;
+        CHECK(record_group_for(a.c, R, 1) == 1 && volume_group_for(a.c, R) == 1);
+        a.c->volume_group = 0;
+    }
+}
+
 int main()
 {
+    lanes_per_ray();
     batch_sample_volumes();
     rgba_copy_gives_way();
     refused_volumes_are_gone();

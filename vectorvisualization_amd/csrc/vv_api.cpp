@@ -780,13 +780,35 @@ vv_status vv_view_block(const vv_ctx* c, const vv_camera* cam, float out24[24])
 //                      1024^2 261 178 174 241 442,  1448^2 244 221 265 411 819
 //   96^3, step 1/128    256^2  71  58  47  45  48,   512^2  69  63  60  65  98,
 //                      1024^2 104  90 105 158 305,  1448^2 114 125 160 268 569
-static int volume_group_for(const vv_ctx* c, const vv_camera* cam)
+// The line modes' samples cost several times as much to evaluate as to
+// composite, so lanes that share them pay earlier: at least 4, and 2^20 in all.
+// 64^3, step 1/128, Zoeckler: 256^2 141  82  55  52  47,  1448^2 433 340 357 540 885.
+static int volume_group_for(const vv_ctx* c, const RenderLaunch& R)
 {
     if (c->volume_group > 0) return c->volume_group;
-    const double g = 16.0 / ((double)c->params.step_size_vol * std::sqrt((double)cam->width * cam->height));
+    const double rays = (double)R.view.width * R.view.height, g = 16.0 / ((double)R.step * std::sqrt(rays));
     int G = 1;
     while (G < 16 && 2.0 * G <= g) G *= 2;
+    while (R.illum >= VV_ILLUM_MALLO && G < 16 && (G < 4 || rays * G < (double)(1 << 20))) G *= 2;
     return G;
+}
+
+// The same of the recorded frame with a column per segment, at most 4: views of
+// up to 2^18 rays take all of them, in larger ones the rays fill the GPU the
+// sooner the cheaper a sample is.  Lanes 1 / 2 / 4 (us):
+//   sample volume      128^3   768^2  83  86 104,  256^3 1024^2 283 245 271,  512^3 1024^2 1114  696  546
+//   its RGBA plane     128^3   768^2 198 168 179,  256^3  768^2 604 364 342,  256^3 2048^2 1300 1354 1584
+//   two volumes        128^3  1024^2 197 179 209,  256^3 1024^2 602 429 404,   64^3 2048^2  405  501  705
+//   line illumination  128^3  1448^2 469 404 467,  256^3 1024^2 934 677 596,  512^3 1024^2 2921 2098 1391
+static int record_group_for(const vv_ctx* c, const RenderLaunch& R, int most)
+{
+    const double rays = (double)R.view.width * R.view.height, g = 16.0 / ((double)R.step * std::sqrt(rays));
+    if (c->volume_group > 0 || rays <= (double)(1 << 18)) return most;
+    const bool line = R.illum >= VV_ILLUM_MALLO;
+    const double two = line ? 0.0 : !R.pair ? 1.5 : R.lc == 4 ? 2.2 : 3.0;
+    const double four = line ? 3.0 : !R.pair ? 4.0 : R.lc == 4 ? 5.0 : 6.0;
+    const int G = g < two ? 1 : g < four ? 2 : 4;
+    return G < most ? G : most;
 }
 
 vv_status vv_render(vv_ctx* c, const vv_camera* cam, float* image, int on_device, uint64_t* samples_out)
@@ -812,7 +834,7 @@ vv_status vv_render(vv_ctx* c, const vv_camera* cam, float* image, int on_device
         }
         st = ensure_pair(c, R);
         if (st) return st;
-        const int G = volume_group_for(c, cam);
+        const int G = volume_group_for(c, R);
         if (G > 1)
             HIPCHK(c, launch_render_rg(R, G, c->stream));
         else
@@ -1011,14 +1033,6 @@ static vv_status adjoint_setup(vv_ctx* c, const vv_camera* cam, AdjointLaunch& A
     // both walks take 4 lanes per ray unless the tuning asks for fewer (with 2
     // the voxel boxes of the opacity-scale windows overflow on oblique views)
     A.group = c->volume_group > 0 && c->volume_group < 4 ? c->volume_group : 4;
-    // a large view has rays enough without lanes for each: recorded frame of
-    // 128^3 at 1/128, 1, 2 and 4 lanes, on an oblique view: 512^2 .130, .125,
-    // .116 ms; 768^2 .127, .134, .153; 1024^2 .142, .162, .207; 1536^2 .182,
-    // .257, .375; of 256^3 at 1/256: 768^2 .246, .237, .248; 1024^2 .351, .290,
-    // .354; 1536^2 .402, .484, .658
-    const long long rays = (long long)cam->width * cam->height;
-    const int most = rays < (1ll << 19) ? 4 : rays < 3 * (1ll << 19) ? 2 : 1;
-    A.fwd_group = c->volume_group > 0 || A.group < most ? A.group : most;
     return VV_OK;
 }
 
@@ -1037,6 +1051,7 @@ static void adjoint_bind(AdjointLaunch& A, char* scratch, const AdjScratchLayout
 // The adjoint's forward pass (header word 0 cleared first).
 static vv_status adjoint_forward(vv_ctx* c, AdjointLaunch& A)
 {
+    A.fwd_group = record_group_for(c, A.r, A.group);
     HIPCHK(c, launch_fill_i64(reinterpret_cast<long long*>(A.hdr), 0, 1, c->stream));
     HIPCHK(c, launch_adjoint_forward(A, c->stream));
     return VV_OK;
