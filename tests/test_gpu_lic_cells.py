@@ -89,3 +89,20 @@ def test_captured_lic_reads_later_fields(ctx):
         got = ctx.download_lic()
         ctx.compute_lic()
         np.testing.assert_array_equal(got, ctx.download_lic())
+
+
+@pytest.mark.parametrize("storage", [vv.STORE_FP32, vv.STORE_FP16, vv.STORE_UNORM8])
+@pytest.mark.parametrize("kind", ["rgba", "rgba_off", "gate"])
+@pytest.mark.parametrize("group", [0, 1, 4])
+@pytest.mark.parametrize("steps,width", [((4, 4), 37), ((5, 4), 37), ((8, 8), 149), ((9, 8), 149)])
+def test_slices_of_short_and_longer_streamlines(ctx, storage, kind, group, steps, width):
+    """Slices on both sides of the length from which they take the caches."""
+    p = _scene(ctx, (13, 11, 7), storage, kind, 0.03, 0)
+    p.step_size_vol = 1 / 32
+    p.steps_forward, p.steps_backward = steps
+    ctx.set_lic_params(p)
+    ctx.set_tuning("render.ray_group", group)
+    cam = fields.orbit_camera(width, 111, (0.5, 0.5, 0.5), 0.4, 0.3)
+    a, b = _both(ctx, lambda: ctx.render_slices(cam))
+    assert np.abs(a).max() > 0
+    np.testing.assert_array_equal(a, b)

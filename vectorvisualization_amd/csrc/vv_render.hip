@@ -2124,21 +2124,33 @@ namespace {
 // pay for every noise, gate and caster (128^3, 20+20 steps, 512 x 512, without
 // and with them: RGBA FP32 fused 6.8 -> 2.0 ms, slices 3.5 -> 1.5; FP16 4.2 ->
 // 2.2, 3.0 -> 2.2; UNORM8 4.1 -> 2.3, 2.9 -> 2.3; gate FP32 7.2 -> 2.9, FP16
-// slices 3.8 -> 2.4), also where a kernel then passes 128 registers.
-// SPEED_OF_FLOW takes 0.
+// slices 3.8 -> 2.4), also where a kernel then passes 128 registers, but for
+// short streamlines in slices: there most of the time is the fragments around
+// the LIC, and three waves per SIMD instead of four (gate in FP32 and UNORM8,
+// 141 registers; RGBA noise in FP16, 136) cost more than the loads.  128^3 with
+// the caches against without: 120^2, 2+2 steps 1.12 to 1.19, 4+4 1.00 to 1.08,
+// 6+6 .90 to .96; 200^2 to 512^2, 2+2 steps 1.12 to 1.21, 8+8 1.02 to 1.16, 12+12
+// .86 to 1.12.  SPEED_OF_FLOW takes 0.
+inline int short_lic(const RenderLaunch& R)
+{
+    return (long long)R.view.width * R.view.height > (1ll << 14) ? 16 : 8;
+}
+
 struct LicVariant {
     bool gate;
     int nc;
     int mode;
 };
 
-LicVariant lic_variant(const LicLaunch& L)
+LicVariant lic_variant(const RenderLaunch& R, const LicLaunch& L, bool slices)
 {
     LicVariant v;
     v.gate = L.gate != 0;
     v.nc = L.nc;
     const LicKind k = lic_kind(L);
-    v.mode = k == LicKind::Direct || L.speed ? 0 : k == LicKind::Copy || k == LicKind::Copy4 ? 2 : 1;
+    const bool three_waves = k == LicKind::Cells && (L.gate ? L.field_type != 1 : L.field_type == 1);
+    const bool direct = k == LicKind::Direct || L.speed || (slices && three_waves && L.F + L.B <= short_lic(R));
+    v.mode = direct ? 0 : k == LicKind::Copy || k == LicKind::Copy4 ? 2 : 1;
     return v;
 }
 
@@ -2180,7 +2192,7 @@ hipError_t launch_render_fused(const RenderLaunch& R, const LicLaunch& L, hipStr
     if (e != hipSuccess) return e;
     dim3 block(bx, by);
     dim3 grid((R.view.width + bx - 1) / bx, (R.view.height + by - 1) / by);
-    const LicVariant v = lic_variant(L);
+    const LicVariant v = lic_variant(R, L, false);
     return with_field_type(R.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
         with_lic_variant<FT>(v, [&](auto nc, auto gate, auto mode) {
@@ -2199,7 +2211,7 @@ hipError_t launch_render_slices(const RenderLaunch& R, const LicLaunch& L, const
     if (e != hipSuccess) return e;
     dim3 block(bx, by);
     dim3 grid((R.view.width + bx - 1) / bx, (R.view.height + by - 1) / by);
-    const LicVariant v = lic_variant(L);
+    const LicVariant v = lic_variant(R, L, true);
     return with_field_type(R.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
         with_lic_variant<FT>(v, [&](auto nc, auto gate, auto mode) {
@@ -2223,7 +2235,7 @@ hipError_t launch_render_group(const RenderLaunch& R, const LicLaunch& L, const 
     const long long nblocks = (long long)((R.view.width + TW - 1) / TW) * ((R.view.height + TH - 1) / TH);
     if (nblocks > 0x7fffffffLL) return hipErrorInvalidValue;
     dim3 grid((unsigned)nblocks), block(kRThreads);
-    const LicVariant v = lic_variant(L);
+    const LicVariant v = lic_variant(R, L, slices);
     return with_field_type(R.field_type, [&](auto tag) {
         using FT = typename decltype(tag)::type;
         with_lic_variant<FT>(v, [&](auto nc, auto gate, auto mode) {
