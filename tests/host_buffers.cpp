@@ -218,12 +218,11 @@ struct Scene {
     hipError_t lic(int channels = 1)
     {
         const hipError_t e = lic_buffer(&c, channels, kDims);
-        if (e == hipSuccess) {
-            c.has_lic = true;
-            c.lch = channels;
-            for (int a = 0; a < 3; ++a) c.ldims[a] = kDims[a];
-        }
-        return e;
+        if (e != hipSuccess) return e;
+        c.has_lic = true;
+        c.lch = channels;
+        for (int a = 0; a < 3; ++a) c.ldims[a] = kDims[a];
+        return pair_buffer(&c);
     }
     // whether a frame large enough to be worth it samples through the sample volume
     bool frame()

@@ -626,6 +626,7 @@ vv_status vv_compute_lic(vv_ctx* c)
         c->lch = nc;
         c->has_lic = true;
         ++c->scene_version;
+        HIPCHK(c, pair_buffer(c));
         return VV_OK;
     });
 }
@@ -673,12 +674,13 @@ vv_status vv_upload_lic(vv_ctx* c, const float* lic, int channels, const int dim
         if (st) return st;
         HIPCHK(c, lic_buffer(c, channels, dims));
         HIPCHK(c, launch_pad_repeat_f32((const float*)c->stage.p, channels, dims, (float*)c->lic.p, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
         for (int a = 0; a < 3; ++a) c->ldims[a] = dims[a];
         c->lch = channels;
         c->has_lic = true;
         c->has_sigma = false;  // opacity scale lives on the LIC grid
         ++c->scene_version;
+        HIPCHK(c, pair_buffer(c));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
         return VV_OK;
     });
 }

@@ -149,7 +149,7 @@ struct vv_ctx {
     // the ray casters' sample volume of lic and the field's channel pair_ch
     // (RenderLaunch::pair), made once the frames since either changed are
     // worth it; pair_used counts their samples.  Its buffer comes with the LIC
-    // volume's (lic_buffer), so no frame allocates, and may be missing.
+    // volume's (pair_buffer), so no frame allocates, and may be missing.
     DevBuf pair;
     bool pair_ok = false;
     int pair_ch = 0;
@@ -522,18 +522,22 @@ inline size_t pair_bytes(int channels, const int d[3])
     return sizeof(float) * (channels == 1 ? 2 : 1) * (size_t)clamp_elems(d);
 }
 
-// Room for a LIC volume of d voxels, and for its sample volume where memory
-// suffices.  A LIC volume of the same size as before allocates nothing and
-// stays where a captured graph has it.
+// Room for a LIC volume of d voxels.  One of the same size as before allocates
+// nothing and stays where a captured graph has it.
 inline hipError_t lic_buffer(vv_ctx* c, int channels, const int d[3])
 {
-    const size_t lic = sizeof(float) * channels * (size_t)repeat_elems(d), pair = pair_bytes(channels, d);
     drop_pair(c);
-    const hipError_t e = c->lic.ensure(lic, c->has_lic);
+    return c->lic.ensure(sizeof(float) * channels * (size_t)repeat_elems(d), c->has_lic);
+}
+
+// Room for the sample volume of the context's LIC volume, where memory
+// suffices: after the LIC volume's launch, which the allocation overlaps.
+inline hipError_t pair_buffer(vv_ctx* c)
+{
     const hipStreamCaptureStatus st = capture_status(c);
     if (st == hipStreamCaptureStatusActive) c->pair_on = 0;
-    if (e != hipSuccess || !c->pair_on || st != hipStreamCaptureStatusNone || (channels == 1 && !pair_addressable(d))) return e;
-    return c->pair.ensure_optional(pair);
+    const bool none = !c->pair_on || st != hipStreamCaptureStatusNone || (c->lch == 1 && !pair_addressable(c->ldims));
+    return none ? hipSuccess : c->pair.ensure_optional(pair_bytes(c->lch, c->ldims));
 }
 
 // R.pair: the sample volume of the context's LIC volume and field, made here
