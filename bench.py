@@ -91,17 +91,17 @@ def roofline(tag: str, kernel: str, ms: float, fetch_bytes: float) -> dict:
     rocprof counter summary of the same kernel and workload
     (profiles/<tag>_pmc.txt).
 
-    The bound that holds is FP32 VALU issue: the fma/add/mul wave64
-    instructions of a launch (SQ_INSTS_VALU_{FMA,ADD,MUL}_F32) issue at most
-    once per clock per CU (the 157.3 TFLOP/s FP32 figure is 256 CUs x 2.4 GHz
-    x 64 lanes x 2 flops x 2 for packed FP32, which the library's kernels do not
-    emit), so `frac` = instructions / (launch clocks x 256 CUs).  Beside it:
-    the FP32 flop rate against 157.3 TFLOP/s, HBM bytes (FETCH_SIZE +
-    WRITE_SIZE, calibrated on a copy of known size) against 8 TB/s, L1
-    cache-line accesses per clock per CU, L2 request bandwidth, and the
-    texture-fetch bytes the reference's shader requests: those are served by
-    the per-lane cell caches, L1 and L2, so they are a gather volume, not an
-    HBM fraction."""
+    The bound that holds for FP32 fields is the L1: `frac` is the share of the
+    launch's clocks (2.4 GHz, 256 CUs) in which its address unit is busy
+    (TA_TA_BUSY).  Beside it: FP32 VALU issue, the fma/add/mul wave64
+    instructions of a launch (SQ_INSTS_VALU_{FMA,ADD,MUL}_F32) against two per
+    clock per CU (157.3 TFLOP/s = 256 CUs x 2.4 GHz x 64 lanes x 2 flops x 2;
+    chains of vector operands reach 1.7, with a scalar operand 0.97), the FP32
+    flop rate against 157.3 TFLOP/s, HBM bytes (FETCH_SIZE + WRITE_SIZE,
+    calibrated on a copy of known size) against 8 TB/s, L1 cache-line accesses
+    per clock per CU, L2 request bandwidth, and the texture-fetch bytes the
+    reference's shader requests: those are served by the per-lane cell caches,
+    L1 and L2, so they are a gather volume, not an HBM fraction."""
     name = f"{tag}_pmc.txt"
     sec = ms / 1000.0
     clocks = sec * MI355X_CUS * MI355X_CLOCK_HZ
@@ -112,18 +112,22 @@ def roofline(tag: str, kernel: str, ms: float, fetch_bytes: float) -> dict:
     traffic = _profile_value(name, "traffic_bytes_per_launch")
     l1 = _profile_value(name, "TCP_TOTAL_CACHE_ACCESSES per launch")
     l2 = _profile_value(name, "TCC requests per launch")
-    rate = None if valu is None else valu / clocks
+    ta = _profile_value(name, "TA_TA_BUSY per launch")
+    busy = None if ta is None else min(ta / clocks, 1.0)
     r = {
-        "bound": "valu_f32",
-        "achieved": rate,
+        "bound": "l1_busy",
+        "achieved": busy,
         "peak": 1.0,
-        "unit": "wave64 FP32 fma/add/mul instructions per clock per CU",
-        "frac": None if rate is None else min(rate, 1.0),
+        "unit": "clocks with the L1's address unit busy per clock",
+        "frac": busy,
         "traffic": traffic,
         "kernel": kernel,
         "launch_ms": ms,
         "counts_from": f"profiles/{name}",
     }
+    if valu is not None:
+        r["valu_f32"] = {"achieved": valu / clocks, "peak": 2.0, "frac": valu / clocks / 2.0,
+                         "unit": "wave64 FP32 fma/add/mul instructions per clock per CU"}
     if None not in (fma, add, mul):
         tflops = (2.0 * fma + add + mul) * 64.0 / sec / 1e12
         r["flops"] = {"achieved": tflops, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",

@@ -301,6 +301,7 @@ __device__ __forceinline__ uint8_t quantize8(float f)
     return (uint8_t)fminf(fmaxf(k, 0.0f), 255.0f);
 }
 
+// raw noise (+ quantised gradients) -> REPEAT-padded texture
 __global__ void __launch_bounds__(kThreads) k_noise_tex(const uint8_t* noise, const uint8_t* rgb,
                                                         int nx, int ny, int nz, void* tex, int nc)
 {
@@ -531,8 +532,6 @@ __global__ void __launch_bounds__(kThreads) k_noise_grad_tex(const uint8_t* __re
     }
 }
 
-// raw noise (+ quantised gradients) -> REPEAT-padded texture
-
 template <typename FT, bool SAME, bool BRICK = false>
 __device__ __forceinline__ void lic_cached_tile(const LicArgs& a, int tile)
 {
@@ -559,9 +558,8 @@ __device__ __forceinline__ void lic_cached_tile(const LicArgs& a, int tile)
     store_repeat<float>(a.out, a.osy, a.osz, x, y, z, nx, ny, nz, acc * a.scl);
 }
 
-// SAME: at most 80 VGPRs (6 waves per SIMD instead of 5, 1-2 registers
-// spilled), measured 1.5 % faster at 256^3 (FP32 5.71 vs 5.80 ms, FP16 4.79
-// vs 4.86 ms); the separate-noise variants keep their 86 registers
+// SAME: at most 80 VGPRs, so six waves per SIMD instead of five (FP32 79, UNORM8
+// 78, FP16 80 with two spilled); the separate-noise variants keep their 82 to 94
 // BRICK: the float4 LIC copy in 8^3 bricks (a.field.p, strides a.bsy/bsz)
 template <typename FT, bool SAME, bool BRICK = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SAME ? 6 : 1)))

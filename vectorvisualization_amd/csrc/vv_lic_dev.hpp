@@ -21,7 +21,7 @@ struct LicArgs {
     int nblocks;         // gx*gy*gz
     int per_xcd;         // tiles handled by each of the 8 XCDs
     int sx, sy, sz;      // super-tile size in tiles (3D-blocked tile order)
-    int speed;           // SPEED_OF_FLOW (uncached path only)
+    int speed;           // SPEED_OF_FLOW, for lic_point (the cached kernels take it as a template argument)
     int bsy, bsz;        // BRICK kernels: field.p is the 8^3-brick copy with these brick-row and
                          // brick-plane strides (elements)
 };
@@ -155,12 +155,13 @@ __device__ __forceinline__ void store_repeat(T* out, int osy, int osz, int x, in
 // NaN keys never hit; a coordinate so little below an integer that its
 // fraction rounds to 1 is filled again, with the same texels.  (Cells
 // outside the volume with different floors but the same clamped texels are
-// reloaded, with the same values.)  On gfx950 floor, compare, convert, med3
-// and 24-bit multiplies issue at about 0.9 wave64 instructions per clock per
-// CU, fma, add, sub, mul and mov at 1.4-1.6 (measured), so the kernels spend
-// their compares and conversions on a miss: 256^3, L = 40, FP16 4.44 -> 4.27 ms,
-// UNORM8 4.73 -> 4.53, FP16 with noise on another grid 7.04 -> 6.31; FP32, which
-// waits for the L1, 5.60 -> 5.59.
+// reloaded, with the same values.)  On gfx950 floor, compare, convert, min, max
+// and 24-bit multiplies issue at 0.97 wave64 instructions per clock per CU,
+// fma, add, sub, mul and mov of vector operands at 1.7 (0.97 with a scalar
+// one; measured), so the kernels spend their compares and conversions on a
+// miss: 256^3, L = 40, FP16 4.44 -> 4.27 ms, UNORM8 4.73 -> 4.53, FP16 with noise on
+// another grid 7.04 -> 6.31.  FP32 fields with the noise in their LIC copy, which
+// wait for the L1, test the floors (fill_hit).
 // v_fma_mix_f32 with one half operand, which the instruction widens exactly
 // (every half is a float), so each form is one rounding of the exact result:
 //   fma_half<HI>(a, b, w) = fmaf(a, b, (float)h), h the low (HI 0) or high
@@ -223,11 +224,11 @@ __device__ __forceinline__ float lerp_pair(float f, unsigned w)
 // FP32 texels of the LIC copy: channel 3 holds the noise byte and the
 // difference to the next texel's as two halves (whole numbers up to 255, held
 // exactly), so a fill subtracts three channels instead of four and keeps one
-// noise word per row instead of two floats: the kernel fits its 80 registers
-// without the five spills it had (256^3, L = 40: 5.65 -> 5.59 ms).  A load of 8
-// to 16 bytes per lane occupies the L1 for 16 clocks or more whichever lanes
-// take part (measured), and the eight loads of a fill make that the bound of
-// the FP32 kernel: 1.1 fills per step, 145 of its 155 clocks per step.
+// noise word per row instead of two floats: 79 registers without a spill.  A
+// load of 8 to 16 bytes per lane occupies the L1 for 16 clocks or more
+// whichever lanes take part (measured), and the eight loads of a fill, 1.1
+// fills per Heun step, make that the bound of the FP32 kernel: the L1's address
+// unit is busy 154 of the 163 clocks that a wave's step takes (256^3, L = 40).
 template <>
 struct FieldCache<float4, 4> {
     float kx, ky, kz;

@@ -10,6 +10,7 @@
 // One thread per pixel; the 256x4 RGBA transfer function and the 256-entry
 // opacity table live in LDS.  The build is -ffp-contract=off; fmaf marks
 // every fused operation of the shared formulation.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -96,14 +97,14 @@ __device__ __forceinline__ float pow_corr(float b, float c, int mode)
     }
 }
 
-// per-pixel ray: analytic entry into [0,extent]^3 (the rasterised front
-// faces of drawCubeFaces), dir = normalize(entry - camera) * scaleVol
 __device__ __forceinline__ void view_vector(const float dir[3], float V[3])
 {
     const float vd[3] = {-dir[0], -dir[1], -dir[2]};
     normalize3(vd, V);
 }
 
+// per-pixel ray: analytic entry into [0,extent]^3 (the rasterised front
+// faces of drawCubeFaces), dir = normalize(entry - camera) * scaleVol
 __device__ __forceinline__ bool ray_setup(const ViewBlock& v, int i, int j, Ray& r)
 {
     const float nxp = fmaf((float)i + 0.5f, v.inv_w2, -1.0f);
@@ -724,8 +725,9 @@ __global__ void __launch_bounds__(kRThreads) k_render_rg(RenderLaunch a, int G_r
 // tiles write.
 // GT > 0: GT lanes per ray (2 or 4) in 256-thread blocks over rg_tile(GT)
 // pixel tiles; GT = 0: one lane per pixel over blockDim pixel tiles.  Four
-// waves per SIMD (at most 128 VGPRs): the scalar-LIC grouped kernels spill 2-4
-// registers and still run the batch faster than at 143 VGPRs and 3 waves.
+// waves per SIMD at least: the sample volume's kernels take 72 to 80 VGPRs, the
+// two volumes' 127 or 128 (up to 3 spilled, and still faster than with 143 and
+// three waves).
 template <typename FT, int LC, int GT>
 __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(4)))
 k_render_batch(const RenderLaunch* views, const int* first,
@@ -989,7 +991,9 @@ __global__ void __launch_bounds__(kRThreads) k_adjoint_forward(AdjointLaunch A)
 // column entries (D.a before it, the part's start position, the checkpoint)
 // while the part's clamp masks, the same in every lane, are written by the
 // group's first lane.  Columns, checkpoints, counts, bounds and image are
-// k_adjoint_forward's bits.
+// k_adjoint_forward's bits.  A clamp and its mask bit share their compares; a
+// hardware clamp with the masks from a second pass over the rounds that
+// clamped was slower (256^3, 512^2, 4 lanes: 143 against 130 us).
 template <typename FT, int LC, int GT>
 __global__ void __launch_bounds__(kRThreads) k_adjoint_forward_rg(AdjointLaunch A)
 {
@@ -1686,9 +1690,9 @@ __device__ __forceinline__ void view_after_lic(Ray& r)
 // (computeLIC, scaled by licKernel.b * gradient.r), shades it and composites
 // it.  A ray stops when it leaves the box or when the sample's own alpha
 // exceeds 0.95 (src.a, :91; the LIC-volume caster tests the accumulated
-// dest.a).  MODE 0: any noise / gate; 1: per-lane cell caches (scalar noise,
-// no gate), renewed for every sample; 2: the same with the noise grid equal
-// to the field grid at freq 1.
+// dest.a).  MODE 0: lic_point; 1: per-lane cell caches, renewed for every
+// sample; 2: the same with the noise in the LIC copy of the field (scalar noise
+// on its grid at freq 1, or RGBA noise on the grid of an FP32 field).
 template <typename FT, int NC, bool GATE, int MODE>
 __global__ void __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(3)))
 k_render_fused(RenderLaunch a, LicArgs L)
@@ -1890,12 +1894,17 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
     // ray and the block's rays in rows, or (kRayQuads) ray by ray within a
     // sample and the rays in Z order, so that a quad of lanes, whose accesses
     // the L1 serves together, is 2 x 2 neighbouring rays (G <= 16).  FP32
-    // waits on the L1 and takes the second where the two registers more leave
-    // the waves per SIMD as they are.  Fused, 512 x 512, first and second:
-    // 256^3, 40+40 steps, scalar noise FP32 8.24 and 7.79 ms, FP16 4.82 and
-    // 5.07, UNORM8 4.92 and 4.99; 128^3, 20+20 steps, gate FP32 2.89 and 2.80,
-    // RGBA without cell caches 6.8 and 4.7, with them 1.85 and 1.95 (131
-    // registers).  Scalar slices take up to 3 % longer with the second.
+    // waits on the L1 and takes the second where its one to four registers
+    // more leave the waves per SIMD as they are and no size loses much.  Time with
+    // the second over the first, 64^3 to 256^3, 128^2 to 900^2 (registers):
+    //   MODE 0           .54 to 1.09 (116-127, 117-130)
+    //   MODE 1  gate     fused .95 to 1.01 (143, 146)   slices .97 to 1.06 (141, 142)
+    //           RGBA     fused .91 to 1.00 (130, 133)   slices 1.02 to 1.20 (128, 129)
+    //           scalar   fused .91 to 1.08 (126, 129)   slices .91 to 1.01 (124, 125)
+    //   MODE 2  scalar   fused .84 to 1.00 (122, 125)   slices .90 to 1.04 (120, 121)
+    //           RGBA     fused .91 to 1.10 (128, 131)   slices .94 to 1.05 (126, 127)
+    // FP16 and UNORM8 lose (256^3, 512^2, 40+40 steps: 4.82 and 5.07 ms, 4.92 and
+    // 4.99).
     constexpr bool kRayQuads =
         std::is_same<FT, float4>::value &&
         (MODE == 0 || (MODE == 2 ? SLICES == (NC == 4) : !SLICES && (NC == 4 || GATE)));
@@ -2127,13 +2136,15 @@ namespace {
 // slices 3.8 -> 2.4), also where a kernel then passes 128 registers, but for
 // short streamlines in slices: there most of the time is the fragments around
 // the LIC, and three waves per SIMD instead of four (gate in FP32 and UNORM8,
-// 141 registers; RGBA noise in FP16, 136) cost more than the loads.  128^3 with
-// the caches against without: 120^2, 2+2 steps 1.12 to 1.19, 4+4 1.00 to 1.08,
-// 6+6 .90 to .96; 200^2 to 512^2, 2+2 steps 1.12 to 1.21, 8+8 1.02 to 1.16, 12+12
-// .86 to 1.12.  SPEED_OF_FLOW takes 0.
-inline int short_lic(const RenderLaunch& R)
+// 141 registers; RGBA noise in FP16, 136) cost more than the loads, the more
+// rays there are to fill the waves.  128^3, with the caches against without:
+//   gate, FP32       200^2: 9+9 steps 1.00, 12+12  .85    340^2: 12+12 1.04, 16+16  .98
+//   RGBA noise, FP16 160^2: 9+9 steps 1.02, 12+12  .92    340^2: 12+12 1.11, 20+20 1.02
+// SPEED_OF_FLOW takes 0.
+inline long long short_lic(const RenderLaunch& R, bool gate)
 {
-    return (long long)R.view.width * R.view.height > (1ll << 14) ? 16 : 8;
+    const long long rays = (long long)R.view.width * R.view.height;
+    return gate ? std::min(24ll, rays / 2200) : std::min(44ll, rays / 1500);
 }
 
 struct LicVariant {
@@ -2149,7 +2160,7 @@ LicVariant lic_variant(const RenderLaunch& R, const LicLaunch& L, bool slices)
     v.nc = L.nc;
     const LicKind k = lic_kind(L);
     const bool three_waves = k == LicKind::Cells && (L.gate ? L.field_type != 1 : L.field_type == 1);
-    const bool direct = k == LicKind::Direct || L.speed || (slices && three_waves && L.F + L.B <= short_lic(R));
+    const bool direct = k == LicKind::Direct || L.speed || (slices && three_waves && L.F + L.B <= short_lic(R, L.gate != 0));
     v.mode = direct ? 0 : k == LicKind::Copy || k == LicKind::Copy4 ? 2 : 1;
     return v;
 }
