@@ -160,8 +160,8 @@ __device__ __forceinline__ void store_repeat(T* out, int osy, int osz, int x, in
 // fma, add, sub, mul and mov of vector operands at 1.7 (0.97 with a scalar
 // one; measured), so the kernels spend their compares and conversions on a
 // miss: 256^3, L = 40, FP16 4.44 -> 4.27 ms, UNORM8 4.73 -> 4.53, FP16 with noise on
-// another grid 7.04 -> 6.31.  FP32 fields with the noise in their LIC copy, which
-// wait for the L1, test the floors (fill_hit).
+// another grid 7.04 -> 6.31.  Some fills of field_at are better tested by floors
+// (fill_hit).
 // v_fma_mix_f32 with one half operand, which the instruction widens exactly
 // (every half is a float), so each form is one rounding of the exact result:
 //   fma_half<HI>(a, b, w) = fmaf(a, b, (float)h), h the low (HI 0) or high
@@ -554,14 +554,23 @@ __device__ __forceinline__ float3 field_rgb_of(const FieldCache<FT, NCH>& fc, co
                        FieldScale<FT>::apply(tri_fc<2>(fc, f.x, f.y, f.z)));
 }
 
-// The hit test of field_at: with FP32 texels by floors, elsewhere by fractions
-// (cell_hit).  An FP32 fill waits on the L1, and floors taken before the test
-// start it sooner: slices of 124 x 32 x 154 voxels at 302 x 174, 31+31 steps,
-// 479 us by fractions, 463 by floors; the LIC volume takes the same by either.
-template <typename FT, int NCH>
-__device__ __forceinline__ bool fill_hit(const FieldCache<FT, NCH>& fc, const P3& t, P3& f)
+// The hit test of field_at: by floors (FLOORS) or by fractions (cell_hit).
+// Floors taken before the test start a fill sooner, fractions spare a hit the
+// floors' issue.  FP32, whose fills wait on the L1, takes floors: slices of
+// 124 x 32 x 154 voxels at 302 x 174, 31+31 steps, 479 us by fractions, 463 by
+// floors; the LIC volume takes the same by either.  FP16 with the noise in its
+// LIC copy takes them in slices, whose lanes wait for a few fragments' fills
+// (78 x 112 x 25, 480 x 300, 20+20 steps: 457 us by fractions, 441 by floors;
+// 128^3, 480 x 480, 10+10: 1888, 1812), and fractions in rays of samples (128^3,
+// 480 x 480, 40+40: floors 3 % more) and in the LIC volume (512^3, 60+60: 54.8 ms,
+// floors 56.0).
+template <typename FT>
+constexpr bool kFloors = std::is_same<FT, float4>::value;
+
+template <bool FLOORS, typename CACHE>
+__device__ __forceinline__ bool fill_hit(const CACHE& fc, const P3& t, P3& f)
 {
-    if constexpr (std::is_same<FT, float4>::value) {
+    if constexpr (FLOORS) {
         const P3 k{floorf(t.x), floorf(t.y), floorf(t.z)};
         f = P3{t.x - k.x, t.y - k.y, t.z - k.z};
         return k.x == fc.kx && k.y == fc.ky && k.z == fc.kz;
@@ -570,10 +579,10 @@ __device__ __forceinline__ bool fill_hit(const FieldCache<FT, NCH>& fc, const P3
     }
 }
 
-template <typename FT, int NCH>
-__device__ __forceinline__ void fill_rekey(FieldCache<FT, NCH>& fc, const P3& t, P3& f)
+template <bool FLOORS, typename CACHE>
+__device__ __forceinline__ void fill_rekey(CACHE& fc, const P3& t, P3& f)
 {
-    if constexpr (std::is_same<FT, float4>::value) {
+    if constexpr (FLOORS) {
         fc.kx = floorf(t.x);
         fc.ky = floorf(t.y);
         fc.kz = floorf(t.z);
@@ -582,11 +591,11 @@ __device__ __forceinline__ void fill_rekey(FieldCache<FT, NCH>& fc, const P3& t,
     }
 }
 
-template <typename FT, int NCH, bool BRICK = false>
+template <typename FT, int NCH, bool BRICK = false, bool FLOORS = kFloors<FT>>
 __device__ __forceinline__ float3 field_at(const CachedArgs& c, FieldCache<FT, NCH>& fc, const P3& t, P3& f)
 {
-    if (!fill_hit(fc, t, f)) {
-        fill_rekey(fc, t, f);
+    if (!fill_hit<FLOORS>(fc, t, f)) {
+        fill_rekey<FLOORS>(fc, t, f);
         // clamped floors; a floor the clamp leaves unchanged lies in [-1, n-1]
         const P3 m = clamp_floors(c, fc.kx, fc.ky, fc.kz);
         if constexpr (NCH == 4) fc.same = m.x == fc.kx && m.y == fc.ky && m.z == fc.kz;
@@ -804,7 +813,7 @@ __device__ __forceinline__ float decode_step(float s, float h)
     return fmaf(2.0f, s, -1.0f) * h;
 }
 
-template <typename FT, bool SAME, bool BRICK = false>
+template <typename FT, bool SAME, bool BRICK = false, bool FLOORS = kFloors<FT>>
 __device__ __forceinline__ float lic_point_cached(const LicArgs& a, const CachedArgs& c, LicFieldCache<FT, SAME>& fc,
                                                   NoiseCache& ncache, float sx, float sy, float sz)
 {
@@ -814,7 +823,7 @@ __device__ __forceinline__ float lic_point_cached(const LicArgs& a, const Cached
     };
     P3 f;
     const float3 s0 =
-        field_at<FT, SAME ? 4 : 3, BRICK>(c, fc, P3{texel(sx, nx), texel(sy, ny), texel(sz, nz)}, f);
+        field_at<FT, SAME ? 4 : 3, BRICK, FLOORS>(c, fc, P3{texel(sx, nx), texel(sy, ny), texel(sz, nz)}, f);
     float n0;
     if constexpr (SAME)
         n0 = noise_same<FT>(c, fc, f);
@@ -842,7 +851,7 @@ __device__ __forceinline__ float lic_point_cached(const LicArgs& a, const Cached
             const float d1z = decode_step(s.z, h);
             const float qx = px + d1x, qy = py + d1y, qz = pz + d1z;
             const float3 s2 =
-                field_at<FT, SAME ? 4 : 3, BRICK>(c, fc, P3{texel(qx, nx), texel(qy, ny), texel(qz, nz)}, f);
+                field_at<FT, SAME ? 4 : 3, BRICK, FLOORS>(c, fc, P3{texel(qx, nx), texel(qy, ny), texel(qz, nz)}, f);
             const float d2x = decode_step(s2.x, h);
             const float d2y = decode_step(s2.y, h);
             const float d2z = decode_step(s2.z, h);
@@ -852,7 +861,7 @@ __device__ __forceinline__ float lic_point_cached(const LicArgs& a, const Cached
             const P3 t{texel(px, nx), texel(py, ny), texel(pz, nz)};
             float nval;
             if constexpr (SAME) {
-                s = field_at<FT, 4, BRICK>(c, fc, t, f);
+                s = field_at<FT, 4, BRICK, FLOORS>(c, fc, t, f);
                 nval = noise_same<FT>(c, fc, f);
             } else {
                 s = field_and_noise<FT>(a, c, fc, ncache, t, noise_texel(px, py, pz), nval);

@@ -1651,7 +1651,7 @@ __device__ __forceinline__ float tf_alpha(const float* tf, float u)
 // cell caches live for one sample: consecutive samples of a lane are G steps
 // apart, so the previous streamline's last cell rarely serves the next one,
 // and the caches' registers are free while shading.
-template <typename FT, int NC, bool GATE, int MODE>
+template <typename FT, int NC, bool GATE, int MODE, bool SLICES>
 __device__ __forceinline__ void sample_lic(const LicArgs& L, const CachedArgs& c, const float pos[3], float l4[4])
 {
     if constexpr (MODE > 0 && NC == 1 && !GATE) {
@@ -1659,7 +1659,8 @@ __device__ __forceinline__ void sample_lic(const LicArgs& L, const CachedArgs& c
         fc.reset();
         NoiseCache nc;
         nc.reset();
-        l4[0] = lic_point_cached<FT, MODE == 2>(L, c, fc, nc, pos[0], pos[1], pos[2]) * L.scl;
+        constexpr bool kFl = kFloors<FT> || (SLICES && MODE == 2);
+        l4[0] = lic_point_cached<FT, MODE == 2, false, kFl>(L, c, fc, nc, pos[0], pos[1], pos[2]) * L.scl;
     } else {
         float4 acc;
         if constexpr (MODE > 0)
@@ -1714,7 +1715,7 @@ k_render_fused(RenderLaunch a, LicArgs L)
             float pos[3] = {r.pos[0], r.pos[1], r.pos[2]};
             for (long long k = 0; k < a.max_samples; ++k) {
                 float l4[4];
-                sample_lic<FT, NC, GATE, MODE>(L, c, pos, l4);
+                sample_lic<FT, NC, GATE, MODE, false>(L, c, pos, l4);
                 view_after_lic(r);
                 const Cell cf = cell_clamp(fv, pos[0], pos[1], pos[2]);
                 Sample s;
@@ -1840,7 +1841,7 @@ k_render_slices(RenderLaunch a, LicArgs L, SliceSetup S)
             const float tfu = tri_ch(fv, cell_clamp(fv, pos[0], pos[1], pos[2]), a.tf_ch);
             if (!(tf_alpha(tf, tfu) > 0.05f)) continue;
             float l4[4];
-            sample_lic<FT, NC, GATE, MODE>(L, c, pos, l4);
+            sample_lic<FT, NC, GATE, MODE, true>(L, c, pos, l4);
             Ray r;
             const Cell cf = slice_fragment<FT, NC>(vb, fv, d, sk, pos, r);
             Sample s;
@@ -1996,7 +1997,7 @@ k_render_group(RenderLaunch a, LicArgs L, SliceSetup S, int G)
             }
             if (ok) {
                 float l4[4];
-                sample_lic<FT, NC, GATE, MODE>(L, c, pos, l4);
+                sample_lic<FT, NC, GATE, MODE, SLICES>(L, c, pos, l4);
                 Cell cf;
                 if constexpr (SLICES) {
                     cf = slice_fragment<FT, NC>(vb, fv, d, sk, pos, r);
