@@ -1659,7 +1659,7 @@ __device__ __forceinline__ void sample_lic(const LicArgs& L, const CachedArgs& c
         fc.reset();
         NoiseCache nc;
         nc.reset();
-        constexpr bool kFl = kFloors<FT> || (SLICES && MODE == 2);
+        constexpr bool kFl = kFloors<FT> || (SLICES && MODE == 2 && std::is_same<FT, half4_t>::value);
         l4[0] = lic_point_cached<FT, MODE == 2, false, kFl>(L, c, fc, nc, pos[0], pos[1], pos[2]) * L.scl;
     } else {
         float4 acc;
